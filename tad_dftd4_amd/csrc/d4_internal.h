@@ -93,8 +93,8 @@ struct Work {
   double* dgw;      // [B*N*8] d gw / d CN (D4S: unused)
   double* dgw0;     // [B*N*8] d gw0 / d CN (D4S: unused)
   double* dgwq;     // [B*N*8] d gw / d q (D4S: dzeta/dq)
-  double* chol;     // [B*NT] packed lower Cholesky factor of the Coulomb block
-  double* ez;       // [B*N] y_e = L^-1 e (forward-substituted border, e = 1 on real atoms)
+  double* chol;     // [B*NT] packed L D L^T of the Coulomb block (L strictly lower, D diagonal)
+  double* ez;       // [B*N] D^-1 L^-1 e (e = 1 on real atoms; tiled EEQ: L^-1 e)
   double* lu;       // [B*(N+1)^2] pivoted LU of the bordered matrix (fallback)
   int32_t* piv;     // [B*(N+1)]
   double* vec;      // [B*(N+1)] right-hand side / solution of the LU path
