@@ -263,6 +263,20 @@ int d4_model_pols_backward(d4_context* ctx, void* stream, int64_t nbatch, int64_
                            const int64_t* numbers, const d4_params* params, int static_only,
                            const double* grad_out, double* grad_gw_out);
 
+/* Inputs that the host has to see, read back in one step: whether any of the
+ * `count` atomic numbers lies outside 0..103, and up to D4_MAX_SCALARS scalars
+ * in device memory (kinds[k]: 0 double, 1 float). d4_inputs_begin enqueues the
+ * read on `stream` and returns a ticket; further calls may be enqueued before
+ * d4_inputs_wait, which waits for the read alone (not for work enqueued behind
+ * it), writes values[k] and *bad and ends the ticket. Every ticket is waited
+ * for once, with the context that began it. Refused while the stream is being
+ * captured. */
+#define D4_MAX_SCALARS 16
+int d4_inputs_begin(d4_context* ctx, void* stream, int64_t count, const int64_t* numbers,
+                    int nscalars, const void* const* scalars, const int32_t* kinds,
+                    void** ticket);
+int d4_inputs_wait(d4_context* ctx, void* ticket, double* values, int32_t* bad);
+
 /* Per-molecule status words of the last call that used `workspace`, copied
  * to host memory (synchronises the stream). Bit 0: EEQ solved by the
  * pivoted-LU path; bit 1: EEQ system singular; bit 2: Z out of range. */

@@ -36,6 +36,7 @@ D4_FLAG_ROWS_MASK = 768
 D4_FLAG_ATM8 = 1024
 D4_FLAG_ONE_STREAM = 2048
 D4_NOALLOC_SCRATCH_BYTES = 64 << 20
+D4_MAX_SCALARS = 16
 
 SLOTS = ("prep", "cn", "eeq", "weights", "pairs", "atm", "atm_rows", "adjoint", "chain")
 D4_PROFILE_SLOTS = 1 << 16
@@ -146,6 +147,11 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _i64, _i64, _vp, ctypes.POINTER(Params), ctypes.c_int, _vp, _vp],
     ),
+    "d4_inputs_begin": (
+        ctypes.c_int,
+        [_vp, _vp, _i64, _vp, ctypes.c_int, ctypes.POINTER(_vp), _ip, ctypes.POINTER(_vp)],
+    ),
+    "d4_inputs_wait": (ctypes.c_int, [_vp, _vp, _dp, _ip]),
     "d4_molecule_status": (ctypes.c_int, [_vp, _i64, _vp, _ip]),
     "d4_profile_enable": (ctypes.c_int, [_vp, ctypes.c_int]),
     "d4_profile_read": (

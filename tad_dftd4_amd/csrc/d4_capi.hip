@@ -32,6 +32,16 @@ struct d4_aux {
 constexpr size_t kScratchBytes = D4_NOALLOC_SCRATCH_BYTES;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
+// One read-back of inputs (d4_inputs_begin): pinned host memory that the
+// kernel writes, and the event behind it. Kept in the context for reuse, one
+// per read-back in flight.
+struct d4_ticket {
+  double* values = nullptr;  // [D4_MAX_SCALARS], then the bad flag
+  hipEvent_t done = nullptr;
+  int count = 0;
+  int32_t* bad() const { return (int32_t*)(values + D4_MAX_SCALARS); }
+};
+
 struct d4_context {
   int device;
   void* mem;
@@ -41,6 +51,8 @@ struct d4_context {
   bool has_model = false;   // alpha and refslot supplied (d4_model_* functions)
   std::mutex aux_mu;
   std::unordered_map<hipStream_t, d4_aux> aux;
+  std::mutex ticket_mu;
+  std::vector<d4_ticket*> tickets;  // idle ones
   // diagnostics: per-kernel event timing
   unsigned profile = 0;  // bit k: bracket launches of slot k with events
   std::vector<d4_event_pair> pending;
@@ -499,6 +511,11 @@ int d4_context_destroy(d4_context* ctx) {
     (void)hipEventDestroy(kv.second.join);
     (void)hipStreamDestroy(kv.second.s);
   }
+  for (d4_ticket* t : ctx->tickets) {
+    (void)hipEventDestroy(t->done);
+    (void)hipHostFree(t->values);
+    delete t;
+  }
   hipError_t e = hipFree(ctx->mem);
   (void)hipSetDevice(prev);
   delete ctx;
@@ -780,6 +797,78 @@ int d4_model_pols_backward(d4_context* ctx, void* stream, int64_t nbatch, int64_
   D4_TRY(d4::launch_model_pols_bwd((hipStream_t)stream, ctx->t, mc, static_only ? 1 : 0,
                                    grad_out, grad_gw_out),
          "model polarisabilities backward");
+  return D4_OK;
+}
+
+int d4_inputs_begin(d4_context* ctx, void* stream, int64_t count, const int64_t* numbers,
+                    int nscalars, const void* const* scalars, const int32_t* kinds,
+                    void** ticket) {
+  if (ticket == nullptr) return set_error(D4_ERR_INVALID, "ticket is NULL");
+  *ticket = nullptr;
+  if (ctx == nullptr) return set_error(D4_ERR_INVALID, "context is NULL");
+  if (count < 0 || (count > 0 && numbers == nullptr))
+    return set_error(D4_ERR_INVALID, "numbers must be non-NULL");
+  if (nscalars < 0 || nscalars > D4_MAX_SCALARS ||
+      (nscalars > 0 && (scalars == nullptr || kinds == nullptr)))
+    return set_error(D4_ERR_INVALID, "between 0 and D4_MAX_SCALARS scalars can be read");
+  d4::InputScalars sc{};
+  sc.count = nscalars;
+  for (int k = 0; k < nscalars; ++k) {
+    if (scalars[k] == nullptr || (kinds[k] != 0 && kinds[k] != 1))
+      return set_error(D4_ERR_INVALID, "a scalar is NULL or of an unknown kind");
+    sc.at[k] = scalars[k];
+    sc.kind[k] = kinds[k];
+  }
+  hipStream_t s = (hipStream_t)stream;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  D4_TRY(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
+  if (cap != hipStreamCaptureStatusNone)
+    return set_error(D4_ERR_DEVICE, "inputs cannot be read back while the stream is captured");
+  d4_ticket* t = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(ctx->ticket_mu);
+    if (!ctx->tickets.empty()) {
+      t = ctx->tickets.back();
+      ctx->tickets.pop_back();
+    }
+  }
+  if (t == nullptr) {
+    t = new d4_ticket;
+    void* mem = nullptr;
+    hipError_t e = hipHostMalloc(&mem, sizeof(double) * (D4_MAX_SCALARS + 1), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&t->done, hipEventDisableTiming);
+    if (e != hipSuccess) {
+      if (mem) (void)hipHostFree(mem);
+      delete t;
+      return hip_error(e, "input read-back buffer");
+    }
+    t->values = (double*)mem;
+  }
+  t->count = nscalars;
+  *t->bad() = 0;
+  hipError_t e = d4::launch_inputs(s, numbers, count, sc, t->values, t->bad());
+  if (e == hipSuccess) e = hipEventRecord(t->done, s);
+  if (e != hipSuccess) {
+    std::lock_guard<std::mutex> lock(ctx->ticket_mu);
+    ctx->tickets.push_back(t);
+    return hip_error(e, "input read-back");
+  }
+  *ticket = t;
+  return D4_OK;
+}
+
+int d4_inputs_wait(d4_context* ctx, void* ticket, double* values, int32_t* bad) {
+  if (ctx == nullptr || ticket == nullptr)
+    return set_error(D4_ERR_INVALID, "context or ticket is NULL");
+  d4_ticket* t = (d4_ticket*)ticket;
+  const hipError_t e = hipEventSynchronize(t->done);
+  for (int k = 0; k < t->count && values != nullptr; ++k) values[k] = t->values[k];
+  if (bad != nullptr) *bad = *t->bad();
+  {
+    std::lock_guard<std::mutex> lock(ctx->ticket_mu);
+    ctx->tickets.push_back(t);
+  }
+  if (e != hipSuccess) return hip_error(e, "input read-back");
   return D4_OK;
 }
 

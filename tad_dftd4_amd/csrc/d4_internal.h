@@ -375,6 +375,15 @@ hipError_t launch_properties(hipStream_t s, const DevTables& t,
                              const Inputs& in, const Work& w, double* c6_out,
                              double* alpha_out);
 hipError_t launch_copy(hipStream_t s, const double* src, double* dst, int64_t count);
+// Read-back of inputs into pinned host memory: bad = 1 if an atomic number lies
+// outside 0..kMaxZ - 1, values[k] = scalar k (kind 0: double, 1: float).
+struct InputScalars {
+  const void* at[D4_MAX_SCALARS];
+  int kind[D4_MAX_SCALARS];
+  int count;
+};
+hipError_t launch_inputs(hipStream_t s, const int64_t* numbers, int64_t count,
+                         const InputScalars& sc, double* values, int32_t* bad);
 // Fill t.pairk (kMaxZ^2 x 4 doubles at `out`) from the per-element tables.
 hipError_t launch_pair_consts(hipStream_t s, const DevTables& t, double* out);
 // Sum of the parameter-gradient partials into out[7] = dL/d(s6, s8, s10, s9,

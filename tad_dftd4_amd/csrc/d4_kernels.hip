@@ -2662,6 +2662,20 @@ __global__ __launch_bounds__(256) void k_copy(const double* src, double* dst,
   if (k < count) dst[k] = src[k];
 }
 
+// (every work-group that finds a bad number writes the same 1)
+__global__ __launch_bounds__(256) void k_inputs(const int64_t* numbers, int64_t count,
+                                                InputScalars sc, double* values, int32_t* bad) {
+  bool out = false;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count;
+       i += (int64_t)gridDim.x * 256)
+    out |= numbers[i] < 0 || numbers[i] >= kMaxZ;
+  if (out) *bad = 1;
+  if (blockIdx.x == 0 && (int)threadIdx.x < sc.count) {
+    const int k = threadIdx.x;
+    values[k] = sc.kind[k] ? (double)*(const float*)sc.at[k] : *(const double*)sc.at[k];
+  }
+}
+
 // Parameter gradients: fixed-order sums of the two-body row partials and the
 // three-body work-group partials into dL/d(s6, s8, s10, s9, a1, a2, alp).
 // mode: 0 pair-tile kernel (one partial per 16 x 16 pair tile), 1 one-pass
@@ -2975,6 +2989,15 @@ hipError_t launch_pgrad_reduce(hipStream_t s, const Params& p, const Inputs& in,
                                       : nb * (nb + 1) / 2;
   hipLaunchKernelGGL(k_pgrad_reduce, dim3(1), dim3(256), 0, s, in, w, mode, tile8 ? 1 : 0,
                      per_mol, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_inputs(hipStream_t s, const int64_t* numbers, int64_t count,
+                         const InputScalars& sc, double* values, int32_t* bad) {
+  int64_t grid = (count + 1023) / 1024;  // four numbers per thread, at most 256 work-groups
+  grid = grid < 1 ? 1 : (grid > 256 ? 256 : grid);
+  hipLaunchKernelGGL(k_inputs, dim3((unsigned)grid), dim3(256), 0, s, numbers, count, sc, values,
+                     bad);
   return hipGetLastError();
 }
 

@@ -39,6 +39,7 @@ from .cutoff import Cutoff
 from .damping import Damping, Param, RationalDamping
 from .model import D4Model, D4SModel
 from .ncoord import cn_d4, erf_count
+from .tables import GA_DEFAULT, GC_DEFAULT
 
 __all__ = ["dftd4", "get_properties", "dftd4_energy_gradient", "dftd4_hessian"]
 
@@ -48,17 +49,47 @@ _STENCIL = (1.0, -1.0, 2.0, -2.0)
 _MODELS = ("d3", "d4", "d4s", "d5")
 
 
-def _value(x) -> float:
+def _value(x, values=None) -> float:
     if isinstance(x, torch.Tensor):
-        return float(x.detach().reshape(()).cpu()) if x.numel() == 1 else _bad(x)
+        if values is not None and id(x) in values:  # read back with the input check
+            return values[id(x)]
+        return float(x.item()) if x.numel() == 1 else _bad(x)
     return float(x)
+
+
+_CUTOFFS = ("disp2", "disp3", "cn_eeq")
+
+
+def _device_scalars(param: Param, cutoff: Cutoff | None, device) -> list[torch.Tensor]:
+    """The parameter and cutoff tensors that one read-back can bring to the
+    host (``runtime.InputCheck``)."""
+    found = [param.get(k) for k in runtime.PARAM_ORDER]
+    if cutoff is not None:
+        found += [getattr(cutoff, k) for k in _CUTOFFS]
+    return [t for t in found
+            if isinstance(t, torch.Tensor) and t.device == device and t.numel() == 1
+            and t.dtype in (torch.float64, torch.float32)]
+
+
+def _params(param: Param, cutoff: Cutoff | None, model_inst, check, scalars):
+    """Kernel parameters of a call whose input check is under way
+    (``_prepare``). Parameters on the device come from the check's read-back,
+    in one wait; without any the caller waits after its launches."""
+    values = None
+    if scalars:
+        values = {id(t): v for t, v in zip(scalars, check.wait())}
+    try:
+        return kernel_params(param, cutoff, model_inst, values)
+    except Exception:
+        check.wait()  # a bad atomic number is reported before a bad parameter
+        raise
 
 
 def _bad(x):
     raise ValueError(f"damping parameters must be scalars, got shape {tuple(x.shape)}")
 
 
-def kernel_params(param: Param, cutoff: Cutoff | None, model: D4Model | None):
+def kernel_params(param: Param, cutoff: Cutoff | None, model: D4Model | None, values=None):
     """Translate the reference's parameter conventions into kernel values.
 
     - a1 and a2 are required by rational damping (``functions.py:264-268``).
@@ -77,19 +108,21 @@ def kernel_params(param: Param, cutoff: Cutoff | None, model: D4Model | None):
     has8 = param.get("s8") is not None or param.get("rs8") is not None
     s10_on = "s10" in param and param["s10"] is not None
     if cutoff is None:
-        cutoff = Cutoff()
+        cuts = (defaults.D4_DISP2_CUTOFF, defaults.D4_DISP3_CUTOFF, defaults.D4_CN_EEQ_CUTOFF)
+    else:
+        cuts = (cutoff.disp2, cutoff.disp3, cutoff.cn_eeq)
     kp = runtime.KernelParams(
-        s6=_value(param.get("s6", defaults.S6)),
-        s8=_value(param.get("s8", defaults.S8)) if has8 else 0.0,
-        s10=_value(param["s10"]) if s10_on else 0.0,
-        s9=_value(param.get("s9", defaults.S9)),
-        a1=_value(param["a1"]),
-        a2=_value(param["a2"]),
-        alp=_value(param.get("alp", defaults.ALP)),
-        cutoff_disp2=_value(cutoff.disp2),
-        cutoff_disp3=_value(cutoff.disp3),
+        s6=_value(param.get("s6", defaults.S6), values),
+        s8=_value(param.get("s8", defaults.S8), values) if has8 else 0.0,
+        s10=_value(param["s10"], values) if s10_on else 0.0,
+        s9=_value(param.get("s9", defaults.S9), values),
+        a1=_value(param["a1"], values),
+        a2=_value(param["a2"], values),
+        alp=_value(param.get("alp", defaults.ALP), values),
+        cutoff_disp2=_value(cuts[0], values),
+        cutoff_disp3=_value(cuts[1], values),
         cutoff_cn=defaults.CN_D4_INTERNAL_CUTOFF,
-        cutoff_eeq=_value(cutoff.cn_eeq),
+        cutoff_eeq=_value(cuts[2], values),
         s10_on=s10_on,
     )
     if model is not None:
@@ -203,7 +236,11 @@ class _D4Grad(torch.autograd.Function):
 
 
 def _prepare(numbers, positions, charge, model, rcov, r4r2, rvdw, q, cn_function,
-             counting_function, damping_function):
+             counting_function, damping_function, param=None, cutoff=None):
+    """Checked inputs in the kernels' layout, and the check of the atomic
+    numbers under way together with the read-back of the parameter tensors
+    that live on the device (``scalars``): see ``_params``; every caller ends
+    with ``check.wait()``."""
     if numbers.shape != positions.shape[:-1]:
         raise ValueError(
             f"Shape of positions ({positions.shape}) is not consistent "
@@ -252,17 +289,21 @@ def _prepare(numbers, positions, charge, model, rcov, r4r2, rvdw, q, cn_function
     lead = numbers.shape[:-1]
     n = numbers.shape[-1]
     nums = numbers.to(device=dev, dtype=torch.int64).reshape(-1, n).contiguous()
-    if nums.numel() and (int(nums.min()) < 0 or int(nums.max()) >= 104):
-        raise ValueError("atomic numbers must lie in 0..103 (0 marks padding)")
+    scalars = _device_scalars(param, cutoff, dev) if param is not None else []
+    ga, gc = (model_inst.ga, model_inst.gc) if model_inst is not None else (GA_DEFAULT, GC_DEFAULT)
+    check = runtime.InputCheck(nums, scalars, ga, gc)
     pos = positions.to(torch.float64).reshape(-1, n, 3)
     if not pos.is_contiguous():
         pos = pos.contiguous()
-    chg = torch.as_tensor(charge, dtype=torch.float64, device=dev)
-    chg = torch.broadcast_to(chg, lead).reshape(-1).contiguous()
+    if isinstance(charge, (int, float)):  # a fill on the device instead of a copy to it
+        chg = torch.full((nums.shape[0],), float(charge), dtype=torch.float64, device=dev)
+    else:
+        chg = torch.as_tensor(charge, dtype=torch.float64, device=dev)
+        chg = torch.broadcast_to(chg, lead).reshape(-1).contiguous()
     # q stays attached to its autograd graph (dL/dq from the backward kernels)
     qq = None if q is None else q.to(dev, torch.float64).reshape(-1, n).contiguous()
     rr = None if r4r2 is None else r4r2.detach().to(dev, torch.float64).reshape(-1, n).contiguous()
-    return model_inst, nums, pos, chg, qq, rr, lead, n
+    return model_inst, nums, pos, chg, qq, rr, lead, n, check, scalars
 
 
 def dftd4(
@@ -292,11 +333,11 @@ def dftd4(
         raise NotImplementedError(
             "gradients with respect to user-supplied r4r2 values are not supported"
         )
-    model_inst, nums, pos, chg, qq, rr, lead, n = _prepare(
+    model_inst, nums, pos, chg, qq, rr, lead, n, check, scalars = _prepare(
         numbers, positions, charge, model, rcov, r4r2, rvdw, q, cn_function,
-        counting_function, damping_function,
+        counting_function, damping_function, param, cutoff,
     )
-    kp = kernel_params(param, cutoff, model_inst)
+    kp = _params(param, cutoff, model_inst, check, scalars)
     pkeys = tuple(
         k for k in runtime.PARAM_ORDER
         if isinstance(param.get(k), torch.Tensor) and param[k].requires_grad
@@ -305,6 +346,7 @@ def dftd4(
         pkeys = ()
     ptensors = tuple(param[k] for k in pkeys)
     energy = _D4Energy.apply(pos, nums, chg, qq, rr, kp, pkeys, *ptensors)
+    check.wait()
     return energy.reshape(*lead, n).to(positions.dtype)
 
 
@@ -322,12 +364,13 @@ def dftd4_energy_gradient(
     """Atom energies and dE_total/dR in one fused pass (no autograd graph).
     Equivalent to ``dftd4`` followed by
     ``torch.autograd.grad(energy.sum(), positions)``."""
-    model_inst, nums, pos, chg, qq, rr, lead, n = _prepare(
+    model_inst, nums, pos, chg, qq, rr, lead, n, check, scalars = _prepare(
         numbers, positions.detach(), charge, model, None, r4r2, None, q, cn_d4,
-        erf_count, RationalDamping(),
+        erf_count, RationalDamping(), param, cutoff,
     )
-    kp = kernel_params(param, cutoff, model_inst)
+    kp = _params(param, cutoff, model_inst, check, scalars)
     energy, grad, _ = runtime.energy_gradient(nums, pos, chg, kp, q=qq, r4r2=rr)
+    check.wait()
     return (energy.reshape(*lead, n).to(positions.dtype),
             grad.reshape(*lead, n, 3).to(positions.dtype))
 
@@ -354,15 +397,16 @@ def dftd4_hessian(
     energy + gradient kernels as one batch (split into batches of at most
     ``max_batch_bytes`` of workspace). The result is symmetrised. Padding
     atoms have zero rows and columns."""
-    model_inst, nums, pos, chg, qq, rr, lead, n = _prepare(
+    model_inst, nums, pos, chg, qq, rr, lead, n, check, scalars = _prepare(
         numbers, positions.detach(), charge, model, None, r4r2, None, q, cn_d4,
-        erf_count, RationalDamping(),
+        erf_count, RationalDamping(), param, cutoff,
     )
-    kp = kernel_params(param, cutoff, model_inst)
+    kp = _params(param, cutoff, model_inst, check, scalars)
     B = nums.shape[0]
     dev = pos.device
     hess = torch.zeros((B, n, 3, n, 3), dtype=torch.float64, device=dev)
     if B == 0 or n == 0:
+        check.wait()
         return hess.reshape(*lead, n, 3, n, 3).to(positions.dtype)
     # unit displacements of every (atom, direction), one molecule per column
     cols = 3 * n
@@ -381,6 +425,7 @@ def dftd4_hessian(
         mask = (real[:, None, None, None] & real[None, None, :, None]).to(torch.float64)
         hess[b] *= mask
     hess = 0.5 * (hess + hess.permute(0, 3, 4, 1, 2))
+    check.wait()
     return hess.reshape(*lead, n, 3, n, 3).to(positions.dtype)
 
 
@@ -394,12 +439,14 @@ def get_properties(
     static polarisabilities (reference ``disp.py:149-197``)."""
     if charge is None:
         charge = 0.0
-    model_inst, nums, pos, chg, _, _, lead, n = _prepare(
+    param = {"a1": 0.4, "a2": 5.0}
+    model_inst, nums, pos, chg, _, _, lead, n, check, scalars = _prepare(
         numbers, positions.detach(), charge, "d4", None, None, None, None, cn_d4,
-        erf_count, RationalDamping(),
+        erf_count, RationalDamping(), param, cutoff,
     )
-    kp = kernel_params({"a1": 0.4, "a2": 5.0}, cutoff, model_inst)
+    kp = _params(param, cutoff, model_inst, check, scalars)
     cn, q, c6, alpha = runtime.properties(nums, pos, chg, kp)
+    check.wait()
     dt = positions.dtype
     return (cn.reshape(*lead, n).to(dt), q.reshape(*lead, n).to(dt),
             c6.reshape(*lead, n, n).to(dt), alpha.reshape(*lead, n).to(dt))

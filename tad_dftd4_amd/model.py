@@ -100,10 +100,11 @@ class D4Model:
                 "tad_dftd4_amd computes on a ROCm device; move the tensors to 'cuda'"
             )
         z = self.numbers.to(device=dev, dtype=torch.int64)
-        if z.numel() and (int(z.min()) < 0 or int(z.max()) >= 104):
-            raise ValueError("atomic numbers must lie in 0..103 (0 marks padding)")
         n = z.shape[-1]
-        return z.reshape(-1, n).contiguous()
+        z = z.reshape(-1, n).contiguous()
+        if z.numel():  # (the kernels index the element tables with z: wait before them)
+            runtime.InputCheck(z, ga=self.ga, gc=self.gc).wait()
+        return z
 
     def _lead(self):
         return tuple(self.numbers.shape[:-1]), self.numbers.shape[-1]

@@ -36,7 +36,7 @@ def cn_d4(numbers: torch.Tensor, positions: torch.Tensor, **kwargs) -> torch.Ten
     from .damping import RationalDamping
     from .disp import _prepare, kernel_params
 
-    model_inst, nums, pos, chg, _, _, lead, n = _prepare(
+    model_inst, nums, pos, chg, _, _, lead, n, check, _ = _prepare(
         numbers, positions.detach(), 0.0, "d4", None, None, None, None, cn_d4,
         erf_count, RationalDamping(),
     )
@@ -44,4 +44,5 @@ def cn_d4(numbers: torch.Tensor, positions: torch.Tensor, **kwargs) -> torch.Ten
     if cutoff is not None:
         kp.cutoff_cn = float(cutoff)
     cn = runtime.properties(nums, pos, chg, kp, cn_only=True)[0]
+    check.wait()
     return cn.reshape(*lead, n).to(positions.dtype)

@@ -156,6 +156,58 @@ def _stream(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+class InputCheck:
+    """Range check of the atomic numbers and read-back of scalars that live on
+    the device, as one small kernel on the current stream and one wait for it
+    alone (``d4_inputs_begin``/``d4_inputs_wait``). Calls enqueued between the
+    constructor and ``wait`` are not waited for, so a caller that needs no
+    device scalar launches its evaluation first and waits at the end."""
+
+    def __init__(self, numbers, scalars=(), ga: float = GA_DEFAULT, gc: float = GC_DEFAULT):
+        dev = numbers.device
+        self._ctx = context(dev, ga, gc)
+        self._n = len(scalars)
+        ptrs = (ctypes.c_void_p * max(self._n, 1))(*[t.data_ptr() for t in scalars])
+        kinds = (ctypes.c_int32 * max(self._n, 1))(
+            *[0 if t.dtype == torch.float64 else 1 for t in scalars])
+        ticket = ctypes.c_void_p()
+        _lib.check(
+            _lib.load().d4_inputs_begin(
+                self._ctx, _stream(dev), numbers.numel(), _vp(numbers), self._n, ptrs, kinds,
+                ctypes.byref(ticket)),
+            "d4_inputs_begin",
+        )
+        self._ticket = ticket
+        self._values: list[float] = []
+        self._bad = False
+
+    def _end(self):
+        if self._ticket is None:
+            return
+        ticket, self._ticket = self._ticket, None
+        values = (ctypes.c_double * max(self._n, 1))()
+        bad = ctypes.c_int32()
+        _lib.check(
+            _lib.load().d4_inputs_wait(self._ctx, ticket, values, ctypes.byref(bad)),
+            "d4_inputs_wait",
+        )
+        self._values = list(values[: self._n])
+        self._bad = bool(bad.value)
+
+    def wait(self) -> list[float]:
+        """The scalars; raises ``ValueError`` for a number outside 0..103."""
+        self._end()
+        if self._bad:
+            raise ValueError("atomic numbers must lie in 0..103 (0 marks padding)")
+        return self._values
+
+    def __del__(self):
+        try:
+            self._end()
+        except Exception:
+            pass
+
+
 def _check_inputs(numbers, positions, charge):
     if not positions.is_cuda:
         raise RuntimeError("tad_dftd4_amd runs on a ROCm device; got CPU tensors")
