@@ -23,234 +23,12 @@ namespace {
 // pivoted-LU kernel below.
 // --------------------------------------------------------------------------
 
-// ---- blocked Cholesky (16-column blocks) on a packed lower triangle -------
-//
-// Row i of the matrix starts at L + tri(i). For each block column kb:
-//  1. wave 0 factorises the diagonal 16 x 16 block D in registers (lane r
-//     holds row r; entries are broadcast with v_readlane, no LDS round trip)
-//     and stores X = D^-1 (lower triangular) in its place;
-//  2. every panel row below becomes a X^T (a = the row's block entries) and
-//     the carried right-hand sides become X b: independent per thread;
-//  3. the trailing triangle is updated in register tiles.
-// The substitutions read X from the stored factor in the same way, so each
-// solve step is a small parallel matrix-vector product between two barriers
-// and no thread runs a serial dependent chain longer than 16 terms.
-// All helpers are force-inlined so that pointers into LDS keep their
-// address space (ds_* instructions rather than flat ones).
-
-constexpr int kNB = 16;
+constexpr int kNB = 16;  // columns of a block
 
 __device__ __forceinline__ double lane_bcast(double v, int src) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
   const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
   return __hiloint2double(hi, lo);
-}
-
-// Factor the diagonal block at kb (nb <= 16 rows) on wave 0 and overwrite it
-// with the inverse of its Cholesky factor. Rows nb..15 are padded with the
-// identity (their columns never mix with the real rows: their off-diagonal
-// entries are zero and stay zero). Returns non-zero (uniform over the wave) if a pivot was not
-// positive; the block is then left unspecified.
-template <typename P>
-__device__ __forceinline__ int chol_diag_block(P L, int kb, int nb) {
-  const int lane = threadIdx.x & 63;
-  double d[kNB];
-#pragma unroll
-  for (int c = 0; c < kNB; ++c) {
-    double v = (c == lane) ? 1.0 : 0.0;
-    if (lane < nb && c <= lane) v = L[tri(kb + lane) + kb + c];
-    d[c] = v;
-  }
-  double invd[kNB];
-  int bad = 0;
-#pragma unroll
-  for (int j = 0; j < kNB; ++j) {
-    const double piv = lane_bcast(d[j], j);
-    bad |= !(piv > 0.0);
-    // 1 / sqrt(piv): hardware estimate and two Newton steps (the diagonal
-    // of the factor itself is never needed, only its reciprocal)
-    const double pv = piv > 0.0 ? piv : 1.0;
-    double inv = __builtin_amdgcn_rsq(pv);
-    inv = inv * fma(-0.5 * pv * inv, inv, 1.5);
-    inv = inv * fma(-0.5 * pv * inv, inv, 1.5);
-    const double s = pv * inv;
-    invd[j] = inv;
-    // Lanes above the diagonal (lane < j) carry junk from here on in d[j] and
-    // in the columns they update; only lanes >= column are ever broadcast
-    // (pivots and L[c][j] with c > j), so the junk is never read.
-    d[j] = lane == j ? s : d[j] * inv;
-#pragma unroll
-    for (int c = j + 1; c < kNB; ++c) d[c] = fma(-d[j], lane_bcast(d[j], c), d[c]);
-  }
-  // lane r forms column r of X = D^-1 by forward substitution
-  double x[kNB];
-#pragma unroll
-  for (int i = 0; i < kNB; ++i) {
-    double s = (i == lane) ? 1.0 : 0.0;
-#pragma unroll
-    for (int k = 0; k < i; ++k) s = fma(-lane_bcast(d[k], i), x[k], s);
-    x[i] = s * invd[i];
-  }
-  if (lane < nb) {
-#pragma unroll
-    for (int i = 0; i < kNB; ++i)
-      if (i >= lane && i < nb) L[tri(kb + i) + kb + lane] = x[i];
-  }
-  return bad;
-}
-
-// Panel row i (full block, nb = 16): L[i][kb..kb+16) <- a X^T.
-template <typename P>
-__device__ __forceinline__ void panel_row(P L, int kb, int i) {
-  P Li = L + tri(i) + kb;
-  double a[kNB];
-#pragma unroll
-  for (int c = 0; c < kNB; ++c) a[c] = Li[c];
-#pragma unroll
-  for (int c = 0; c < kNB; ++c) {
-    P Xc = L + tri(kb + c) + kb;
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k <= c; ++k) s = fma(a[k], Xc[k], s);
-    Li[c] = s;
-  }
-}
-
-// Block forward step on a vector: v[kb..kb+nb) <- X v[kb..kb+nb), copied to y.
-template <typename P, typename V>
-__device__ __forceinline__ void block_lower(P L, int kb, int nb, V v, double* y) {
-  double a[kNB];
-#pragma unroll
-  for (int c = 0; c < kNB; ++c) a[c] = c < nb ? v[kb + c] : 0.0;
-#pragma unroll
-  for (int c = 0; c < kNB; ++c) {
-    if (c < nb) {
-      P Xc = L + tri(kb + c) + kb;
-      double s = 0.0;
-#pragma unroll
-      for (int k = 0; k <= c; ++k) s = fma(a[k], Xc[k], s);
-      v[kb + c] = s;
-      y[c] = s;
-    }
-  }
-}
-
-// Trailing update of one T x T tile: rows r0 + T ti + a, columns r0 + T tj + b
-// (lower part only) lose the product of their panel rows.
-template <int T, typename P>
-__device__ __forceinline__ void trailing_tile(P L, int kb, int r0, int ti, int tj, int n) {
-  const int i0 = r0 + T * ti, j0 = r0 + T * tj;
-  P pi[T], pj[T];
-#pragma unroll
-  for (int a = 0; a < T; ++a) {
-    pi[a] = L + tri(min(i0 + a, n - 1)) + kb;
-    pj[a] = L + tri(min(j0 + a, n - 1)) + kb;
-  }
-  double acc[T][T];
-#pragma unroll
-  for (int a = 0; a < T; ++a)
-#pragma unroll
-    for (int b = 0; b < T; ++b) acc[a][b] = 0.0;
-#pragma unroll 1  // a rolled loop keeps only one chunk of rows in registers
-  for (int c0 = 0; c0 < kNB; c0 += 4) {
-    double xi[T][4], xj[T][4];
-#pragma unroll
-    for (int a = 0; a < T; ++a)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        xi[a][c] = pi[a][c0 + c];
-        xj[a][c] = pj[a][c0 + c];
-      }
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int a = 0; a < T; ++a)
-#pragma unroll
-        for (int b = 0; b < T; ++b) acc[a][b] = fma(xi[a][c], xj[b][c], acc[a][b]);
-  }
-#pragma unroll
-  for (int a = 0; a < T; ++a)
-#pragma unroll
-    for (int b = 0; b < T; ++b) {
-      const int i = i0 + a, j = j0 + b;
-      if (i < n && j <= i) L[tri(i) + j] -= acc[a][b];
-    }
-}
-
-__device__ __forceinline__ void tile_index(int e, int& ti, int& tj) {
-  int r = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-  while (r * (r + 1) / 2 > e) --r;
-  while ((r + 1) * (r + 2) / 2 <= e) ++r;
-  ti = r;
-  tj = e - r * (r + 1) / 2;
-}
-
-// Trailing triangle (rows and columns r0..n-1) in T x T tiles, plus the
-// update of the two carried right-hand sides by the block's solution y.
-template <int T, bool RHS, typename P, typename V>
-__device__ __forceinline__ void trailing_update(P L, int kb, int n, V rb, V re,
-                                                const double* yblk) {
-  const int r0 = kb + kNB;
-  const int mr = n - r0;
-  const int mt = (mr + T - 1) / T;
-  const int ntl = mt * (mt + 1) / 2;
-  // right-hand-side rows first, on the threads that the tiles leave idle last
-  const int first = (256 - (ntl + mr) % 256) % 256;
-  for (int e = threadIdx.x - first; RHS && e < mr; e += 256) {
-    if (e < 0) continue;
-    const int i = r0 + e;
-    P Pi = L + tri(i) + kb;
-    double sb = 0.0, se = 0.0;
-#pragma unroll
-    for (int c = 0; c < kNB; ++c) {
-      sb = fma(Pi[c], yblk[c], sb);
-      se = fma(Pi[c], yblk[kNB + c], se);
-    }
-    rb[i] -= sb;
-    re[i] -= se;
-  }
-  for (int e = threadIdx.x; e < ntl; e += 256) {
-    int ti, tj;
-    tile_index(e, ti, tj);
-    trailing_tile<T>(L, kb, r0, ti, tj, n);
-  }
-}
-
-// Blocked right-looking Cholesky of the assembled n x n lower triangle; the
-// diagonal blocks end up holding their inverses. With RHS, two right-hand
-// sides are carried along (forward substitution fused): on return rb, re
-// hold L^-1 b and L^-1 e. yblk: 2 * kNB doubles of LDS, flag: one double.
-// Returns non-zero if a pivot was not positive.
-template <bool RHS, typename P, typename V>
-__device__ __forceinline__ int chol_factor(P L, int n, V rb, V re, double* yblk,
-                                           double* flag) {
-  const int tid = threadIdx.x;
-  constexpr int nrhs = RHS ? 2 : 0;
-  for (int kb = 0; kb < n; kb += kNB) {
-    const int nb = min(kNB, n - kb);
-    if (tid < 64) {
-      const int bad = chol_diag_block(L, kb, nb);
-      if (tid == 0) flag[0] = bad ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    if (flag[0] != 0.0) return 1;  // uniform
-    const int mr = n - kb - nb;    // > 0 only for full blocks
-    for (int t2 = tid; t2 < mr + nrhs; t2 += 256) {
-      if (t2 < mr)
-        panel_row(L, kb, kb + nb + t2);
-      else if (RHS)
-        block_lower(L, kb, nb, t2 == mr ? rb : re, yblk + (t2 - mr) * kNB);
-    }
-    __syncthreads();
-    if (mr > 0) {
-      if (mr >= 48)
-        trailing_update<4, RHS>(L, kb, n, rb, re, yblk);
-      else
-        trailing_update<2, RHS>(L, kb, n, rb, re, yblk);
-    }
-    __syncthreads();
-  }
-  return 0;
 }
 
 // ---- L D L^T by whole waves (molecules held in LDS) ------------------------
@@ -331,11 +109,11 @@ __device__ __forceinline__ void panel_columns(Panel& P, double t, double t2) {
 // by the pivot.
 constexpr int kFcmpOgt = 2;  // ordered and greater than
 
-template <bool ROWS, int J>
-__device__ __forceinline__ void panel_step(Panel& P, int nb) {
+template <bool ROWS, bool FULL, bool WLDS, int J>
+__device__ __forceinline__ void panel_step(Panel& P, int nb, double* W) {
   if constexpr (J + 1 < kNB) {
     P.w[J + 1] = 0.0;
-    if (J + 1 < nb) {  // uniform (columns past nb are padding)
+    if (FULL || J + 1 < nb) {  // uniform (columns past nb are padding)
       const double t = -P.D[J] * P.w[J], t2 = ROWS ? -P.d[J] * P.w[J] : 0.0;
       panel_columns<ROWS, J, J + 1, J + 2>(P, t, t2);
       const double pv = row_bcast<J + 1>(P.D[J + 1]);
@@ -346,19 +124,26 @@ __device__ __forceinline__ void panel_step(Panel& P, int nb) {
       const double e2 = fma(e, e, e);
       panel_columns<ROWS, J, J + 7, J + 9>(P, t, t2);
       P.w[J + 1] = fma(r, e2, r);  // third-order step: 1 / pv
+      if (WLDS) W[J + 1] = P.w[J + 1];  // (every lane the same value)
       P.good &= __builtin_amdgcn_fcmp(pv, 0.0, kFcmpOgt);
       panel_columns<ROWS, J, J + 9, kNB>(P, t, t2);
+      __builtin_amdgcn_sched_barrier(0);  // (hoisting across columns only costs registers)
     }
-    panel_step<ROWS, J + 1>(P, nb);
+    panel_step<ROWS, FULL, WLDS, J + 1>(P, nb, W);
   }
 }
 
-template <bool ROWS>
-__device__ __forceinline__ void panel_factor(Panel& P, int nb) {
+// (whole panels have no branches between their columns: 2.1 k clocks for the
+// block alone, 3.0 k with the rows below, against 4-5 k)
+// WLDS: the reciprocal pivots also go to W in LDS, for a caller that has no
+// registers to keep them.
+template <bool ROWS, bool FULL, bool WLDS = false>
+__device__ __forceinline__ void panel_factor(Panel& P, int nb, double* W = nullptr) {
   const double pv = row_bcast<0>(P.D[0]);
   P.good = __builtin_amdgcn_fcmp(pv, 0.0, kFcmpOgt);
   P.w[0] = rcp_nt(pv);
-  panel_step<ROWS, 0>(P, nb);
+  if (WLDS) W[0] = P.w[0];
+  panel_step<ROWS, FULL, WLDS, 0>(P, nb, W);
 }
 
 // Left-looking update of the 16 x 16 tile (TWO: and a second one) of block
@@ -428,6 +213,37 @@ struct EeqSmall {
   int* idx;            // one per wave
 };
 
+// A wave's share of a panel in LDS: its 64 rows below the block (`row`; a border
+// row goes to `border`, not divided by the pivots).
+template <bool FULL>
+__device__ __forceinline__ void panel_rows(Panel& P, double* L, int n, int kb, int nb, int row,
+                                           double* border) {
+  panel_factor<true, FULL>(P, nb);
+  if (FULL && row < n) {  // (there are rows below a full block only)
+    double* Lr = L + tri(row) + kb;
+#pragma unroll
+    for (int c = 0; c < kNB; ++c) Lr[c] = P.d[c] * P.w[c];
+  }
+  if (border != nullptr) {
+#pragma unroll
+    for (int c = 0; c < kNB; ++c) border[c] = P.d[c];
+  }
+}
+
+// The block itself, by one wave: L below the diagonal, the pivots on it.
+template <bool FULL>
+__device__ __forceinline__ void panel_block(Panel& P, double* L, int kb, int nb, int* flag) {
+  const int lane = threadIdx.x & 63;
+  panel_factor<false, FULL>(P, nb);
+  if (lane == 0) *flag = P.good != 0ull ? 0 : 1;
+  if (lane < nb) {
+    double* Dr = L + tri(kb + lane) + kb;
+#pragma unroll
+    for (int c = 0; c < kNB; ++c)
+      if (c <= lane) Dr[c] = c < lane ? P.D[c] * P.w[c] : P.D[c];
+  }
+}
+
 // Factor the assembled n x n matrix (n + 2 <= 208) with its border rows:
 // thread i < n holds b_i and e_i, on return L^-1 b and L^-1 e. Three waves do
 // the rows of the panels and a fourth the block itself, all NW >= 4 the
@@ -494,25 +310,15 @@ __device__ __forceinline__ int ldl_factor_waves(double* L, int n, double& vb, do
     }
     __syncthreads();  // the block is read before wave 3 replaces it
     if (rows) {
-      panel_factor<true>(P, nb);
-      if (row < n) {  // (only below a full block)
-        double* Lr = L + tri(row) + kb;
-#pragma unroll
-        for (int c = 0; c < kNB; ++c) Lr[c] = P.d[c] * P.w[c];
-      }
-      if (is_border) {  // L^-1 b and L^-1 e are not divided by the pivots
-#pragma unroll
-        for (int c = 0; c < kNB; ++c) sm.y[border][c] = P.d[c];
-      }
+      if (nb == kNB)
+        panel_rows<true>(P, L, n, kb, nb, row, is_border ? sm.y[border] : nullptr);
+      else
+        panel_rows<false>(P, L, n, kb, nb, row, is_border ? sm.y[border] : nullptr);
     } else if (wave == 3) {
-      panel_factor<false>(P, nb);
-      if (lane == 0) sm.idx[0] = P.good != 0ull ? 0 : 1;
-      if (lane < nb) {
-        double* Dr = L + tri(kb + lane) + kb;
-#pragma unroll
-        for (int c = 0; c < kNB; ++c)
-          if (c <= lane) Dr[c] = c < lane ? P.D[c] * P.w[c] : P.D[c];
-      }
+      if (nb == kNB)
+        panel_block<true>(P, L, kb, nb, sm.idx);
+      else
+        panel_block<false>(P, L, kb, nb, sm.idx);
     }
     __syncthreads();
     if (sm.idx[0]) return 1;
@@ -864,7 +670,7 @@ inline int eeq_waves(int64_t N) { return N > 140 ? 8 : 4; }
 // b-th smallest molecule: half the CUs hold the solve, and the others are
 // free from the start for the three-body kernel on the companion stream.
 template <int NW, int NV, bool PAIRED>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_eeq_chol(
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 3 : 2))) void k_eeq_chol(
     DevTables t, Params p, Inputs in, Work w, int doubles, int ordered) {
   extern __shared__ double smem[];
   __shared__ double s_blk[4][kNB];
@@ -880,6 +686,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     return;
   }
   const int64_t b2 = w.B - 1 - b;
+#pragma unroll 1
   for (int k = 0; k < (b2 > b ? 2 : 1); ++k) {
     if (k) __syncthreads();  // the LDS is reused
     eeq_chol_molecule<NW, NV>(t, p, in, w, w.eqord[k ? b2 : b], smem, doubles, sm);
@@ -1063,19 +870,27 @@ __global__ __launch_bounds__(256) void k_eeq_lu(DevTables t, Params p, Inputs in
 //
 // The matrix lives in HBM in the LU workspace as row-major rows of length N:
 // rows 0..n-1 hold the lower triangle of C, row n holds b and row n+1 holds
-// e. With the two border rows below the matrix, the forward substitution of
-// b and e is just the panel and trailing steps applied to those rows. Per
-// 64-column block step:
-//   k_tf_diag   one work-group factors the 64 x 64 diagonal block in LDS
-//               (16-column blocked Cholesky), forms X = D^-1 and stores it in
-//               place of D;
-//   k_tf_panel  64-row tiles below the block (and the border rows) become
-//               A X^T;
-//   k_tf_update 64 x 64 tiles of the trailing triangle lose P_I P_J^T.
-// The substitutions then run one launch per block step: every work-group of
-// a molecule recomputes the block's 64-entry solution from the same inputs
-// and work-group 0 alone stores it, so no work-group reads what another
-// writes within a launch.
+// e (the forward substitution of b and e is the elimination of those rows).
+// L D L^T in 64-column blocks, one launch per block (k_tl_step): the launch of
+// block kb applies block kb - 64 to everything behind it, and factors its own.
+//  - A work-group of panel row tile y updates the diagonal tile and its own
+//    64-row tile (MFMA), factors the diagonal tile in LDS and finishes its own
+//    rows beside it. Every one factors the same diagonal tile, so the rows
+//    need no other launch; work-group 0 alone stores it.
+//  - The other work-groups update the 64 x 64 tiles of the trailing triangle.
+// The finished diagonal tile goes transposed into the upper triangle of A (the
+// tile itself is still being read by the other work-groups), its pivots to
+// w.dpiv; the rows below are finished in place. So a work-group only reads
+// what earlier launches wrote or what it writes itself.
+// The substitutions go by 256 entries: one work-group per molecule solves them
+// (k_tl_solve, 64 at a time with the vector in LDS), then many work-groups take
+// their share off the rest of the vector (k_tl_gemv).
+// What bounds it: the panel chain (four 16-column panels a launch) and launch
+// latency. One 701-atom molecule (11 blocks): 26 us a launch of k_tl_step
+// (loads and update 6-12 us, panels 8) where the three launches per block
+// that were here before took 115 (diagonal block 65, panel 23, update 27), and
+// 22 us per 256 entries of a substitution against 60-100; its energy and
+// forces through autograd 2.4 -> 1.3 ms.
 // ==========================================================================
 
 constexpr int kTB = 64;
@@ -1142,177 +957,293 @@ __global__ __launch_bounds__(256) void k_tf_assemble(DevTables t, Params p, Inpu
   }
 }
 
-// Factor the diagonal block at kb and replace it by the inverse of its factor.
-// The tiled kernels take their LDS as dynamic shared memory and at most 64
-// VGPRs (eight waves per SIMD as far as registers go): a work-group then fits
-// beside the three-body kernel's waves (two per SIMD with 220 VGPRs) on any
-// CU instead of waiting until one is nearly empty.
-constexpr size_t kTfDiagLds = sizeof(double) * (kTB * (kTB + 1) / 2 + kTB * kTB + kNB * kTB +
-                                                2 * kNB + 2);
-constexpr size_t kTfTileLds = sizeof(double) * 2 * kTB * (kTB + 1);
+// The tiled kernels take their LDS as dynamic shared memory and at most 80
+// VGPRs: a work-group then fits beside the three-body kernel's waves (two per
+// SIMD with 216 VGPRs, 86 KB of LDS per CU) on any CU instead of waiting until
+// one is nearly empty.
+constexpr int kTS = kTB + 1;  // row stride of a tile in LDS
+constexpr size_t kTlLds = sizeof(double) * (2 * kTB * kTS + kTB + 3 * kNB + 2);
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_tf_diag(
-    Inputs in, Work w, int kb) {
-  tf_priority();
-  extern __shared__ double s_tf[];
-  double* F = s_tf;                                             // [tri(kTB)]
-  auto X = reinterpret_cast<double (*)[kTB]>(F + kTB * (kTB + 1) / 2);  // [kTB][kTB]
-  auto T = reinterpret_cast<double (*)[kTB]>(&X[kTB][0]);      // [kNB][kTB]
-  double* s_small = &T[kNB][0];                                 // [2 kNB + 2]
-  const int64_t m = blockIdx.x;
-  if (!tf_active(in, w, m, kb)) return;
-  const int tid = threadIdx.x;
-  const int64_t N = w.N;
-  const int n = w.natom[m];
-  const int nb = min(kTB, n - kb);
-  double* A = tf_matrix(w, m);
-  for (int e = tid; e < tri(nb); e += 256) {
-    const int r = incl_row(e), c = e - tri(r);
-    F[e] = A[(size_t)(kb + r) * N + kb + c];
+// c0 (TWO: and c1) -= rows r0 .. of P times rows q0 .. (q1 ..) of Q over K
+// columns, the columns weighted by piv[k * ps] (P, Q: tiles in LDS).
+template <bool TWO>
+__device__ __forceinline__ void tl_product(const double* P, int r0, const double* Q, int q0, int q1,
+                                           const double* piv, int ps, int K, d4_acc& c0,
+                                           d4_acc& c1) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const double* pa = P + (r0 + l16) * kTS + 4 * g;
+  const double* pb = Q + (q0 + l16) * kTS + 4 * g;
+  const double* pc = Q + (q1 + l16) * kTS + 4 * g;
+  const double* pd = piv + 4 * g * ps;
+#pragma unroll 1
+  for (int k = 0; k < K; k += kNB) {
+    double a[4], b[4], c[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      a[s] = -pa[k + s] * pd[(k + s) * ps];
+      b[s] = pb[k + s];
+      if (TWO) c[s] = pc[k + s];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], c0, 0, 0, 0);
+      if (TWO) c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], c[s], c1, 0, 0, 0);
+    }
+  }
+}
+
+// Rows r0 .. r0 + 63 (below `rows`, else zero), columns c0 .. c0 + 63 (below
+// `cols`, else zero) of A into a tile, eight loads in flight per thread.
+__device__ __forceinline__ void tl_load(const double* A, int64_t N, int r0, int rows, int c0,
+                                        int cols, double* T) {
+  const int c = threadIdx.x & (kTB - 1), rr = threadIdx.x >> 6;
+  const double* p = A + (size_t)r0 * N + c0 + min(c, cols - 1);
+#pragma unroll 1
+  for (int h = 0; h < 2; ++h) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[min(rr + 32 * h + 4 * u, rows - 1) * (int)N];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int r = rr + 32 * h + 4 * u;
+      T[r * kTS + c] = r < rows && c < cols ? v[u] : 0.0;
+    }
+  }
+}
+
+// A wave's share of a 16-column panel in the tiles (block of D at c0, nbs
+// columns used): the block itself (ROWS = false: L below the diagonal, the
+// pivots on it, junk that nothing reads right of it), or a row per lane
+// (`row` null: none). All waves read the block before any writes it. W: 16
+// doubles of LDS of the wave.
+template <bool ROWS, bool FULL>
+__device__ __forceinline__ void tl_panel(double* D, int c0, int nbs, double* row, double* W,
+                                         int* flag) {
+  const int lane = threadIdx.x & 63;
+  Panel P;
+  const double* Dl = D + (c0 + (lane & 15)) * kTS + c0;
+  const double* rl = ROWS && row != nullptr ? row : Dl;
+#pragma unroll
+  for (int c = 0; c < kNB; ++c) {
+    P.D[c] = Dl[FULL ? c : min(c, nbs - 1)];
+    if (ROWS) P.d[c] = rl[FULL ? c : min(c, nbs - 1)];
   }
   __syncthreads();
-  if (chol_factor<false>(F, nb, (double*)nullptr, (double*)nullptr, s_small,
-                         s_small + 2 * kNB)) {
-    if (tid == 0) w.status[m] |= kStatusLU;
+  panel_factor<ROWS, FULL, true>(P, nbs, W);
+  if (ROWS) {
+    if (row != nullptr) {
+#pragma unroll
+      for (int c = 0; c < kNB; ++c)
+        if (FULL || c < nbs) row[c] = P.d[c] * W[c];
+    }
     return;
   }
-  // X = F^-1 by block forward substitution over the 16-row sub-blocks, whose
-  // own inverses the factorisation left on the diagonal of F:
-  // X_s = X16_s (I_s - F_{s,<s} X_{<s})
-  for (int r0 = 0; r0 < nb; r0 += kNB) {
-    const int rn = min(kNB, nb - r0);
-    const int ncol = r0 + rn;
-    for (int e = tid; e < rn * ncol; e += 256) {
-      const int r = e / ncol, c = e - r * ncol;
-      const double* Fr = F + tri(r0 + r);
-      double sacc = (r0 + r == c) ? 1.0 : 0.0;
-      for (int k = c; k < r0; ++k) sacc = fma(-Fr[k], X[k][c], sacc);
-      T[r][c] = sacc;
+  if (lane == 0) *flag = P.good != 0ull ? 0 : 1;
+  if (lane < nbs) {
+    double* Dr = D + (c0 + lane) * kTS + c0;
+    double pivot = P.D[0];
+#pragma unroll
+    for (int c = 0; c < kNB; ++c) {
+      pivot = lane == c ? P.D[c] : pivot;
+      Dr[c] = P.D[c] * (FULL || c < nbs ? W[c] : 0.0);
     }
-    __syncthreads();
-    for (int e = tid; e < rn * ncol; e += 256) {
-      const int r = e / ncol, c = e - r * ncol;
-      const double* Xr = F + tri(r0 + r) + r0;
-      double sacc = 0.0;
-      for (int rr = 0; rr <= r; ++rr) sacc = fma(Xr[rr], T[rr][c], sacc);
-      X[r0 + r][c] = c <= r0 + r ? sacc : 0.0;
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < tri(nb); e += 256) {
-    const int r = incl_row(e), c = e - tri(r);
-    A[(size_t)(kb + r) * N + kb + c] = X[r][c];
+    Dr[lane] = pivot;
   }
 }
 
-// Panel tile: rows kb + nb + 64 y ... of the matrix and border become A X^T.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_tf_panel(
-    Inputs in, Work w, int kb) {
+template <bool FULL>
+__device__ __forceinline__ void tl_panels(double* D, double* T, bool own, int dmax, int c0, int nbs,
+                                          double* W, int* flag, int wave) {
+  const int lane = threadIdx.x & 63;
+  if (wave == 0 && own) {
+    tl_panel<true, FULL>(D, c0, nbs, T + lane * kTS + c0, W, flag);
+  } else if (wave == 1) {
+    const int r = c0 + nbs + lane;
+    tl_panel<true, FULL>(D, c0, nbs, r < dmax ? D + r * kTS + c0 : nullptr, W + kNB, flag);
+  } else if (wave == 3) {
+    tl_panel<false, FULL>(D, c0, nbs, nullptr, W + 2 * kNB, flag);
+  } else {
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_tl_step(
+    Inputs in, Work w, int kb, int npanel) {
   tf_priority();
-  extern __shared__ double s_tf[];
-  auto Xs = reinterpret_cast<double (*)[kTB + 1]>(s_tf);  // [kTB][kTB + 1]
-  auto As = Xs + kTB;                                      // [kTB][kTB + 1]
+  extern __shared__ double s_tl[];
+  double* X = s_tl;               // [64][65]
+  double* Y = X + kTB * kTS;      // [64][65]
+  double* piv = Y + kTB * kTS;    // [64] pivots of block kb - 64
+  double* W = piv + kTB;          // [3][16] reciprocal pivots
+  int* flag = reinterpret_cast<int*>(W + 3 * kNB);
   const int64_t m = blockIdx.x;
   if (!tf_active(in, w, m, kb)) return;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t N = w.N;
-  const int n = w.natom[m];
-  const int nb = min(kTB, n - kb);
-  const int r0 = kb + nb + (int)blockIdx.y * kTB;
-  const int rows = min(kTB, n + 2 - r0);
+  const int n = w.natom[m], last = n + 2;  // rows with the border
+  const int nb = min(kTB, n - kb), pk = kb - kTB;
+  double* A = tf_matrix(w, m);
+  double* dpiv = w.dpiv + m * N;
+  const int y = (int)blockIdx.y;
+  if (kb > 0 && tid < kTB) piv[tid] = dpiv[pk + tid];
+
+  if (y >= npanel) {  // a trailing tile
+    const int e = y - npanel, r0 = kb + kTB;
+    if (r0 >= n) return;
+    const int I = incl_row(e), J = e - tri(I);
+    const int i0 = r0 + I * kTB, j0 = r0 + J * kTB;
+    if (i0 >= last || j0 >= n) return;
+    tl_load(A, N, i0, last - i0, pk, kTB, X);
+    tl_load(A, N, j0, n - j0, pk, kTB, Y);
+    __syncthreads();
+#pragma unroll 1
+    for (int ct = 0; ct < 4; ct += 2) {
+      d4_acc c[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int j = j0 + kNB * (ct + h) + l16;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = i0 + kNB * wave + 4 * r + g;
+          c[h][r] = i < last && j < n && j <= i ? A[(size_t)i * N + j] : 0.0;
+        }
+      }
+      tl_product<true>(X, kNB * wave, Y, kNB * ct, kNB * ct + kNB, piv, 1, kTB, c[0], c[1]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int j = j0 + kNB * (ct + h) + l16;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = i0 + kNB * wave + 4 * r + g;
+          if (i < last && j < n && j <= i) A[(size_t)i * N + j] = c[h][r];
+        }
+      }
+    }
+    return;
+  }
+
+  // a panel row tile: D the diagonal tile (its rows past nb: border rows), T
+  // the work-group's own rows
+  const int r0 = kb + y * kTB, rows = last - r0, drows = last - kb;
   if (rows <= 0) return;
-  double* A = tf_matrix(w, m);
-  for (int e = tid; e < kTB * kTB; e += 256) {
-    const int r = e >> 6, c = e & (kTB - 1);
-    Xs[r][c] = (r < nb && c <= r) ? A[(size_t)(kb + r) * N + kb + c] : 0.0;
-    As[r][c] = (r < rows && c < nb) ? A[(size_t)(r0 + r) * N + kb + c] : 0.0;
-  }
-  __syncthreads();
-  const int tr = tid >> 4, tc = tid & 15;
-  double acc[4][4];
+  const bool own = y > 0;
+  double* D = Y;
+  double* T = X;
+  if (kb == 0) {
+    tl_load(A, N, 0, drows, 0, nb, D);
+    if (own) tl_load(A, N, r0, rows, 0, nb, T);
+    __syncthreads();
+  } else {
+    d4_acc o[4];
+    if (own) {
+      const double* Ao = A + (size_t)r0 * N + kb;
+      tl_load(A, N, r0, rows, pk, kTB, Y);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+      for (int ct = 0; ct < 4; ++ct) {
+        const int c = kNB * ct + l16;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-  for (int k = 0; k < kTB; ++k) {
-    double av[4], xv[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      av[a] = As[4 * tr + a][k];
-      xv[a] = Xs[4 * tc + a][k];
+        for (int r = 0; r < 4; ++r) {
+          const int i = kNB * wave + 4 * r + g;
+          o[ct][r] = i < rows && c < nb ? Ao[i * (int)N + c] : 0.0;
+        }
+      }
     }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = fma(av[a], xv[b], acc[a][b]);
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int r = 4 * tr + a, c = 4 * tc + b;
-      if (r < rows && c < nb) A[(size_t)(r0 + r) * N + kb + c] = acc[a][b];
+    tl_load(A, N, kb, drows, pk, kTB, X);
+    __syncthreads();
+    if (own) {
+      tl_product<true>(Y, kNB * wave, X, 0, kNB, piv, 1, kTB, o[0], o[1]);
+      tl_product<true>(Y, kNB * wave, X, 2 * kNB, 3 * kNB, piv, 1, kTB, o[2], o[3]);
+      __syncthreads();  // Y is free
     }
-}
+    // the ten 16 x 16 tiles on and below the diagonal, as five pairs: wave q
+    // row 3 columns (0, 1), row 3 columns (2, 3), row 2 columns (0, 1) and row
+    // 1 columns (0, 1), then waves 0 and 1 the diagonal tiles (2, 2) and (0, 0)
+#pragma unroll 1
+    for (int q = wave; q < 6; q += 4) {
+      const int rt = q < 2 ? 3 : q == 2 || q == 4 ? 2 : q == 3 ? 1 : 0;
+      const int ct = q == 1 ? 2 : q == 4 ? 2 : 0;
+      const bool two = q < 4;
+      d4_acc v[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int c = kNB * (ct + h) + l16;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = kNB * rt + 4 * r + g;
+          v[h][r] = (h == 0 || two) && i < drows && c < nb && c <= i
+                        ? A[(size_t)(kb + i) * N + kb + c] : 0.0;
+        }
+      }
+      if (two)
+        tl_product<true>(X, kNB * rt, X, kNB * ct, kNB * ct + kNB, piv, 1, kTB, v[0], v[1]);
+      else
+        tl_product<false>(X, kNB * rt, X, kNB * ct, 0, piv, 1, kTB, v[0], v[1]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (h == 0 || two) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            D[(kNB * rt + 4 * r + g) * kTS + kNB * (ct + h) + l16] = v[h][r];
+        }
+    }
+    __syncthreads();  // X is free
+    if (own) {
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          T[(kNB * wave + 4 * r + g) * kTS + kNB * ct + l16] = o[ct][r];
+    }
+    __syncthreads();
+  }
 
-// Trailing tile (I, J): rows r0 + 64 I.. (matrix and border), columns
-// r0 + 64 J.. of the matrix, r0 = kb + 64, lose P_I P_J^T.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_tf_update(
-    Inputs in, Work w, int kb) {
-  tf_priority();
-  extern __shared__ double s_tf[];
-  auto Pi = reinterpret_cast<double (*)[kTB + 1]>(s_tf);  // [kTB][kTB + 1]
-  auto Pj = Pi + kTB;                                      // [kTB][kTB + 1]
-  const int64_t m = blockIdx.x;
-  if (!tf_active(in, w, m, kb)) return;
-  const int tid = threadIdx.x;
-  const int64_t N = w.N;
-  const int n = w.natom[m];
-  const int r0 = kb + kTB;
-  if (r0 >= n) return;
-  const int nI = (n + 2 - r0 + kTB - 1) / kTB, nJ = (n - r0 + kTB - 1) / kTB;
-  const int e = (int)blockIdx.y;
-  if (e >= nI * (nI + 1) / 2) return;
-  const int I = incl_row(e), J = e - tri(I);
-  if (J >= nJ) return;
-  const int i0 = r0 + I * kTB, j0 = r0 + J * kTB;
-  double* A = tf_matrix(w, m);
-  for (int x = tid; x < kTB * kTB; x += 256) {
-    const int r = x >> 6, c = x & (kTB - 1);
-    Pi[r][c] = (i0 + r < n + 2) ? A[(size_t)(i0 + r) * N + kb + c] : 0.0;
-    Pj[r][c] = (j0 + r < n) ? A[(size_t)(j0 + r) * N + kb + c] : 0.0;
-  }
-  __syncthreads();
-  const int tr = tid >> 4, tc = tid & 15;
-  double acc[4][4];
+  const int dmax = min(kTB, drows);
+  for (int c0 = 0; c0 < nb; c0 += kNB) {
+    const int nbs = min(kNB, nb - c0);
+    if (c0 > 0) {
+      // left-looking update of the 16 columns in D's rows from c0 on and in T
+      const int nd = 4 - c0 / kNB, total = nd + (own ? 4 : 0);
+      for (int t = wave; t < total; t += 4) {
+        double* M = t < nd ? D : T;
+        const int rt = t < nd ? c0 + kNB * t : kNB * (t - nd);
+        d4_acc c = {0.0, 0.0, 0.0, 0.0};
+        tl_product<false>(M, rt, D, c0, 0, D, kTS + 1, c0, c, c);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-  for (int k = 0; k < kTB; ++k) {
-    double iv[4], jv[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      iv[a] = Pi[4 * tr + a][k];
-      jv[a] = Pj[4 * tc + a][k];
+        for (int r = 0; r < 4; ++r) M[(rt + 4 * r + g) * kTS + c0 + l16] += c[r];
+      }
+      __syncthreads();
     }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = fma(iv[a], jv[b], acc[a][b]);
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int i = i0 + 4 * tr + a, j = j0 + 4 * tc + b;
-      if (i < n + 2 && j < n && j <= i) A[(size_t)i * N + j] -= acc[a][b];
+    if (nbs == kNB)
+      tl_panels<true>(D, T, own, dmax, c0, nbs, W, flag, wave);
+    else
+      tl_panels<false>(D, T, own, dmax, c0, nbs, W, flag, wave);
+    __syncthreads();
+    if (*flag) {  // uniform
+      if (y == 0 && tid == 0) w.status[m] |= kStatusLU;
+      return;
     }
+  }
+
+  if (own) {
+    for (int e = tid; e < kTB * kTB; e += 256) {
+      const int r = e >> 6, c = e & (kTB - 1);
+      if (r < rows && c < nb) A[(size_t)(r0 + r) * N + kb + c] = T[r * kTS + c];
+    }
+    return;
+  }
+  for (int e = tid; e < kTB * kTB; e += 256) {
+    const int c = e >> 6, r = e & (kTB - 1);
+    if (c < r && r < nb) A[(size_t)(kb + c) * N + kb + r] = D[r * kTS + c];
+  }
+  if (tid < nb) dpiv[kb + tid] = D[tid * (kTS + 1)];
+  for (int r = nb; r < dmax; ++r)  // border rows in the diagonal tile
+    if (tid < nb) A[(size_t)(kb + r) * N + kb + tid] = D[r * kTS + tid];
 }
 
 // After the factorisation: charges given or padding, then mu and the
-// right-hand side y_b - mu y_e of the backward substitution (in vec); y_e is
-// kept for the adjoint.
+// right-hand side D^-1 L^-1 (b - mu e) of the backward substitution (in vec);
+// D^-1 L^-1 e is kept for the adjoint.
 __global__ __launch_bounds__(256) void k_tf_reduce(Inputs in, Work w) {
   tf_priority();
   __shared__ double red[2 * kWaves];
@@ -1329,13 +1260,16 @@ __global__ __launch_bounds__(256) void k_tf_reduce(Inputs in, Work w) {
   }
   for (int i = n + tid; i < N; i += 256) q[i] = 0.0;
   if (n == 0 || (w.status[m] & kStatusLU)) return;
+  // the border rows hold D^-1 L^-1 b and D^-1 L^-1 e
   const double* A = tf_matrix(w, m);
-  const double* yb = A + (size_t)n * N;
-  const double* ye = A + (size_t)(n + 1) * N;
+  const double* zb = A + (size_t)n * N;
+  const double* ze = A + (size_t)(n + 1) * N;
+  const double* dpiv = w.dpiv + m * N;
   double sbe = 0.0, see = 0.0;
   for (int i = tid; i < n; i += 256) {
-    sbe = fma(ye[i], yb[i], sbe);
-    see = fma(ye[i], ye[i], see);
+    const double u = ze[i] * dpiv[i];
+    sbe = fma(u, zb[i], sbe);
+    see = fma(u, ze[i], see);
   }
   sbe = block_sum(sbe, red);
   see = block_sum(see, red + kWaves);
@@ -1343,77 +1277,181 @@ __global__ __launch_bounds__(256) void k_tf_reduce(Inputs in, Work w) {
   double* v = w.vec + m * (N + 1);
   double* gz = w.ez + m * N;
   for (int i = tid; i < n; i += 256) {
-    v[i] = fma(-mu, ye[i], yb[i]);
-    gz[i] = ye[i];
+    v[i] = fma(-mu, ze[i], zb[i]);
+    gz[i] = ze[i];
   }
 }
 
-// One backward-substitution step L^T x = v at block kb (descending kb):
-// x_kb = X^T v_kb is stored to dst (zero on padding atoms) by work-group 0;
-// work-group y updates v[j] for j in [256 y, 256 y + 256) below kb.
-__global__ __launch_bounds__(256) void k_tf_bsolve(Inputs in, Work w, int kb,
-                                                   double* dst_base) {
+// Vector entries of one k_tl_solve: one per thread of a work-group of four
+// waves, which fits beside the three-body waves (a work-group of sixteen waits
+// for a CU without any).
+constexpr int kTV = 256;
+constexpr int kTQ = kTB * kTB / kTV;  // tile entries per thread
+constexpr size_t kTlSolveLds = sizeof(double) * (kTB * kTS + kTV + kTB);
+
+// Whether the substitutions of molecule m run (charges solved by this factor).
+__device__ __forceinline__ bool tl_solving(const Inputs& in, const Work& w, int64_t m) {
+  return in.q_in == nullptr && !(w.status[m] & (kStatusLU | kStatusSingular));
+}
+
+// 64 steps of a substitution within a diagonal tile, lane r: entry r of the
+// vector. BACK: x = L^-T v, else y = L^-1 v; T[c][r] = L[r][c], zero unless
+// r > c.
+template <bool BACK>
+__device__ __forceinline__ double tl_tile_solve(const double* T, double v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int h = 0; h < 8; ++h) {
+    double l[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = BACK ? 63 - 8 * h - u : 8 * h + u;
+      l[u] = BACK ? T[lane * kTS + k] : T[k * kTS + lane];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = BACK ? 63 - 8 * h - u : 8 * h + u;
+      v = fma(-l[u], lane_bcast(v, k), v);
+    }
+  }
+  return v;
+}
+
+// Entries s0 .. s0 + kTV - 1 of L^T x = v (BACK, their later entries already
+// taken off) or L y = v; the result goes to w.vec and to dst (BACK: zero on
+// padding atoms).
+template <bool BACK>
+__global__ __launch_bounds__(kTV) __attribute__((amdgpu_waves_per_eu(6))) void k_tl_solve(
+    Inputs in, Work w, int s0, double* dst) {
   tf_priority();
-  __shared__ double xs[kTB];
+  extern __shared__ double s_tl[];
+  double* s_t = s_tl;              // [64][65]
+  double* s_v = s_t + kTB * kTS;   // [kTV]
+  double* s_x = s_v + kTV;         // [64]
   const int64_t m = blockIdx.x;
-  const int y = (int)blockIdx.y;
-  const int tid = threadIdx.x;
   const int64_t N = w.N;
   const int n = w.natom[m];
-  if (in.q_in != nullptr || kb >= n || (w.status[m] & kStatusLU)) return;
-  const int j = y * 256 + tid;
-  if (y > 0 && y * 256 >= kb) return;
-  const int nb = min(kTB, n - kb);
+  if (s0 >= n || !tl_solving(in, w, m)) return;
+  const int tid = threadIdx.x;
+  const int s1 = min(s0 + kTV, n), nblk = (s1 - s0 + kTB - 1) / kTB;
   const double* A = tf_matrix(w, m);
   double* v = w.vec + m * (N + 1);
-  if (tid < nb) {
-    double sacc = 0.0;
-    for (int k = tid; k < nb; ++k) sacc = fma(A[(size_t)(kb + k) * N + kb + tid], v[kb + k], sacc);
-    xs[tid] = sacc;
+  s_v[tid] = s0 + tid < s1 ? v[s0 + tid] : 0.0;
+  double next[kTQ];  // the tile of the next block, transposed as it is stored
+  auto fetch = [&](int b) {
+    const int kb = s0 + kTB * b;
+#pragma unroll
+    for (int u = 0; u < kTQ; ++u) {
+      const int e = tid + kTV * u, c = e >> 6, r = e & (kTB - 1);
+      next[u] = c < r && kb + r < n ? A[(size_t)(kb + c) * N + kb + r] : 0.0;
+    }
+  };
+  fetch(BACK ? nblk - 1 : 0);
+  for (int q = 0; q < nblk; ++q) {
+    const int b = BACK ? nblk - 1 - q : q;
+    const int kb = s0 + kTB * b, nb = min(kTB, s1 - kb);
+#pragma unroll
+    for (int u = 0; u < kTQ; ++u) {
+      const int e = tid + kTV * u;
+      s_t[(e >> 6) * kTS + (e & (kTB - 1))] = next[u];
+    }
+    __syncthreads();
+    if (tid < kTB) {
+      const double x = tl_tile_solve<BACK>(s_t, s_v[kTB * b + tid]);
+      s_x[tid] = x;
+      s_v[kTB * b + tid] = x;
+    }
+    __syncthreads();
+    if (q + 1 < nblk) {
+      fetch(BACK ? b - 1 : b + 1);  // in flight during the update
+      if (BACK) {
+        // entries before the block, a thread each
+        if (tid < kTB * b) {
+          const double* p = A + (size_t)kb * N + s0 + tid;
+          double acc = 0.0;
+#pragma unroll 1
+          for (int c = 0; c < nb; c += 8) {  // (s_x is zero past the last atom)
+            double l[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) l[u] = p[min(c + u, nb - 1) * (int)N];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc = fma(l[u], s_x[c + u], acc);
+          }
+          s_v[tid] -= acc;
+        }
+      } else {
+        // entries behind the block, a thread each
+        if (tid >= kTB * (b + 1) && s0 + tid < s1) {
+          const double* p = A + (size_t)(s0 + tid) * N + kb;
+          double acc = 0.0;
+#pragma unroll 1
+          for (int c = 0; c < kTB; c += 8) {
+            double l[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) l[u] = p[c + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc = fma(l[u], s_x[c + u], acc);
+          }
+          s_v[tid] -= acc;
+        }
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  if (y == 0 && tid < nb) {
-    const int64_t* Z = in.numbers + m * N;
-    dst_base[m * N + kb + tid] = Z[kb + tid] != 0 ? xs[tid] : 0.0;
-  }
-  if (j < kb) {
-    double sacc = 0.0;
-    for (int c = 0; c < nb; ++c) sacc = fma(A[(size_t)(kb + c) * N + j], xs[c], sacc);
-    v[j] -= sacc;
+  const int64_t* Z = in.numbers + m * N;
+  if (s0 + tid < s1) {
+    const double x = s_v[tid];
+    v[s0 + tid] = x;
+    dst[m * N + s0 + tid] = BACK && Z[s0 + tid] == 0 ? 0.0 : x;
   }
 }
 
-// One forward-substitution step L y = v at block kb (ascending kb): y_kb =
-// X v_kb is stored to dst by work-group 0; work-group y updates the rows
-// kb + nb + 256 y .. below the block.
-__global__ __launch_bounds__(256) void k_tf_fsolve(Inputs in, Work w, int kb,
-                                                   double* dst_base) {
+// The share of the solved entries s0 .. s0 + kTV - 1 in the entries before them
+// (BACK: 64 per work-group) or behind them (16 per work-group).
+template <bool BACK>
+__global__ __launch_bounds__(kTV) void k_tl_gemv(Inputs in, Work w, int s0) {
   tf_priority();
-  __shared__ double ys[kTB];
+  __shared__ double s_x[kTV];
+  __shared__ double s_p[4][kTB];
   const int64_t m = blockIdx.x;
-  const int y = (int)blockIdx.y;
-  const int tid = threadIdx.x;
   const int64_t N = w.N;
   const int n = w.natom[m];
-  if (in.q_in != nullptr || kb >= n || (w.status[m] & (kStatusLU | kStatusSingular))) return;
-  const int nb = min(kTB, n - kb);
-  const int j = kb + nb + y * 256 + tid;
-  if (y > 0 && kb + nb + y * 256 >= n) return;
+  if (s0 >= n || !tl_solving(in, w, m)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int s1 = min(s0 + kTV, n), len = s1 - s0;
   const double* A = tf_matrix(w, m);
   double* v = w.vec + m * (N + 1);
-  if (tid < nb) {
-    const double* Xr = A + (size_t)(kb + tid) * N + kb;
-    double sacc = 0.0;
-    for (int k = 0; k <= tid; ++k) sacc = fma(Xr[k], v[kb + k], sacc);
-    ys[tid] = sacc;
-  }
+  if (!BACK && s1 + 16 * (int)blockIdx.y >= n) return;
+  s_x[tid] = tid < len ? v[s0 + tid] : 0.0;
   __syncthreads();
-  if (y == 0 && tid < nb) dst_base[m * N + kb + tid] = ys[tid];
-  if (j < n) {
-    const double* Aj = A + (size_t)j * N + kb;
-    double sacc = 0.0;
-    for (int c = 0; c < nb; ++c) sacc = fma(Aj[c], ys[c], sacc);
-    v[j] -= sacc;
+  if (BACK) {
+    const int j = kTB * (int)blockIdx.y + lane;  // < s0
+    const double* p = A + (size_t)s0 * N + j;
+    double acc = 0.0;
+    for (int c = wave; c < len; c += 32) {  // every fourth row, eight in flight
+      double l[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) l[u] = p[(size_t)min(c + 4 * u, len - 1) * N];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc = fma(l[u], c + 4 * u < len ? s_x[c + 4 * u] : 0.0, acc);
+    }
+    s_p[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0) v[j] -= (s_p[0][lane] + s_p[1][lane]) + (s_p[2][lane] + s_p[3][lane]);
+  } else {
+    // (len = kTV: there are entries behind)
+    for (int k = 0; k < 4; ++k) {
+      const int i = s1 + 16 * (int)blockIdx.y + 4 * k + wave;
+      if (i >= n) break;  // uniform over the wave
+      const double* p = A + (size_t)i * N + s0 + lane;
+      double l[kTV / 64], acc = 0.0;
+#pragma unroll
+      for (int u = 0; u < kTV / 64; ++u) l[u] = p[64 * u];
+#pragma unroll
+      for (int u = 0; u < kTV / 64; ++u) acc = fma(l[u], s_x[64 * u + lane], acc);
+      acc = wave_sum(acc);
+      if (lane == 0) v[i] -= acc;
+    }
   }
 }
 
@@ -1423,34 +1461,35 @@ __global__ __launch_bounds__(256) void k_tf_adj_init(Inputs in, Work w) {
   const int64_t m = blockIdx.x;
   const int64_t N = w.N;
   const int n = w.natom[m];
-  if (in.q_in != nullptr || (w.status[m] & (kStatusLU | kStatusSingular))) return;
+  if (!tl_solving(in, w, m)) return;
   const int64_t* Z = in.numbers + m * N;
   double* v = w.vec + m * (N + 1);
   for (int i = threadIdx.x; i < n; i += 256) v[i] = Z[i] != 0 ? w.dldq[m * N + i] : 0.0;
 }
 
-// Between the two adjoint substitutions: w' = L^-1 g is in lam; v = w' - nu y_e
-// with nu = y_e . w' / y_e . y_e.
+// Between the two adjoint substitutions: w' = L^-1 g is in lam; v = D^-1 w' -
+// nu z_e with z_e = D^-1 L^-1 e and nu = z_e . w' / z_e . D z_e.
 __global__ __launch_bounds__(256) void k_tf_adj_mid(Inputs in, Work w) {
   tf_priority();
   __shared__ double red[2 * kWaves];
   const int64_t m = blockIdx.x;
   const int64_t N = w.N;
   const int n = w.natom[m];
-  if (in.q_in != nullptr || n == 0 || (w.status[m] & (kStatusLU | kStatusSingular))) return;
+  if (n == 0 || !tl_solving(in, w, m)) return;
   const int tid = threadIdx.x;
   const double* wl = w.lam + m * N;
-  const double* ye = w.ez + m * N;
+  const double* ze = w.ez + m * N;
+  const double* dpiv = w.dpiv + m * N;
   double sw = 0.0, sz = 0.0;
   for (int i = tid; i < n; i += 256) {
-    sw = fma(ye[i], wl[i], sw);
-    sz = fma(ye[i], ye[i], sz);
+    sw = fma(ze[i], wl[i], sw);
+    sz = fma(ze[i] * dpiv[i], ze[i], sz);
   }
   sw = block_sum(sw, red);
   sz = block_sum(sz, red + kWaves);
   const double nu = sw / sz;
   double* v = w.vec + m * (N + 1);
-  for (int i = tid; i < n; i += 256) v[i] = fma(-nu, ye[i], wl[i]);
+  for (int i = tid; i < n; i += 256) v[i] = fma(-nu, ze[i], wl[i] * rcp_nt(dpiv[i]));
 }
 
 // --------------------------------------------------------------------------
@@ -1619,31 +1658,36 @@ inline bool eeq_tiled(const Params& p, int64_t N) {
   return p.force_tiled || N > kEeqMaxN;
 }
 
+// Substitution over all entries of the tiled factor, kTV at a time.
+template <bool BACK>
+void launch_tl_substitution(hipStream_t s, const Inputs& in, const Work& w, double* dst) {
+  const int N = (int)w.N, blocks = (N + kTV - 1) / kTV;
+  const unsigned B = (unsigned)w.B;
+  for (int k = 0; k < blocks; ++k) {
+    const int s0 = kTV * (BACK ? blocks - 1 - k : k);
+    hipLaunchKernelGGL(k_tl_solve<BACK>, dim3(B), dim3(kTV), kTlSolveLds, s, in, w, s0, dst);
+    if (k + 1 == blocks) break;
+    const unsigned tiles = (unsigned)(BACK ? s0 / kTB : (N - s0 - kTV + 15) / 16);
+    hipLaunchKernelGGL(k_tl_gemv<BACK>, dim3(B, tiles), dim3(kTV), 0, s, in, w, s0);
+  }
+}
+
 hipError_t launch_eeq_tiled(hipStream_t s, const DevTables& t, const Params& p,
                             const Inputs& in, const Work& w) {
   const int N = (int)w.N;
   const unsigned B = (unsigned)w.B;
   const unsigned rows = (unsigned)((w.B * (w.N + 2) + kWaves - 1) / kWaves);
   hipLaunchKernelGGL(k_tf_assemble, dim3(rows), dim3(256), 0, s, t, p, in, w);
-  hipError_t e = ensure_lds((const void*)k_tf_diag, kTfDiagLds);
-  if (e == hipSuccess) e = ensure_lds((const void*)k_tf_panel, kTfTileLds);
-  if (e == hipSuccess) e = ensure_lds((const void*)k_tf_update, kTfTileLds);
+  hipError_t e = ensure_lds((const void*)k_tl_step, kTlLds);
   if (e != hipSuccess) return e;
   for (int kb = 0; kb < N; kb += kTB) {
-    hipLaunchKernelGGL(k_tf_diag, dim3(B), dim3(256), kTfDiagLds, s, in, w, kb);
-    const unsigned ptiles = (unsigned)((N - kb + 1 + kTB - 1) / kTB);
-    hipLaunchKernelGGL(k_tf_panel, dim3(B, ptiles), dim3(256), kTfTileLds, s, in, w, kb);
-    if (kb + kTB < N) {
-      const int nI = (N + 2 - kb - kTB + kTB - 1) / kTB;
-      hipLaunchKernelGGL(k_tf_update, dim3(B, (unsigned)(nI * (nI + 1) / 2)), dim3(256),
-                         kTfTileLds, s, in, w, kb);
-    }
+    const int npanel = (N + 2 - kb + kTB - 1) / kTB;
+    const int nI = kb > 0 ? npanel - 1 : 0;  // row tiles behind the panel
+    hipLaunchKernelGGL(k_tl_step, dim3(B, (unsigned)(npanel + nI * (nI + 1) / 2)), dim3(256),
+                       kTlLds, s, in, w, kb, npanel);
   }
   hipLaunchKernelGGL(k_tf_reduce, dim3(B), dim3(256), 0, s, in, w);
-  for (int kb = ((N - 1) / kTB) * kTB; kb >= 0; kb -= kTB) {
-    const unsigned chunks = (unsigned)max(1, (kb + 255) / 256);
-    hipLaunchKernelGGL(k_tf_bsolve, dim3(B, chunks), dim3(256), 0, s, in, w, kb, w.q);
-  }
+  launch_tl_substitution<true>(s, in, w, w.q);
   return hipGetLastError();
 }
 
@@ -1700,17 +1744,10 @@ hipError_t launch_adjoint(hipStream_t s, const DevTables& t, const Params& p,
   const unsigned grid = (unsigned)w.B;
   const int ordered = eeq_ordered(w) ? 1 : 0;
   if (eeq_tiled(p, w.N)) {
-    const int N = (int)w.N;
     hipLaunchKernelGGL(k_tf_adj_init, dim3(grid), dim3(256), 0, s, in, w);
-    for (int kb = 0; kb < N; kb += kTB) {
-      const unsigned chunks = (unsigned)max(1, (N - kb + 255) / 256);
-      hipLaunchKernelGGL(k_tf_fsolve, dim3(grid, chunks), dim3(256), 0, s, in, w, kb, w.lam);
-    }
+    launch_tl_substitution<false>(s, in, w, w.lam);
     hipLaunchKernelGGL(k_tf_adj_mid, dim3(grid), dim3(256), 0, s, in, w);
-    for (int kb = ((N - 1) / kTB) * kTB; kb >= 0; kb -= kTB) {
-      const unsigned chunks = (unsigned)max(1, (kb + 255) / 256);
-      hipLaunchKernelGGL(k_tf_bsolve, dim3(grid, chunks), dim3(256), 0, s, in, w, kb, w.lam);
-    }
+    launch_tl_substitution<true>(s, in, w, w.lam);
     hipLaunchKernelGGL((k_adjoint<true, 2>), dim3(grid), dim3(256), 0, s, t, p, in, w, ordered);
     return hipGetLastError();
   }

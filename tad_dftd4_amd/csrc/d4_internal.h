@@ -94,7 +94,8 @@ struct Work {
   double* dgw0;     // [B*N*8] d gw0 / d CN (D4S: unused)
   double* dgwq;     // [B*N*8] d gw / d q (D4S: dzeta/dq)
   double* chol;     // [B*NT] packed L D L^T of the Coulomb block (L strictly lower, D diagonal)
-  double* ez;       // [B*N] D^-1 L^-1 e (e = 1 on real atoms; tiled EEQ: L^-1 e)
+  double* ez;       // [B*N] D^-1 L^-1 e (e = 1 on real atoms)
+  double* dpiv;     // [B*N] pivots D of the tiled EEQ factor
   double* lu;       // [B*(N+1)^2] pivoted LU of the bordered matrix (fallback)
   int32_t* piv;     // [B*(N+1)]
   double* vec;      // [B*(N+1)] right-hand side / solution of the LU path
@@ -281,6 +282,7 @@ inline size_t layout(int64_t B, int64_t N, char* base, Work* w) {
   v.dgwq = (double*)take(8 * bn * kRefStride);
   v.chol = (double*)take(8 * size_t(B) * nt);
   v.ez = (double*)take(8 * bn);
+  v.dpiv = (double*)take(8 * bn);
   v.lu = (double*)take(8 * size_t(B) * n1 * n1);
   v.piv = (int32_t*)take(sizeof(int32_t) * size_t(B) * n1);
   v.vec = (double*)take(8 * size_t(B) * n1);

@@ -63,3 +63,27 @@ def test_batches_in_and_out_of_order():
                                             positions[part].contiguous(),
                                             charge[part].contiguous(), kp)
         assert torch.equal(e[part], ep) and torch.equal(g[part], gp)
+
+
+TILED = (1, 15, 16, 62, 63, 64, 65, 80, 126, 127, 128, 129, 255, 256, 257, 320, 511, 513)
+
+
+@pytest.mark.parametrize("n", TILED)
+def test_tiled_charges_and_adjoint(n):
+    # edges of the 64-column blocks (the border rows fall into the last diagonal
+    # tile for 64 k + 1 .. 64 k + 62 atoms, across it for 63, behind it for 64)
+    # and of the 256-entry substitutions; same bounds as above, n = 513
+    print(f"[case] tiled EEQ n = {n}", flush=True)
+    for pad in {n, n + 3}:
+        numbers, positions, charge = _batch(n, pad)
+        ref = dense.eeq_charges(numbers, positions, charge)
+        dev = [t.cuda() for t in (numbers, positions, charge)]
+        kp = runtime.KernelParams(force_tiled=True)
+        q = runtime.properties(*dev, kp)[1].cpu()
+        assert (q - ref).abs().max().item() < 1e-10
+        e, g, ws = runtime.energy_gradient(*dev, kp)
+        assert not runtime.molecule_status(ws, len(numbers)).any()
+        e_lu, g_lu, _ = runtime.energy_gradient(
+            *dev, runtime.KernelParams(force_tiled=True, force_lu=True))
+        assert (e - e_lu).abs().max().item() < 1e-13
+        assert (g - g_lu).abs().max().item() < 1e-11
