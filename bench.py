@@ -390,7 +390,7 @@ def main() -> int:
     kp.one_stream = args.one_stream
     rows, tile = kp.shapes(N, forces)
     rows = rows or (16 if N <= 160 else 32 if N <= 384 else 64)
-    tile = tile or (8 if forces else 16)
+    tile = tile or 8
     ws = runtime.new_workspace(B, N, dev)
     energy = torch.empty((B, N), dtype=torch.float64, device=dev)
     grad = torch.empty((B, N, 3), dtype=torch.float64, device=dev)

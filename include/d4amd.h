@@ -48,8 +48,8 @@ extern "C" {
 #define D4_FLAG_FORCE_PAIR_TILES 16 /* testing: the large-system three-body kernel at any size */
 #define D4_FLAG_D4S 32     /* D4S model: Gaussian weights with pairwise factors
                               (reference src/tad_dftd4/model/d4s.py:56-285) */
-#define D4_FLAG_ATM16 64   /* gradient calls: one-pass three-body kernel with 16 x 16 pair
-                              tiles (default 8 x 8; energy-only calls use 16 x 16) */
+#define D4_FLAG_ATM16 64   /* one-pass three-body kernel with 16 x 16 pair tiles (default
+                              8 x 8) */
 #define D4_FLAG_PAIR_OWNER 128 /* testing: large systems take the pair-owner three-body
                                   kernel (each triple from its three pairs) */
 /* Launch shapes (results agree to rounding; used by the shape tuner,
@@ -59,9 +59,8 @@ extern "C" {
 #define D4_FLAG_ROWS_32 512
 #define D4_FLAG_ROWS_64 768
 #define D4_FLAG_ROWS_MASK 768
-#define D4_FLAG_ATM8 1024  /* energy-only calls: one-pass three-body kernel with 8 x 8
-                              pair tiles (default 16 x 16; gradient calls use 8 x 8
-                              unless D4_FLAG_ATM16) */
+#define D4_FLAG_ATM8 1024  /* one-pass three-body kernel with 8 x 8 pair tiles (the
+                              default) */
 #define D4_FLAG_ONE_STREAM 2048 /* testing/profiling: run the three-body side on the
                                    caller's stream too (no companion stream), so a
                                    kernel trace shows each kernel's own time */

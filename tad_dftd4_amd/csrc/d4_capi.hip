@@ -111,7 +111,6 @@ d4::Params to_params(const d4_params* p) {
   k.pair_owner = (p->flags & D4_FLAG_PAIR_OWNER) ? 1 : 0;
   const unsigned rows = ((unsigned)p->flags & D4_FLAG_ROWS_MASK) >> 8;
   k.row_lanes = rows == 0 ? 0 : 8 << rows;  // 1, 2, 3 -> 16, 32, 64
-  k.atm8 = (p->flags & D4_FLAG_ATM8) ? 1 : 0;
   k.one_stream = (p->flags & D4_FLAG_ONE_STREAM) ? 1 : 0;
   return k;
 }

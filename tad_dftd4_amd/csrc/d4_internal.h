@@ -68,10 +68,9 @@ struct Params {
   int force_pairtiles;
   int pgrad;  // accumulate parameter gradients (backward only)
   int d4s;    // D4S model: Gaussian weights with pairwise factors
-  int atm16;  // one-pass three-body kernel with 16 x 16 pair tiles (testing)
+  int atm16;  // one-pass three-body kernel with 16 x 16 pair tiles
   int pair_owner;  // large systems: pair-owner three-body kernel (testing)
   int row_lanes;   // lanes per atom row of the row passes (16, 32, 64; 0: by length)
-  int atm8;        // energy-only calls: one-pass three-body kernel with 8 x 8 tiles
   int one_stream;  // no companion stream (testing, profiling)
 };
 
@@ -144,18 +143,23 @@ constexpr int kAtm1Acc = 5;  // energy share, gradient (3), dL/dCN
 __host__ __device__ inline int atm1_splits(int n);
 // The 8 x 8 variant (one wave per work-group, kAtm8-atom blocks; the
 // gradient passes) splits a molecule over atm8_splits(n) waves, also a
-// function of n alone: about one 40-atom molecule of work (n^3 = 65536) each,
-// at most 64 (each split writes a partial sum per atom). On a 1024 x 20-120
-// batch, 32768 per split gave the same kernel time alone but a 2.5 % slower
-// two-stream step (twice the waves and partial sums); 49152 and 81920 or
-// more were slower.
+// function of n alone: up to 16 splits of about one 25-atom molecule of work
+// (n^3 = 16384) each, more only at 65536 each, at most 64 (each split writes a
+// partial sum per atom). The fine splits of molecules up to about 100 atoms end
+// the kernel sooner where a batch does not fill the chip (energies + forces of
+// one 64-atom molecule 113 -> 86 us, 96 x 10-80 atoms 167 -> 136, 384 x 6-60
+// 206 -> 137); past 16 the partial sums cost more: 1024 x 20-120 atoms 854 us
+// with 65536 per split throughout and with at most 8, 12 or 16 fine splits, 912
+// with 16384 per split throughout.
 constexpr int kAtm8 = 8;
 constexpr int kAtm8MaxSplits = 64;
 __host__ __device__ inline int atm8_splits(int n) {
   const int nb = (n + kAtm8 - 1) / kAtm8;
   const int tiles = nb * (nb + 1) / 2;
   const long long work = (long long)n * n * n;
+  const int fine = (int)((work + 16383) / 16384);
   int s = (int)((work + 65535) / 65536);
+  s = s > 16 ? s : (fine < 16 ? fine : 16);
   s = s > kAtm8MaxSplits ? kAtm8MaxSplits : s;
   return tiles < 1 ? 1 : (s < 1 ? 1 : (s > tiles ? tiles : s));
 }
@@ -241,11 +245,11 @@ __host__ __device__ inline int one_pass_splits(int n, bool tile8) {
   return tile8 ? atm8_splits(n) : atm1_splits(n);
 }
 
-// The gradient passes use the 8 x 8 one-pass kernel, energies alone the
-// 16 x 16 one (fewer, larger work-groups suit the lighter energy slots).
-inline bool one_pass_tile8(const Params& p, bool grad) {
-  return grad ? !p.atm16 : p.atm8 != 0;
-}
+// The one-pass kernel is the 8 x 8 one unless the caller asks for 16 x 16
+// (energy steps, us, 16 x 16 against 8 x 8: one 64-atom molecule 104 / 62, 384
+// x 6-60 atoms 160 / 102, 1024 x 20-120 693 / 586, 256 x 8-160 372 / 345, 256 x
+// 8-200 531 / 527).
+inline bool one_pass_tile8(const Params& p) { return !p.atm16; }
 
 inline size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 

@@ -2848,7 +2848,7 @@ hipError_t launch_atm8(hipStream_t s, const Params& p, const Inputs& in, const W
 
 hipError_t launch_atm1(hipStream_t s, const Params& p, const Inputs& in, const Work& w,
                        bool energy, bool grad) {
-  if (one_pass_tile8(p, grad)) return launch_atm8(s, p, in, w, energy, grad);
+  if (one_pass_tile8(p)) return launch_atm8(s, p, in, w, energy, grad);
   const int S = atm1_splits((int)w.N);
   const int64_t nblocks = w.B * S;
   const int64_t grid = (nblocks + 7) / 8 * 8;  // multiple of 8 for the XCD remap
@@ -2919,7 +2919,7 @@ hipError_t launch_atm_rows(hipStream_t s, const Params& p, const Inputs& in, con
                            double* grad_out) {
   if (one_pass(p, w)) {
     const unsigned grid = (unsigned)((w.B * w.N * 8 + 255) / 256);
-    const int tile8 = one_pass_tile8(p, grad) ? 1 : 0;
+    const int tile8 = one_pass_tile8(p) ? 1 : 0;
     if (energy && grad)
       hipLaunchKernelGGL((k_atm1_rows<true, true>), dim3(grid), dim3(256), 0, s, in, w, tile8,
                          energy_out, grad_out);
@@ -2981,7 +2981,7 @@ hipError_t launch_properties(hipStream_t s, const DevTables& t, const Inputs& in
 hipError_t launch_pgrad_reduce(hipStream_t s, const Params& p, const Inputs& in,
                                const Work& w, double* out) {
   const bool op = one_pass(p, w);
-  const bool tile8 = one_pass_tile8(p, true);
+  const bool tile8 = one_pass_tile8(p);
   const int64_t nb = n_groups(w.N);
   const int mode = op ? 1 : (p.pair_owner ? 0 : 2);
   const int64_t per_mol = mode == 1   ? one_pass_splits((int)w.N, tile8)

@@ -110,8 +110,8 @@ class KernelParams:
     pair_owner: bool = False  # testing: large systems take the pair-owner three-body kernel
     # launch shapes (results agree to rounding): lanes per atom row of the CN,
     # pair and chain passes (16, 32, 64; 0: by padded length) and the pair tile
-    # of the one-pass three-body kernel (8, 16; 0: 16 for energies, 8 with
-    # gradients). With both at 0 an activated shape table decides.
+    # of the one-pass three-body kernel (8, 16; 0: 8). With both at 0 an
+    # activated shape table decides.
     row_lanes: int = 0
     atm_tile: int = 0
     one_stream: bool = False  # profiling: no companion stream for the three-body side
