@@ -117,7 +117,7 @@ struct Work {
   double* gsph;     // [B*NG*4] bounding sphere (centre, radius) of each 16-atom group
   double* gsph8;    // [B*NG8*4] bounding sphere of each 8-atom group
   int64_t* wix;     // [B*(2*NG8+3)] slot tables of the screened one-pass kernel
-  double* apart;    // [B*S*5*N] per-split atom sums of the one-pass three-body kernel
+  double* apart;    // [B*S*5*N] per-split atom sums of the one-pass three-body kernel (in pg)
   double* rt4;      // [B*N] sqrt(r4r2) per atom (parameter gradients)
   int32_t* zslot;   // [B*kMaxZ] element -> slot in the molecule's element list (-1: none)
   int32_t* nzs;     // [B] distinct elements of the molecule, -1 if more than kZSlots
@@ -141,27 +141,26 @@ __host__ __device__ inline int64_t n_groups(int64_t N) { return (N + kGroup - 1)
 constexpr int kAtm1MaxN = 256;
 constexpr int kAtm1Acc = 5;  // energy share, gradient (3), dL/dCN
 __host__ __device__ inline int atm1_splits(int n);
-// The 8 x 8 variant (one wave per work-group, kAtm8-atom blocks; the
-// gradient passes) splits a molecule over atm8_splits(n) waves, also a
-// function of n alone: up to 16 splits of about one 25-atom molecule of work
-// (n^3 = 16384) each, more only at 65536 each, at most 64 (each split writes a
-// partial sum per atom). The fine splits of molecules up to about 100 atoms end
-// the kernel sooner where a batch does not fill the chip (energies + forces of
-// one 64-atom molecule 113 -> 86 us, 96 x 10-80 atoms 167 -> 136, 384 x 6-60
-// 206 -> 137); past 16 the partial sums cost more: 1024 x 20-120 atoms 854 us
-// with 65536 per split throughout and with at most 8, 12 or 16 fine splits, 912
-// with 16384 per split throughout.
+// The 8 x 8 variant (one wave per work-group, kAtm8-atom blocks) walks a list
+// of chunks (tile, 8 third atoms), each tile preceded by kAtm8TileCost places
+// for its own loads and sums; the atm8_splits(n) waves of a molecule, also a
+// function of n alone, take equal parts of that list. n^2 / 250 parts keep the
+// partial sums (5 n doubles each) a fixed small share of the n^3 / 6 triples:
+// 12 to 16 chunks per part up to 160 atoms, more above, where 3 n / 5 parts is
+// what the buffer holds. Steps in us with n^2 / 160, / 250, / 400: 256 x 8-200
+// energies 466 / 458 / 467, 1024 x 20-120 forces 931 / 886 / 897, 256 x 20-120
+// D4S 480 / 471 / 485; whole tiles dealt to at most 64 parts: 589 / 894 / 509.
 constexpr int kAtm8 = 8;
-constexpr int kAtm8MaxSplits = 64;
+constexpr int kAtm8TileCost = 2;
+__host__ __device__ inline int atm8_chunks(int nb) {
+  const int M = nb - 1, nw = (nb + 1) / 2;
+  const int pairs = M > 1 ? (M - 1) * M / 2 : 0;
+  return nw * (nb + kAtm8TileCost) + (M > 1 ? (M - 1) * M * (M + 1) / 6 : 0) +
+         pairs * kAtm8TileCost;
+}
 __host__ __device__ inline int atm8_splits(int n) {
-  const int nb = (n + kAtm8 - 1) / kAtm8;
-  const int tiles = nb * (nb + 1) / 2;
-  const long long work = (long long)n * n * n;
-  const int fine = (int)((work + 16383) / 16384);
-  int s = (int)((work + 65535) / 65536);
-  s = s > 16 ? s : (fine < 16 ? fine : 16);
-  s = s > kAtm8MaxSplits ? kAtm8MaxSplits : s;
-  return tiles < 1 ? 1 : (s < 1 ? 1 : (s > tiles ? tiles : s));
+  const int s = (n * n + 249) / 250, cap = 3 * n / 5;
+  return cap < 1 ? 1 : (s > cap ? cap : s);
 }
 
 // Screened one-pass three-body kernel (large systems, atoms in spatial
@@ -312,10 +311,10 @@ inline size_t layout(int64_t B, int64_t N, char* base, Work* w) {
   v.gsph = (double*)take(32 * size_t(B) * size_t(n_groups(N)));
   v.gsph8 = (double*)take(32 * size_t(B) * size_t(n_groups8(N)));
   v.wix = (int64_t*)take(8 * size_t(B) * size_t(atm8s_table_len(N)));
-  v.apart = (double*)take(N <= kAtm1MaxN
-                              ? 8 * size_t(B) * size_t(one_pass_split_max((int)N)) * kAtm1Acc *
-                                    size_t(N)
-                              : 0);
+  // (the pair tiles and the screened kernel, which use pg, ph and pe, do not
+  // run with the one-pass kernels; one_pass_split_max(N) * kAtm1Acc * N <=
+  // 3 N^2 or 48 doubles, at most the stride of pg)
+  v.apart = v.pg;
   v.rt4 = (double*)take(8 * bn);
   v.zslot = (int32_t*)take(4 * size_t(B) * kMaxZ);
   v.nzs = (int32_t*)take(4 * size_t(B));

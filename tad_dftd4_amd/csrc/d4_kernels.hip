@@ -1525,8 +1525,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D4_ATM1_WAV
 // tiles, on third atoms z <= y and past the end of the molecule.
 //
 // Every triple of the 8-atom blocks of molecule m is counted once, by one of
-// two kinds of tiles, and work-group (m, s) takes every S-th tile (S =
-// atm8_splits(n)):
+// two kinds of tiles, each a list of chunks of 8 third atoms; work-group (m, s)
+// takes an equal part of the molecule's chunks (atm8_splits(n) parts, a tile
+// may be shared by two of them):
 //  - W-tile t (the first ceil(nb / 2) tiles): the 28 pairs u < v inside
 //    block 2 t (lanes 0..27) and inside block 2 t + 1 (lanes 32..59) against
 //    the third atoms of every block; in the pair's own block only z > v
@@ -1546,6 +1547,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D4_ATM1_WAV
 // DPP moves; one more xor 7 after the last step (so the moves repeat every
 // four steps) leaves lane tx with its row's sums for z0 + tx.
 // Every sum is added in a fixed order (no atomics).
+// Bound by FP64 VALU issue: 1024 x 20-120 atoms, energies + forces, 67% of the
+// issue slots over the kernel, 74% while a CU is busy. With whole tiles dealt
+// to the splits and the splits of a molecule kept on one XCD the CUs were busy
+// 76% of the time (now 90%): 256 x 8-200 energies 363 -> 232 us alone (with the
+// 16-byte records), a 150-atom molecule 84 -> 45 us.
+// Energies hold 102 VGPRs and 4.6 KB: four waves per SIMD. Forces hold 210
+// VGPRs, two waves; held to 168 for three they spill (880 -> 1060 us per step).
 // --------------------------------------------------------------------------
 
 // Lane L of each 8-lane group receives the value of lane L ^ d (d = 1, 3, 7).
@@ -1580,10 +1588,30 @@ constexpr double kAtmFar = 1.0e6;  // position of lanes and third atoms without 
 // not overlap, so with zl = tx ^ k the address is a lane constant xor a step
 // constant (one v_xor per read, no multiply), and the (zl << 4) skew puts
 // the eight lanes of a row on distinct 16-byte bank groups.
-constexpr int kAtm8Row = 128;  // doubles per row
+// Energies alone read only (t, p) of a record: 16-byte records in rows of 512
+// bytes, c = 16 and 17 the third atom's (x, y) and (z, -), record c of row zl
+// at byte (zl << 9) | ((c ^ skew(zl)) << 4). The skew is multiplication by a
+// generator of GF(8): linear over xor like zl << 4 above, and both zl and
+// (zl ^ k) -> zl ^ skew(zl ^ k) are one-to-one, so the eight lanes of a row
+// again read distinct bank groups.
 constexpr int kAtm8RecZ = 16, kAtm8RecRt = 17;
+template <bool GRAD>
+constexpr int kAtm8Row = GRAD ? 128 : 64;  // doubles per row
+__device__ __forceinline__ uint32_t atm8_skew(uint32_t zl) {
+  return ((zl << 1) & 7u) ^ ((zl >> 2) * 3u);
+}
+// the row part and the column part of a record's address (xor of the two)
+template <bool GRAD>
+__device__ __forceinline__ uint32_t atm8_row(uint32_t zl) {
+  return GRAD ? (zl << 10) | (zl << 4) : (zl << 9) | (atm8_skew(zl) << 4);
+}
+template <bool GRAD>
+__device__ __forceinline__ uint32_t atm8_col(int c) {
+  return (uint32_t)c << (GRAD ? 5 : 4);
+}
+template <bool GRAD>
 __device__ __forceinline__ uint32_t atm8_rec(int zl, int c) {
-  return ((uint32_t)zl << 10) | (((uint32_t)c << 5) ^ ((uint32_t)zl << 4));
+  return atm8_row<GRAD>((uint32_t)zl) ^ atm8_col<GRAD>(c);
 }
 template <typename T>
 __device__ __forceinline__ const T* atm8_at(const double* s_zc, uint32_t off) {
@@ -1704,22 +1732,25 @@ __device__ __forceinline__ void atm8_fetch(Atm8Chunk& c, const Inputs& in, const
   }
 }
 
-template <bool PG>
+template <bool GRAD, bool PG>
 __device__ __forceinline__ void atm8_stage(const Atm8Chunk& c, double* s_zc, int lane) {
   char* base = reinterpret_cast<char*>(s_zc);
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int e = lane + 64 * r;
     const int zl = e >> 4, cl = e & 15;
-    double2* dst = reinterpret_cast<double2*>(base + atm8_rec(zl, cl));
+    double2* dst = reinterpret_cast<double2*>(base + atm8_rec<GRAD>(zl, cl));
     dst[0] = make_double2(c.t[r], c.p[r]);
-    dst[1] = make_double2(c.kz[r], c.kc[r]);
+    if (GRAD) dst[1] = make_double2(c.kz[r], c.kc[r]);
   }
   if (lane < kAtm8) {
-    double2* r = reinterpret_cast<double2*>(base + atm8_rec(lane, kAtm8RecZ));
+    double2* r = reinterpret_cast<double2*>(base + atm8_rec<GRAD>(lane, kAtm8RecZ));
     r[0] = make_double2(c.r[0], c.r[1]);
-    r[1] = make_double2(c.r[2], c.r[3]);
-    if (PG) *reinterpret_cast<double*>(base + atm8_rec(lane, kAtm8RecRt)) = c.r[4];
+    if (GRAD)
+      r[1] = make_double2(c.r[2], c.r[3]);
+    else
+      *reinterpret_cast<double*>(base + atm8_rec<GRAD>(lane, kAtm8RecZ + 1)) = c.r[2];
+    if (PG) *reinterpret_cast<double*>(base + atm8_rec<GRAD>(lane, kAtm8RecRt)) = c.r[4];
   }
 }
 
@@ -1734,12 +1765,12 @@ __device__ __forceinline__ void atm8_chunk(const Params& p, const Atm8Pair& q, A
                                            int z0, int y, int cx = -1, int cy = -1,
                                            bool own = true) {
   constexpr int T8 = kAtm8;
-  // lane parts of the record addresses (the step part is (k << 10) | (k << 4))
-  const uint32_t lrow = ((uint32_t)tx << 10) | ((uint32_t)tx << 4);
-  const uint32_t ox = lrow ^ ((uint32_t)(cx < 0 ? tx : cx) << 5);
-  const uint32_t oy = lrow ^ ((uint32_t)(cy < 0 ? T8 + ty : cy) << 5);
-  const uint32_t oz = lrow ^ ((uint32_t)kAtm8RecZ << 5);
-  const uint32_t ort = lrow ^ ((uint32_t)kAtm8RecRt << 5);
+  // lane parts of the record addresses (the step part is the row part of k)
+  const uint32_t lrow = atm8_row<GRAD>((uint32_t)tx);
+  const uint32_t ox = lrow ^ atm8_col<GRAD>(cx < 0 ? tx : cx);
+  const uint32_t oy = lrow ^ atm8_col<GRAD>(cy < 0 ? T8 + ty : cy);
+  const uint32_t oz = lrow ^ atm8_col<GRAD>(kAtm8RecZ);
+  const uint32_t ort = lrow ^ atm8_col<GRAD>(kAtm8RecRt);
   const double c3sq = p.cut3sq, alp = p.alp, a1p = p.a1, a2p = p.a2, sq3 = 1.7320508075688772;
   // alp T f = alp / 6 (1 - f), f = 1 / (1 + 6 T): H below needs no alp T
   const double alp6 = alp / 6.0, h0 = alp6 - 2.5;
@@ -1751,9 +1782,11 @@ __device__ __forceinline__ void atm8_chunk(const Params& p, const Atm8Pair& q, A
   constexpr int kUnroll = PG ? 2 : D4_ATM8_UNROLL;
   D4_UNROLL(kUnroll)
   for (int k = 0; k < T8; ++k) {
-    const uint32_t ks = ((uint32_t)k << 10) | ((uint32_t)k << 4);
+    const uint32_t ks = atm8_row<GRAD>((uint32_t)k);
     const double2* pz = atm8_at<double2>(s_zc, oz ^ ks);
-    const double2 rz01 = pz[0], rz23 = pz[1];
+    const double2 rz01 = pz[0];
+    const double2 rz23 =
+        GRAD ? pz[1] : make_double2(*atm8_at<double>(s_zc, ort ^ ks), 0.0);
     const double4 rz = make_double4(rz01.x, rz01.y, rz23.x, rz23.y);
     // records of x and y against z = z0 + (tx ^ k)
     const double2* px = atm8_at<double2>(s_zc, ox ^ ks);
@@ -1896,12 +1929,13 @@ __device__ __forceinline__ void atm8_fold_sca(const Atm8Pair& q, Atm8Sums& u) {
 // Stage five per-lane values (energy share, gradient at half weight, dL/dCN)
 // in s_red for the sums over rows or columns of the tile; gs scales the
 // gradient parts (6 where the chunks left out the constant weight 6, else 1).
-template <int NA>
+template <bool GRAD>
 __device__ __forceinline__ void atm8_stage_sums(double (*s_red)[64], int lane, double e,
                                                 double f0, double f1, double f2, double c,
                                                 double gs = 1.0) {
   const double g2 = 2.0 * gs;
   s_red[0][lane] = e;
+  if (!GRAD) return;
   s_red[1][lane] = g2 * f0;
   s_red[2][lane] = g2 * f1;
   s_red[3][lane] = g2 * f2;
@@ -1920,35 +1954,25 @@ __device__ __forceinline__ void atm8_store_pgrad(const Atm8Sums& u, int lane, do
 }
 
 template <bool ENERGY, bool GRAD, bool PG>
-#ifndef D4_ATM8_WAVES
-#define D4_ATM8_WAVES 2
-#endif
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D4_ATM8_WAVES))) void k_atm8(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_atm8(
     Params p, Inputs in, Work w, int S, int64_t nblocks) {
-  constexpr int NA = kAtm1Acc;
+  constexpr int NA = GRAD ? kAtm1Acc : 1;
   constexpr int T8 = kAtm8;
-  __shared__ __align__(16) double s_zc[T8 * kAtm8Row];
+  __shared__ __align__(16) double s_zc[T8 * kAtm8Row<GRAD>];
   __shared__ double s_red[NA][64];
-  __shared__ double s_red2[NA][64];
+  double (*s_red2)[64] = reinterpret_cast<double (*)[64]>(s_zc);  // between two tiles
+  static_assert(NA * 64 <= T8 * kAtm8Row<GRAD>, "s_red2");
   extern __shared__ double s_acc[];             // [NA][N] atom sums of this split
 
-  // block b runs on XCD b mod 8. Molecules go to the XCDs in runs of eight
-  // (molecules 8c .. 8c + 7 to XCD c mod 8), all splits of a molecule in
-  // consecutive blocks of its XCD: neighbouring molecules share an XCD's L2,
-  // and a batch sorted by size still spreads its large molecules over all
-  // XCDs (with whole eighths of the batch per XCD, a sorted 1024 x 20-120
-  // batch took 1.86 ms per step instead of 1.10)
-  const int64_t b = blockIdx.x, j = b >> 3, l = j / S;
-  const int64_t m = (((l >> 3) << 3) + (b & 7)) * 8 + (l & 7);
+  const int64_t b = blockIdx.x, m = b / S;
   if (m >= nblocks) return;  // nblocks: the number of molecules
-  const int s = (int)(j - l * S);
+  const int s = (int)(b - m * S);
   const int64_t N = w.N;
   const int n = w.natom[m];
   const int Sm = atm8_splits(n);  // this molecule's split count (S is the batch maximum)
   if (s >= Sm) return;
   const int nb = (n + T8 - 1) / T8;
   const int nw = (nb + 1) / 2;  // W-tiles, then the pair tiles bx < by <= nb - 2
-  const int tiles = nw + (nb > 1 ? (nb - 1) * (nb - 2) / 2 : 0);
   const int lane = threadIdx.x, tx = lane & (T8 - 1), ty = lane >> 3;
   const int64_t* Z = in.numbers + m * N;
   const double c3sq = p.cut3sq;
@@ -1970,7 +1994,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D4_ATM8_WAVE
   while (wok && (wv + 1) * wv / 2 <= wp) ++wv;
   const int wu = wok ? wp - wv * (wv - 1) / 2 : 0;
 
-  for (int t = s; t < tiles; t += Sm) {
+  // this split's share [pos, end) of the molecule's chunk list and the tile
+  // (and chunk of the tile) it starts in
+  const int V = atm8_chunks(nb);
+  int pos = (int)((int64_t)V * s / Sm);
+  const int end = (int)((int64_t)V * (s + 1) / Sm);
+  int t, pbx = 0, pby = 1, off;  // next tile, its blocks if a pair tile, chunks to skip
+  {
+    const int wlen = nb + kAtm8TileCost;
+    if (pos < nw * wlen) {
+      t = pos / wlen;
+      off = pos - t * wlen;
+    } else {
+      off = pos - nw * wlen;
+      int len = nb - 2 + kAtm8TileCost;  // of the tiles (., by)
+      t = nw;
+      while (off >= pby * len) {
+        off -= pby * len;
+        t += pby;
+        ++pby;
+        --len;
+      }
+      pbx = off / len;
+      off -= pbx * len;
+      t += pbx;
+    }
+  }
+  while (pos < end) {
     const bool wt = t < nw;
     int bx, by, x, y, cx, cy, z1;  // staged blocks, pair, its record columns, first chunk
     if (wt) {
@@ -1982,16 +2032,30 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D4_ATM8_WAVE
       cy = T8 * wh + wv;
       z1 = 0;
     } else {
-      const int t2 = t - nw;  // = by (by - 1) / 2 + bx
-      by = 1;
-      while ((by + 1) * by / 2 <= t2) ++by;
-      bx = t2 - by * (by - 1) / 2;
+      bx = pbx;
+      by = pby;
+      if (++pbx == pby) {
+        pbx = 0;
+        ++pby;
+      }
       x = bx * T8 + tx;
       y = by * T8 + ty;
       cx = tx;
       cy = T8 + ty;
       z1 = (by + 1) * T8;
     }
+    // the chunks [c0, c1) of the tile that fall in the share (the first
+    // kAtm8TileCost places of a tile stand for its own loads and sums)
+    const int len = (wt ? nb : nb - by - 1) + kAtm8TileCost;
+    const int upto = min(len, off + end - pos);
+    const int c0 = max(0, off - kAtm8TileCost), c1 = upto - kAtm8TileCost;
+    const int tw = t;
+    pos += upto - off;
+    off = 0;
+    ++t;
+    if (c0 >= c1) continue;
+    const int zend = min(n, z1 + c1 * T8);
+    z1 += c0 * T8;
     const bool valid = (wok || !wt) && x < y && y < n && Z[x] != 0 && Z[y] != 0;
     const Atm8Pair q = atm8_pair<GRAD, PG>(p, in, w, m, x, y, valid);
     u.ex = u.ey = u.cx = u.cy = u.sca = 0.0;
@@ -1999,17 +2063,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D4_ATM8_WAVE
 
     Atm8Chunk ch;
     atm8_fetch<GRAD, PG>(ch, in, w, m, n, z1, bx * T8, by * T8, lane);
-    for (int z0 = z1; z0 < n; z0 += T8) {
+    for (int z0 = z1; z0 < zend; z0 += T8) {
       __syncthreads();
-      atm8_stage<PG>(ch, s_zc, lane);
+      atm8_stage<GRAD, PG>(ch, s_zc, lane);
       __syncthreads();
-      if (z0 + T8 < n)  // in flight during this chunk
+      if (z0 + T8 < zend)  // in flight during this chunk
         atm8_fetch<GRAD, PG>(ch, in, w, m, n, z0 + T8, bx * T8, by * T8, lane);
 
       Atm8Ring rr = {0.0, 0.0, 0.0, 0.0, 0.0};
       // the two chunks of a W-tile's own blocks: third atoms up to y of the
       // lane's own block carry no weight
-      const bool first = wt && (z0 >> 4) == t;
+      const bool first = wt && (z0 >> 4) == tw;
       const bool own = z0 == T8 * (bx + wh);
       if (full) {
         if (first)
@@ -2029,7 +2093,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D4_ATM8_WAVE
       if (full) rr.E *= 2.0;
       // lane tx of every row now holds that row's sums for z0 + tx (the
       // gradient parts at half weight); add the 8 rows in order
-      atm8_stage_sums<NA>(s_red, lane, rr.E, rr.F0, rr.F1, rr.F2, rr.D, gs);
+      atm8_stage_sums<GRAD>(s_red, lane, rr.E, rr.F0, rr.F1, rr.F2, rr.D, gs);
       __syncthreads();
       if (lane < T8 * NA) {
         const int l = lane & (T8 - 1), c = lane >> 3;  // column l holds z0 + l
@@ -2048,14 +2112,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D4_ATM8_WAVE
     }
     atm8_fold_sca(q, u);
     __syncthreads();
-    atm8_stage_sums<NA>(s_red, lane, u.ex, u.fx0, u.fx1, u.fx2, u.cx, gs);
-    atm8_stage_sums<NA>(s_red2, lane, u.ey, u.fy0, u.fy1, u.fy2, u.cy, gs);
+    atm8_stage_sums<GRAD>(s_red, lane, u.ex, u.fx0, u.fx1, u.fx2, u.cx, gs);
+    atm8_stage_sums<GRAD>(s_red2, lane, u.ey, u.fy0, u.fy1, u.fy2, u.cy, gs);
     __syncthreads();
     if (wt) {
       // atom a of block 2 t + hh: x of the pairs (a, v > a), y of (u < a, a)
       for (int e = lane; e < 2 * T8 * NA; e += 64) {
         const int c = e >> 4, a16 = e & 15, hh = a16 >> 3, a = a16 & 7;
-        const int atom = 2 * T8 * t + a16;
+        const int atom = 2 * T8 * tw + a16;
         if ((c == 0 ? ENERGY : GRAD) && atom < n) {
           const double* sx = s_red[c] + 32 * hh;
           const double* sy = s_red2[c] + 32 * hh + a * (a - 1) / 2;
@@ -2190,7 +2254,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   constexpr int T8 = kAtm8;
   constexpr int KS = kAtm8sMaxSplits;
   constexpr int kWin = NA * T8;  // doubles per slot: [NA][8 atoms]
-  __shared__ __align__(16) double s_zc[T8 * kAtm8Row];
+  __shared__ __align__(16) double s_zc[T8 * kAtm8Row<GRAD>];
   __shared__ double s_red[NA][64];
 
   const int64_t b = blockIdx.x;
@@ -2275,7 +2339,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       if (gz < G) atm8_fetch<GRAD, PG>(ch, in, w, m, n, gz * T8, gx * T8, gy * T8, lane);
       while (gz < G) {
         __syncthreads();
-        atm8_stage<PG>(ch, s_zc, lane);
+        atm8_stage<GRAD, PG>(ch, s_zc, lane);
         __syncthreads();
         const int gzn = next_z();
         if (gzn < G)  // in flight during this chunk
@@ -2291,7 +2355,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         else
           atm8_chunk<ENERGY, GRAD, PG, false, false>(p, q, u, rr, s_zc, tx, ty,
                                                      gz * T8, y);
-        atm8_stage_sums<NA>(s_red, lane, rr.E, rr.F0, rr.F1, rr.F2, rr.D);
+        atm8_stage_sums<GRAD>(s_red, lane, rr.E, rr.F0, rr.F1, rr.F2, rr.D);
         __syncthreads();
         if (lane < kWin) {
           const int l = lane & (T8 - 1), c = lane >> 3;
@@ -2306,7 +2370,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       // the y atoms' tile sums (over the columns)
       atm8_fold_sca(q, u);
       __syncthreads();
-      atm8_stage_sums<NA>(s_red, lane, u.ey, u.fy0, u.fy1, u.fy2, u.cy);
+      atm8_stage_sums<GRAD>(s_red, lane, u.ey, u.fy0, u.fy1, u.fy2, u.cy);
       __syncthreads();
       if (lane < kWin) {
         const int row = lane & (T8 - 1), c = lane >> 3;
@@ -2321,7 +2385,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   }
   // the x atoms' sums over all tiles (over the rows)
   __syncthreads();
-  atm8_stage_sums<NA>(s_red, lane, u.ex, u.fx0, u.fx1, u.fx2, u.cx);
+  atm8_stage_sums<GRAD>(s_red, lane, u.ex, u.fx0, u.fx1, u.fx2, u.cx);
   __syncthreads();
   if (lane < kWin) {
     const int col = lane & (T8 - 1), c = lane >> 3;
@@ -2410,14 +2474,17 @@ __global__ __launch_bounds__(256) void k_atm1_rows(Inputs in, Work w, int tile8,
     return;
   }
   const int S = one_pass_splits(n, tile8 != 0);
-  const int64_t stride = (int64_t)one_pass_splits((int)N, tile8 != 0) * kAtm1Acc * N;
+  // the 8 x 8 kernel writes the energy alone where no gradient is asked for
+  const int64_t na = (GRAD || tile8 == 0) ? kAtm1Acc : 1;
+  const int64_t stride = (int64_t)one_pass_splits((int)N, tile8 != 0) * na * N;
   const double* part = w.apart + m * stride + i;
+  constexpr int c0 = ENERGY ? 0 : 1, c1 = GRAD ? kAtm1Acc : 1;
   double acc[kAtm1Acc] = {0.0, 0.0, 0.0, 0.0, 0.0};
   for (int s = l; s < S; s += 8)
 #pragma unroll
-    for (int c = 0; c < kAtm1Acc; ++c) acc[c] += part[(s * kAtm1Acc + c) * N];
+    for (int c = c0; c < c1; ++c) acc[c] += part[(s * na + c) * N];
 #pragma unroll
-  for (int c = 0; c < kAtm1Acc; ++c) acc[c] = sum_lanes8(acc[c]);
+  for (int c = c0; c < c1; ++c) acc[c] = sum_lanes8(acc[c]);
   if (l != 0) return;
   const double sixth = 1.0 / 6.0;
   if (ENERGY) energy_out[row] = w.e2[row] + acc[0] * sixth;
@@ -2828,11 +2895,10 @@ hipError_t launch_pairs(hipStream_t s, const DevTables& t, const Params& p,
 hipError_t launch_atm8(hipStream_t s, const Params& p, const Inputs& in, const Work& w,
                        bool energy, bool grad) {
   const int S = atm8_splits((int)w.N);
-  const int64_t nblocks = w.B;  // molecules; block b -> (m, s) as in k_atm8 (runs of 64
-                                // molecules per round of the eight XCDs)
-  const int64_t grid = (w.B + 63) / 64 * 64 * S;
+  const int64_t nblocks = w.B;  // molecules; block b -> (m, s) = (b / S, b mod S)
+  const int64_t grid = w.B * S;
   if (grid == 0) return hipSuccess;
-  const size_t shmem = sizeof(double) * kAtm1Acc * (size_t)w.N;
+  const size_t shmem = sizeof(double) * (grad ? kAtm1Acc : 1) * (size_t)w.N;
   const dim3 g((unsigned)grid), blk(64);
   if (energy && grad && in.gE != nullptr) return hipErrorInvalidValue;  // unit dL/dE only
   if (energy && grad)

@@ -1,0 +1,51 @@
+"""
+The 8 x 8 one-pass three-body kernel (equal parts of a molecule's chunk list)
+against the 16 x 16 one (whole tiles, another enumeration of the triples): at
+the edges of the 8-atom blocks, where the number of parts changes, with and
+without padding, for energies, gradients and both.
+
+The two sum the same triples in another order. An atom's three-body energy is
+a sum of at most 256^2 / 2 terms whose total stays below 1e-2 Eh, its gradient
+below 1e-1 Eh/bohr: with each term good to about 1e-14 of its size the sums
+agree far within 1e-13 and 1e-12.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from tad_dftd4_amd import runtime, synth
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (2, 3, 7, 8, 9, 15, 16, 17, 24, 25, 32, 33, 63, 64, 65, 121, 150, 199, 255, 256)
+
+
+@pytest.mark.parametrize("cutoff", [40.0, 12.0])
+@pytest.mark.parametrize("n", SIZES)
+def test_parts_of_the_chunk_list(n, cutoff):
+    print(f"[case] three-body n = {n}, cutoff {cutoff}", flush=True)
+    rng = np.random.default_rng(400 + n)
+    mols = [synth.molecule(rng, k, synth.MIX_HCNO, 2.8, (0,)) for k in (n, max(2, n - 5))]
+    kp = runtime.KernelParams(s8=1.2, a1=0.4, a2=5.0, cutoff_disp3=cutoff)
+    kp16 = runtime.KernelParams(s8=1.2, a1=0.4, a2=5.0, cutoff_disp3=cutoff, atm16=True)
+    ref = None
+    for pad in sorted({n, min(256, n + 7)}):
+        dev = [t.cuda() for t in synth.pack(mols, pad_to=pad)]
+        e, g, _ = runtime.energy_gradient(*dev, kp)
+        e16, g16, _ = runtime.energy_gradient(*dev, kp16)
+        assert (e - e16).abs().max().item() < 1e-13
+        assert (g - g16).abs().max().item() < 1e-12
+        # energies alone, and the gradient alone (weighted dL/dE)
+        ef, ws = runtime.forward(*dev, kp)
+        assert (ef - e16).abs().max().item() < 1e-13
+        w = torch.linspace(0.5, 1.5, pad, dtype=torch.float64, device="cuda").expand(2, pad)
+        gb = runtime.backward(*dev, kp, ws, w.contiguous())
+        ef16, ws16 = runtime.forward(*dev, kp16)
+        gb16 = runtime.backward(*dev, kp16, ws16, w.contiguous())
+        assert (gb - gb16).abs().max().item() < 1e-12
+        # the same bits whatever the padding (the row passes change at 160
+        # atoms, the charge solve at 140 and 201; from 256 on the atoms are sorted)
+        if ref is not None and not any(n <= edge < pad for edge in (140, 160, 201, 255)):
+            assert torch.equal(ref[0], e[:, :n]) and torch.equal(ref[1], g[:, :n])
+        ref = (e, g)
