@@ -164,29 +164,19 @@ __host__ __device__ inline int atm8_splits(int n) {
 }
 
 // Screened one-pass three-body kernel (large systems, atoms in spatial
-// order): 8-atom groups; x-group gx of a molecule with G groups is split over
-// atm8s_splits(G, gx, smax) work items, about smax ((G - gx) / G)^2 (the
-// work of gx falls with its forward neighbourhood), smax = atm8s_smax(n) at
-// most kAtm8sMaxSplits. Item (gx, s) has one window slot (5 x 8 doubles) for
-// each group g >= gx; the slots of a molecule fill at most atm8s_budget(n)
-// doubles (12 n^2 from kAtm1MaxN to 16384 atoms, else 3 n^2: the pair-matrix
-// space pg, ph, pe is allocated atm8s_stride(N) doubles per molecule), and
-// smax is the largest power of two that fits. All of it depends on the atom
-// count n alone.
+// order): 8-atom groups; the pair tiles and third-atom groups of x-group gx
+// form a chunk list that its work items share equally. Item i of x-group gx
+// has one window slot (5 x 8 doubles) for each group g >= gx. The number of
+// items follows from the lengths of the lists, so that the slots of a
+// molecule, behind its list tables, fill at most atm8s_budget(n) doubles (12
+// n^2 from kAtm1MaxN to 16384 atoms, else 3 n^2: the pair-matrix space pg, ph,
+// pe is allocated atm8s_stride(N) doubles per molecule) and its items at most
+// kAtm8sMaxSplits work-groups per group. All of it depends on the molecule
+// alone.
 constexpr int kAtm8sMaxSplits = 64;
 __host__ __device__ inline int64_t n_groups8(int64_t N) { return (N + kAtm8 - 1) / kAtm8; }
 // 64-bit words of one row of the group near bits
 __host__ __device__ inline int64_t near_words8(int64_t N) { return (n_groups8(N) + 63) / 64; }
-__host__ __device__ inline int atm8s_splits(int G, int gx, int smax) {
-  const long long r = G - gx, GG = (long long)G * G;
-  const long long s = (smax * r * r + GG - 1) / GG;
-  return s < 1 ? 1 : (s > smax ? smax : (int)s);
-}
-__host__ __device__ inline long long atm8s_slots(int G, int smax) {
-  long long t = 0;
-  for (int gx = 0; gx < G; ++gx) t += (long long)atm8s_splits(G, gx, smax) * (G - gx);
-  return t;
-}
 constexpr int64_t kAtm8sWideMax = 16384;
 __host__ __device__ inline int64_t atm8s_budget(int64_t n) {
   const int64_t a = (n > kAtm1MaxN && n <= kAtm8sWideMax ? 12 : 3) * n * n;
@@ -197,11 +187,14 @@ __host__ __device__ inline int64_t atm8s_stride(int64_t N) {
   const int64_t a = atm8s_budget(N), b = atm8s_budget(N < kAtm8sWideMax ? N : kAtm8sWideMax);
   return a > b ? a : b;
 }
-__host__ __device__ inline int atm8s_smax(int n) {
-  const int G = (n + kAtm8 - 1) / kAtm8;
-  for (int s = kAtm8sMaxSplits; s > 1; s >>= 1)
-    if (atm8s_slots(G, s) * kAtm1Acc * kAtm8 <= atm8s_budget(n)) return s;
-  return 1;
+// Doubles of the list tables (G rows of G + 1 32-bit entries) before the
+// windows, and the number of window slots that remain.
+__host__ __device__ inline int64_t atm8s_head(int64_t n) {
+  const int64_t G = n_groups8(n);
+  return (G * (G + 1) / 2 + 8) / 8 * 8;
+}
+__host__ __device__ inline int64_t atm8s_windows(int64_t n) {
+  return (atm8s_budget(n) - atm8s_head(n)) / (kAtm1Acc * kAtm8);
 }
 // Work-groups per molecule (x-groups padded to a multiple of 8, times the
 // largest split count) and the length of a molecule's slot table.

@@ -2155,48 +2155,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 
 // --------------------------------------------------------------------------
 // One-pass three-body kernel for large systems (the atoms in spatial order):
-// the 8 x 8 evaluation above with group screening. Work item (m, gx, s)
-// owns the x atoms of 8-atom group gx and takes every S-th of the pair tiles
-// (gx, gy), gy >= gx, whose groups can hold a counted triple (bounding
-// spheres within 2 c3); per tile it streams the third-atom groups gz >= gy
-// with at least two of the three group-to-group gaps within c3. Screened-out
-// triples contribute exact zeros, so the screening changes no bit of the
-// result beyond the order of the sums.
+// the 8 x 8 evaluation above with group screening. The x atoms of 8-atom
+// group gx against the pair tiles (gx, gy), gy >= gx, whose groups can hold a
+// counted triple (bounding spheres within 2 c3), and per tile the third-atom
+// groups gz >= gy with at least two of the three group-to-group gaps within
+// c3, form one list of chunks; the work items of gx take equal parts of it (a
+// tile may be shared by two). Screened-out triples contribute exact zeros.
 //
 // Outputs: each item adds its sums for the atoms of group g (x, y or z) to
 // its own slot of g in the window buffer: slots of group g are contiguous,
-// one per item (gx <= g, s), in item order, so k_atm8s_rows adds them in a
-// fixed order. The number of splits S of x-group gx depends on the
-// molecule's atom count alone (more for the first groups, whose forward
-// neighbourhood is largest), and heavy items are dispatched first.
+// one per item of the x-groups up to g, in item order, so k_atm8s_rows adds
+// them in a fixed order.
+//
+// Bound by FP64 VALU issue. The lists differ by more than ten between a corner
+// and the middle of a cluster: with every S-th tile to an item and S a function
+// of the group's number alone the last items ran by themselves for a fifth of
+// the kernel (27% of the wave slots empty) and one of 88 groups had a single
+// item of twice the mean. 5000-atom cluster, cutoff 25, energies + forces 51.2
+// -> 42.0 ms; 701 atoms, cutoff 40, energy, then forces 1250 -> 1073 us.
 // --------------------------------------------------------------------------
 
-// Slot tables of molecule m: [0] = largest split count, [1 + g] = first slot
-// of items of x-group g in the list of any later group (g = 0 .. GN), then
+// Slot tables of molecule m: [0] = number of work items, [1 + g] = first item
+// of x-group g (g = 0 .. GN; also the number of items of earlier groups), then
 // [GN + 2 + g] = first slot of group g in the window buffer (g = 0 .. GN).
 __device__ __forceinline__ const int64_t* atm8s_table(const Work& w, int64_t m) {
   return w.wix + m * atm8s_table_len(w.N);
 }
 
-// Build the slot tables of every molecule (one thread per molecule: O(G)).
-__global__ __launch_bounds__(64) void k_atm8s_index(Work w) {
-  const int64_t m = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (m >= w.B) return;
-  const int n = w.natom[m];
-  const int G = (n + kAtm8 - 1) / kAtm8;
-  const int64_t GN = n_groups8(w.N);
-  int64_t* t = w.wix + m * atm8s_table_len(w.N);
-  const int smax = atm8s_smax(n);
-  t[0] = smax;
-  int64_t pre = 0, base = 0;
-  for (int g = 0; g <= GN; ++g) {
-    t[1 + g] = pre;
-    t[GN + 2 + g] = base;
-    if (g < G) {
-      pre += atm8s_splits(G, g, smax);
-      base += pre;  // group g has one slot per item of x-groups 0 .. g
-    }
-  }
+// The molecule's part of pg: per x-group g the places of its chunk list
+// before pair tile (g, y), y = 0 .. G (row g of G + 1 entries, used from y = g
+// on), then the windows.
+__device__ __forceinline__ int32_t* atm8s_places(const Work& w, int64_t m) {
+  return reinterpret_cast<int32_t*>(w.pg + m * atm8s_stride(w.N));
 }
 
 // Near bits of the 8-atom groups: bit j of row i of molecule m is set when a
@@ -2247,12 +2237,133 @@ __global__ __launch_bounds__(64) void k_atm8s_near(Params p, Inputs in, Work w) 
   if (lane == 0) w.gnear[(m * GN + i) * WN + word] = bits;
 }
 
+// Third-atom groups z >= gy (word zw of the near bits) of pair tile (gx, gy).
+__device__ __forceinline__ unsigned long long atm8s_zword(const uint64_t* NX, const uint64_t* NY,
+                                                          bool nxy, int gy, int zw) {
+  const unsigned long long a = NX[zw], c = NY[zw];
+  const unsigned long long k = nxy ? (a | c) : (a & c);
+  return zw == (gy >> 6) ? k & (~0ull << (gy & 63)) : k;
+}
+
+// Chunk lists: one wave per (molecule, x-group), a lane per pair tile; a tile
+// with chunks takes kAtm8TileCost more places for its own loads and sums.
+__global__ __launch_bounds__(64) void k_atm8s_count(Params p, Inputs in, Work w) {
+  const int64_t GN = n_groups8(w.N), WN = near_words8(w.N);
+  const int64_t m = blockIdx.x / GN;
+  const int gx = (int)(blockIdx.x - m * GN);
+  const int G = (w.natom[m] + kAtm8 - 1) / kAtm8;
+  if (gx >= G) return;
+  const int lane = threadIdx.x;
+  const double* S8 = w.gsph8 + 4 * m * GN;
+  const double c3 = sqrt(p.cut3sq) * (1.0 + 1e-10) + 1e-10;  // margin for rounding in the bounds
+  const uint64_t* NEAR = w.gnear + m * GN * WN;
+  const uint64_t* NX = NEAR + gx * WN;
+  int32_t* pre = atm8s_places(w, m) + (int64_t)gx * (G + 1);
+  int done = 0;
+  for (int ybase = gx; ybase < G; ybase += 64) {
+    const int gy = ybase + lane;
+    int c = 0;
+    if (gy < G && sphere_gap(S8 + 4 * gx, S8 + 4 * gy) <= 2.0 * c3) {
+      const uint64_t* NY = NEAR + gy * WN;
+      const bool nxy = (NX[gy >> 6] >> (gy & 63)) & 1ull;
+      for (int zw = gy >> 6; zw * 64 < G; ++zw) c += __popcll(atm8s_zword(NX, NY, nxy, gy, zw));
+      if (c > 0) c += kAtm8TileCost;
+    }
+    int run = c;  // inclusive sum over the lanes
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(run, d);
+      if (lane >= d) run += v;
+    }
+    if (gy < G) pre[gy] = done + run - c;
+    done += __shfl(run, 63);
+  }
+  if (lane == 0) pre[G] = done;
+}
+
+// Work items of every molecule: x-group g with w_g places gets 1 + w_g G / (u
+// (G - g)) items (of at least eight places), u the smallest size for which the
+// windows (an item of g has one per group from g on) and the grid suffice.
+// Later groups, whose items need fewer windows and run last, are split finer:
+// the kernel ends evenly.
+__global__ __launch_bounds__(256) void k_atm8s_index(Work w) {
+  __shared__ int64_t s_a[256], s_b[256];
+  const int64_t m = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int n = w.natom[m];
+  const int G = (n + kAtm8 - 1) / kAtm8;
+  const int64_t GN = n_groups8(w.N);
+  const int32_t* pre = atm8s_places(w, m);
+  int64_t* t = w.wix + m * atm8s_table_len(w.N);
+  auto places = [&](int g) { return (int64_t)pre[(int64_t)g * (G + 1) + G]; };
+  int64_t W = 0, X = 0;
+  for (int g = tid; g < G; g += 256) {
+    const int64_t wg = places(g);
+    W += wg;
+    X += wg * G / (G - g) + 1;
+  }
+  s_a[tid] = W;
+  s_b[tid] = X;
+  __syncthreads();
+  for (int d = 128; d >= 1; d >>= 1) {
+    if (tid < d) {
+      s_a[tid] += s_a[tid + d];
+      s_b[tid] += s_b[tid + d];
+    }
+    __syncthreads();
+  }
+  W = s_a[0];
+  X = s_b[0];
+  const int64_t room = atm8s_windows(n) - (int64_t)G * (G + 1) / 2;
+  const int64_t items = atm8s_blocks_per_mol(n) - G;
+  int64_t u = 1;
+  if (G > 0) {
+    const int64_t u1 = room > 0 ? (W * G + room - 1) / room : INT64_MAX / (G + 1);
+    const int64_t u2 = (X + items - 1) / items;
+    u = max((int64_t)1, max(u1, u2));
+  }
+  int64_t pre0 = 0, base0 = 0;  // items and slots before this round of 256 groups
+  for (int g0 = 0; g0 <= GN; g0 += 256) {
+    const int g = g0 + tid;
+    int64_t S = 0;
+    if (g < G) {
+      const int64_t wg = places(g);
+      S = 1 + min(wg * G / (u * (G - g)), wg / 8);
+    }
+    // inclusive sums of S, then of the items up to each group
+    __syncthreads();
+    s_a[tid] = S;
+    __syncthreads();
+    for (int d = 1; d < 256; d <<= 1) {
+      const int64_t v = tid >= d ? s_a[tid - d] : 0;
+      __syncthreads();
+      s_a[tid] += v;
+      __syncthreads();
+    }
+    const int64_t upto = pre0 + s_a[tid], slots = g < G ? upto : 0;
+    s_b[tid] = slots;
+    __syncthreads();
+    for (int d = 1; d < 256; d <<= 1) {
+      const int64_t v = tid >= d ? s_b[tid - d] : 0;
+      __syncthreads();
+      s_b[tid] += v;
+      __syncthreads();
+    }
+    if (g <= GN) {
+      t[1 + g] = upto - S;
+      t[GN + 2 + g] = base0 + s_b[tid] - slots;  // group g: a slot per item of groups 0 .. g
+      if (g == GN) t[0] = upto;
+    }
+    pre0 += s_a[255];
+    base0 += s_b[255];
+  }
+}
+
 template <bool ENERGY, bool GRAD, bool PG>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_atm8s(
     Params p, Inputs in, Work w, int64_t nblocks) {
   constexpr int NA = kAtm1Acc;
   constexpr int T8 = kAtm8;
-  constexpr int KS = kAtm8sMaxSplits;
   constexpr int kWin = NA * T8;  // doubles per slot: [NA][8 atoms]
   __shared__ __align__(16) double s_zc[T8 * kAtm8Row<GRAD>];
   __shared__ double s_red[NA][64];
@@ -2263,46 +2374,58 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const int64_t N = w.N;
   const int64_t per_mol = atm8s_blocks_per_mol(N);
   const int64_t m = b / per_mol;
-  // block r of a molecule runs on XCD r % 8: x-group gx stays on XCD gx % 8
-  // with all its splits, and the heavy low groups come first
-  const int r = (int)(b - m * per_mol);
-  const int s = (r >> 3) % KS, gx = ((r >> 3) / KS) * 8 + (r & 7);
+  // block r of a molecule runs on XCD r % 8: eight consecutive items (mostly
+  // of one x-group) on one XCD, the next eight on the next
+  const int r = (int)(b - m * per_mol), rq = r >> 3;
+  const int64_t item = ((rq >> 3) * 8 + (r & 7)) * 8 + (rq & 7);
   const int n = w.natom[m];
   const int G = (n + T8 - 1) / T8;
+  const int64_t GN = n_groups8(N);
   const int64_t* tab = atm8s_table(w, m);
-  const int smax = (int)tab[0];
-  const int S = gx < G ? atm8s_splits(G, gx, smax) : 0;
-  if (s >= S) {
+  if (item >= tab[0]) {
     if (PG && lane < 4) w.pg3[b * 4 + lane] = 0.0;
     return;
   }
-  const int64_t GN = n_groups8(N);
-  const int64_t slot = tab[1 + gx] + s;  // this item's slot in the list of every group >= gx
+  // the item's x-group: the last one whose first item is not behind it
+  int gx = 0;
+  for (int len = G; len > 1;) {
+    const int step = (len + 63) / 64, g = gx + lane * step;
+    const bool le = lane * step < len && tab[1 + g] <= item;
+    const int k = __popcll(__ballot(le)) - 1;
+    gx += k * step;
+    len = min(step, len - k * step);
+  }
+  const int s = (int)(item - tab[1 + gx]), S = (int)(tab[2 + gx] - tab[1 + gx]);
   const int64_t* gbase = tab + GN + 2;
-  double* win = w.pg + m * atm8s_stride(N);
-  auto slot_of = [&](int g) { return win + (gbase[g] + slot) * kWin; };
+  double* win = w.pg + m * atm8s_stride(N) + atm8s_head(n);
+  auto slot_of = [&](int g) { return win + (gbase[g] + item) * kWin; };
   for (int g = gx; g < G; ++g)
     if (lane < kWin) slot_of(g)[lane] = 0.0;
   __syncthreads();
 
   const int64_t* Z = in.numbers + m * N;
-  const double* S8 = w.gsph8 + 4 * m * GN;
-  const double* SX = S8 + 4 * gx;
-  const double c3 = sqrt(p.cut3sq) * (1.0 + 1e-10) + 1e-10;  // margin for rounding in the bounds
   const int64_t WN = near_words8(N);
   const uint64_t* NEAR = w.gnear + m * GN * WN;
   const uint64_t* NX = NEAR + gx * WN;
   const int x = gx * T8 + tx;
   Atm8Sums u = {};
-  int kept = 0;  // pair tiles of this x-group seen so far
+  // this item's share [lo, hi) of the places of the x-group
+  const int32_t* pre = atm8s_places(w, m) + (int64_t)gx * (G + 1);
+  const int total = pre[G];
+  const int lo = (int)((int64_t)total * s / S), hi = (int)((int64_t)total * (s + 1) / S);
   for (int ybase = gx; ybase < G; ybase += 64) {
     const int cand = ybase + lane;
-    const bool ykeep = cand < G && sphere_gap(SX, S8 + 4 * cand) <= 2.0 * c3;
-    unsigned long long ymask = __ballot(ykeep);
+    const int at0 = cand < G ? pre[cand] : total, at1 = cand < G ? pre[cand + 1] : total;
+    // (tiles without chunks take no place)
+    unsigned long long ymask = __ballot(at1 > at0 && at0 < hi && at1 > lo);
     while (ymask) {
-      const int gy = ybase + __builtin_ctzll(ymask);
+      const int yl = __builtin_ctzll(ymask), gy = ybase + yl;
       ymask &= ymask - 1;
-      if (kept++ % S != s) continue;
+      // the tile's chunks [c0, c1) of the share
+      const int p0 = __shfl(at0, yl) + kAtm8TileCost;
+      int skip = max(0, lo - p0);
+      int left = min(__shfl(at1, yl), hi) - p0 - skip;
+      if (left <= 0) continue;
       const uint64_t* NY = NEAR + gy * WN;
       const bool nxy = (NX[gy >> 6] >> (gy & 63)) & 1ull;
       const int y = gy * T8 + ty;
@@ -2315,14 +2438,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       // bits: two of near(x, y), near(x, z), near(y, z) set (groups past the
       // molecule have no bits)
       int zw = gy >> 6;
-      auto zscan = [&]() {
-        const unsigned long long a = NX[zw], c = NY[zw];
-        unsigned long long k = nxy ? (a | c) : (a & c);
-        if (zw == (gy >> 6)) k &= ~0ull << (gy & 63);
-        return k;
-      };
-      unsigned long long zmask = zscan();
+      unsigned long long zmask = atm8s_zword(NX, NY, nxy, gy, zw);
+      while (skip > 0) {
+        const int c = __popcll(zmask);
+        if (c <= skip) {
+          skip -= c;
+          ++zw;
+          zmask = zw * 64 < G ? atm8s_zword(NX, NY, nxy, gy, zw) : 0ull;
+          if (zw * 64 >= G) break;
+        } else {
+          for (; skip > 0; --skip) zmask &= zmask - 1;
+        }
+      }
       auto next_z = [&]() {
+        if (left-- <= 0) return G;
         while (true) {
           if (zmask) {
             const int g = zw * 64 + __builtin_ctzll(zmask);
@@ -2331,7 +2460,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
           }
           ++zw;
           if (zw * 64 >= G) return G;
-          zmask = zscan();
+          zmask = atm8s_zword(NX, NY, nxy, gy, zw);
         }
       };
       Atm8Chunk ch;
@@ -2418,7 +2547,7 @@ __global__ __launch_bounds__(1024) void k_atm8s_rows(Inputs in, Work w, double* 
   if (g < G && j < J) {
     const int64_t* tab = atm8s_table(w, m);
     const int64_t cnt = tab[1 + g + 1];  // items of x-groups 0 .. g
-    const double* src = w.pg + m * atm8s_stride(N) + tab[GN + 2 + g] * kWin + v;
+    const double* src = w.pg + m * atm8s_stride(N) + atm8s_head(n) + tab[GN + 2 + g] * kWin + v;
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
     int64_t k = j;
     for (; k + 3 * J < cnt; k += 4 * J) {
@@ -2941,7 +3070,9 @@ hipError_t launch_atm8s(hipStream_t s, const Params& p, const Inputs& in, const 
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_atm8s_near, dim3((unsigned)(w.B * n_groups8(w.N) * near_words8(w.N))),
                      dim3(64), 0, s, p, in, w);
-  hipLaunchKernelGGL(k_atm8s_index, dim3((unsigned)((w.B + 63) / 64)), dim3(64), 0, s, w);
+  hipLaunchKernelGGL(k_atm8s_count, dim3((unsigned)(w.B * n_groups8(w.N))), dim3(64), 0, s, p, in,
+                     w);
+  hipLaunchKernelGGL(k_atm8s_index, dim3((unsigned)w.B), dim3(256), 0, s, w);
   const dim3 g((unsigned)nblocks), blk(64);
   if (energy && grad)
     hipLaunchKernelGGL((k_atm8s<true, true, false>), g, blk, 0, s, p, in, w, nblocks);

@@ -49,3 +49,32 @@ def test_parts_of_the_chunk_list(n, cutoff):
         if ref is not None and not any(n <= edge < pad for edge in (140, 160, 201, 255)):
             assert torch.equal(ref[0], e[:, :n]) and torch.equal(ref[1], g[:, :n])
         ref = (e, g)
+
+
+@pytest.mark.parametrize("cutoff", [40.0, 14.0])
+@pytest.mark.parametrize("n", [257, 264, 265, 519, 778])
+def test_items_of_the_screened_kernel(n, cutoff):
+    """Large molecules: the shares of the x-groups' chunk lists against the
+    pair-owner kernel (each triple from its three pairs), one of two molecules
+    shorter and with padding atoms inside; parameter gradients, sums of all
+    triples, to 1e-10 of their size."""
+    print(f"[case] screened three-body n = {n}, cutoff {cutoff}", flush=True)
+    rng = np.random.default_rng(500 + n)
+    mols = [synth.molecule(rng, k, synth.MIX_HCNO, 2.8, (0,)) for k in (n, n // 3)]
+    numbers, positions, charge = synth.pack(mols, pad_to=n + 5)
+    numbers[1, 20:37] = 0  # two whole groups and more without atoms
+    dev = [t.cuda() for t in (numbers, positions, charge)]
+    par = dict(s8=1.2, a1=0.4, a2=5.0, cutoff_disp3=cutoff)
+    kp, ko = runtime.KernelParams(**par), runtime.KernelParams(**par, pair_owner=True)
+    e, g, _ = runtime.energy_gradient(*dev, kp)
+    eo, go, _ = runtime.energy_gradient(*dev, ko)
+    assert (e - eo).abs().max().item() < 1e-13
+    assert (g - go).abs().max().item() < 1e-12
+    w = torch.linspace(0.5, 1.5, n + 5, dtype=torch.float64, device="cuda").expand(2, n + 5)
+    ef, ws = runtime.forward(*dev, kp)
+    gb, pb = runtime.backward(*dev, kp, ws, w.contiguous(), params=True)
+    efo, wso = runtime.forward(*dev, ko)
+    gbo, pbo = runtime.backward(*dev, ko, wso, w.contiguous(), params=True)
+    assert (ef - efo).abs().max().item() < 1e-13
+    assert (gb - gbo).abs().max().item() < 1e-12
+    assert ((pb - pbo).abs() <= 1e-10 * pbo.abs()).all()
