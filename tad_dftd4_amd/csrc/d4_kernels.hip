@@ -144,15 +144,40 @@ __device__ __forceinline__ double sum_lanes8(double v) {
 // step starts with one launch instead of three.
 constexpr int kCnWaves = 8;
 
-template <bool ZS>
+// Tiles (A, b) of block row A in the order and grouping of the two kernels
+// below, which deal tile tl = by (by + 1) / 2 + bx to wave tl % 8: value of
+// component c, atom a of block A, from the tiles of wave k in rising tl. sums
+// holds [c][b][2][8]: the row sums (b <= A: block A is the y block; sign sy)
+// and the column sums (b >= A: the x block).
+__device__ __forceinline__ double tile_row_sum(const double* sums, int nb, int A, int a, int c,
+                                               int k, bool minus) {
+  double f = 0.0;
+  for (int b = 0; b < nb; ++b) {
+    const int by = max(A, b), bx = min(A, b);
+    if (((by * (by + 1) / 2 + bx) & 7) != k) continue;
+    const double* e = sums + ((c * nb + b) * 2) * 8 + a;
+    if (b <= A) f = minus ? f - e[0] : f + e[0];
+    if (b >= A) f += e[8];
+  }
+  return f;
+}
+
+// ROWS: a work-group per 8-atom block A of a molecule instead of one per
+// molecule; it takes the tiles of block row A (each pair twice over the
+// molecule) and forms the same sums in the same order, so the results are the
+// same bits.
+template <bool ZS, bool ROWS>
 __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p, Inputs in,
                                                             Work w) {
   extern __shared__ double s_dyn[];  // [n][4] x, y, z, Z; [kCnWaves][2][n] sums
   __shared__ int s_red[2][kCnWaves];
   __shared__ int s_present[kMaxZ];
   constexpr int NT = 64 * kCnWaves;
-  const int64_t m = blockIdx.x;
   const int64_t N = w.N;
+  const int rb = ROWS ? (int)((N + 7) >> 3) : 1;  // work-groups per molecule
+  const int64_t m = blockIdx.x / rb;
+  const int A = (int)(blockIdx.x - m * rb);
+  const bool lead = A == 0;  // stores the molecule's extent, status, slots and box
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   int n;
   {
@@ -163,7 +188,7 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
       if (zi != 0) last = (int)i;
       if (zi < 0 || zi >= kMaxZ) bad = 1;
     }
-    if (ZS)
+    if (ZS && lead)
       for (int e = tid; e < kMaxZ; e += NT) s_present[e] = 0;
     last = wave_max(last);
     bad = wave_or(bad);
@@ -179,11 +204,11 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
     last = max(last, s_red[0][0]);
     bad |= s_red[1][0];
     n = bad ? 0 : last + 1;
-    if (tid == 0) {
+    if (tid == 0 && lead) {
       w.natom[m] = n;
       w.status[m] = bad ? kStatusBadZ : 0;
     }
-    if (ZS) {
+    if (ZS && lead) {
       // element slots: the molecule's distinct elements in increasing Z
       for (int i = tid; i < n; i += NT) {
         const int64_t zi = z[i];
@@ -220,8 +245,11 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
     at[2] = R[3 * i + 2];
     at[3] = (double)Z[i];
   }
-  for (int e = tid; e < kCnWaves * 2 * n; e += NT) s_f[e] = 0.0;
-  {
+  if (!ROWS)
+    for (int e = tid; e < kCnWaves * 2 * n; e += NT) s_f[e] = 0.0;
+  if (!lead) {
+    __syncthreads();
+  } else {
     // the molecule's bounding box (the three-body kernel reads its squared
     // diagonal: a molecule inside the cutoff sphere has no screening)
     __shared__ double s_bb[kCnWaves][6];
@@ -251,13 +279,19 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
     }
   }
   const int nb = (n + 7) >> 3;
-  const int tiles = nb * (nb + 1) / 2;
+  const int tiles = ROWS ? (A < nb ? nb : 0) : nb * (nb + 1) / 2;
   double* f = s_f + (size_t)wv * 2 * n;
   for (int tl = wv; tl < tiles; tl += kCnWaves) {
-    int by = (int)((sqrt(8.0 * tl + 1.0) - 1.0) * 0.5);
-    while (by * (by + 1) / 2 > tl) --by;
-    while ((by + 1) * (by + 2) / 2 <= tl) ++by;
-    const int bx = tl - by * (by + 1) / 2;
+    int bx, by;
+    if (ROWS) {
+      bx = min(A, tl);
+      by = max(A, tl);
+    } else {
+      by = (int)((sqrt(8.0 * tl + 1.0) - 1.0) * 0.5);
+      while (by * (by + 1) / 2 > tl) --by;
+      while ((by + 1) * (by + 2) / 2 <= tl) ++by;
+      bx = tl - by * (by + 1) / 2;
+    }
     const int x = 8 * bx + tx, y = 8 * by + ty;
     double v[2] = {0.0, 0.0};  // D4 CN term, EEQ CN term
     if (x < y && y < n) {
@@ -281,12 +315,25 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
       cs += __shfl_xor(cs, 8);
       cs += __shfl_xor(cs, 16);
       cs += __shfl_xor(cs, 32);
-      if (tx == 0 && y < n) f[c * n + y] += rs;
-      if (ty == 0 && x < n) f[c * n + x] += cs;
+      if (ROWS) {
+        double* e = s_f + ((c * nb + tl) * 2) * 8;
+        if (tx == 0) e[ty] = rs;
+        if (ty == 0) e[8 + tx] = cs;
+      } else {
+        if (tx == 0 && y < n) f[c * n + y] += rs;
+        if (ty == 0 && x < n) f[c * n + x] += cs;
+      }
     }
   }
   __syncthreads();
-  for (int i = tid; i < N; i += NT) {
+  if (ROWS) {
+    // thread (c, k, a): wave k's part of component c of atom 8 A + a
+    double* part = s_f + (size_t)2 * nb * 16;
+    if (A < nb && tid < 128)
+      part[tid] = tile_row_sum(s_f, nb, A, tid & 7, tid >> 6, (tid >> 3) & 7, false);
+    __syncthreads();
+  }
+  for (int i = ROWS ? 8 * A + tid : tid; i < (ROWS ? min((int)N, 8 * A + 8) : N); i += NT) {
     const int64_t row = m * N + i;
     if (i >= n || s_at[4 * i + 3] == 0.0) {
       w.cn[row] = 0.0;
@@ -296,8 +343,14 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
     }
     double s4 = 0.0, se = 0.0;
     for (int k = 0; k < kCnWaves; ++k) {
-      s4 += s_f[(size_t)k * 2 * n + i];
-      se += s_f[(size_t)k * 2 * n + n + i];
+      if (ROWS) {
+        const double* part = s_f + (size_t)2 * nb * 16 + 8 * k + (i - 8 * A);
+        s4 += part[0];
+        se += part[64];
+      } else {
+        s4 += s_f[(size_t)k * 2 * n + i];
+        se += s_f[(size_t)k * 2 * n + n + i];
+      }
     }
     w.cn[row] = s4;
     // smooth cap: log(1 + e^cmax) - log(1 + e^(cmax - cn))
@@ -2699,14 +2752,17 @@ __global__ __launch_bounds__(256) void k_chain(DevTables t, Params p, Inputs in,
 constexpr int kChainAtom = 8;   // doubles per staged atom: x, y, z, dL/dCN, beta, lam, q, Z
 constexpr int kChainWaves = 8;  // waves per work-group
 
+template <bool ROWS>
 __global__ __launch_bounds__(64 * kChainWaves) void k_chain_sym(DevTables t, Params p,
                                                                   Inputs in, Work w,
                                                                   double* grad_out) {
   extern __shared__ double s_dyn[];  // [n][kChainAtom] atoms, [kChainWaves][3][n] sums
-  const int64_t m = blockIdx.x;
   const int64_t N = w.N;
+  const int rb = ROWS ? (int)((N + 7) >> 3) : 1;  // work-groups per molecule
+  const int64_t m = blockIdx.x / rb;
+  const int A = (int)(blockIdx.x - m * rb);
   const int n = w.natom[m];
-  if (n < 2) return;
+  if (n < 2 || 8 * A >= n) return;
   constexpr int NT = 64 * kChainWaves;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int tx = lane & 7, ty = lane >> 3;
@@ -2727,16 +2783,23 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_chain_sym(DevTables t, Par
     at[6] = eeq ? w.q[row] : 0.0;
     at[7] = (double)Z[i];
   }
-  for (int e = tid; e < kChainWaves * 3 * n; e += NT) s_f[e] = 0.0;
+  if (!ROWS)
+    for (int e = tid; e < kChainWaves * 3 * n; e += NT) s_f[e] = 0.0;
   __syncthreads();
   const int nb = (n + 7) >> 3;
-  const int tiles = nb * (nb + 1) / 2;
+  const int tiles = ROWS ? nb : nb * (nb + 1) / 2;
   double* f = s_f + (size_t)wv * 3 * n;
   for (int tl = wv; tl < tiles; tl += kChainWaves) {
-    int by = (int)((sqrt(8.0 * tl + 1.0) - 1.0) * 0.5);
-    while (by * (by + 1) / 2 > tl) --by;
-    while ((by + 1) * (by + 2) / 2 <= tl) ++by;
-    const int bx = tl - by * (by + 1) / 2;
+    int bx, by;
+    if (ROWS) {
+      bx = min(A, tl);
+      by = max(A, tl);
+    } else {
+      by = (int)((sqrt(8.0 * tl + 1.0) - 1.0) * 0.5);
+      while (by * (by + 1) / 2 > tl) --by;
+      while ((by + 1) * (by + 2) / 2 <= tl) ++by;
+      bx = tl - by * (by + 1) / 2;
+    }
     const int x = 8 * bx + tx, y = 8 * by + ty;
     double fc[3] = {0.0, 0.0, 0.0};
     if (x < y && y < n) {
@@ -2775,11 +2838,30 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_chain_sym(DevTables t, Par
       cs += __shfl_xor(cs, 8);
       cs += __shfl_xor(cs, 16);
       cs += __shfl_xor(cs, 32);
-      if (tx == 0 && y < n) f[c * n + y] -= rs;
-      if (ty == 0 && x < n) f[c * n + x] += cs;
+      if (ROWS) {
+        double* e = s_f + ((c * nb + tl) * 2) * 8;
+        if (tx == 0) e[ty] = rs;
+        if (ty == 0) e[8 + tx] = cs;
+      } else {
+        if (tx == 0 && y < n) f[c * n + y] -= rs;
+        if (ty == 0 && x < n) f[c * n + x] += cs;
+      }
     }
   }
   __syncthreads();
+  if (ROWS) {
+    // thread (c, k, a): wave k's part of component c of atom 8 A + a
+    double* part = s_f + (size_t)3 * nb * 16;
+    if (tid < 192) part[tid] = tile_row_sum(s_f, nb, A, tid & 7, tid >> 6, (tid >> 3) & 7, true);
+    __syncthreads();
+    const int a = tid & 7, c = tid >> 3, i = 8 * A + a;
+    if (c < 3 && i < n && s_at[kChainAtom * i + 7] != 0.0) {
+      double g = 0.0;
+      for (int k = 0; k < kChainWaves; ++k) g += part[64 * c + 8 * k + a];
+      grad_out[(m * N + i) * 3 + c] += g;
+    }
+    return;
+  }
   for (int e = tid; e < 3 * n; e += NT) {
     const int c = e / n, i = e - c * n;
     if (s_at[kChainAtom * i + 7] == 0.0) continue;
@@ -2939,6 +3021,16 @@ inline unsigned rows_grid(const Work& w) {
 
 }  // namespace
 
+// Work-groups per block row instead of per molecule in the tiled coordination-
+// number and chain passes: where the molecules are fewer than their padded
+// length, one work-group's walk over a molecule (its tiles / 8, about 1.3 us
+// each) is longer than the doubled pair work on the whole chip. Coordination
+// numbers / chain in us, per molecule against per row: 1 x 250 atoms 33 / 45
+// against 10 / 9, 64 x 160 36 / 50 against 18 / 20, 64 x 80 14 / 17 against 10 /
+// 11, 128 x 80 15 / 17 against 17 / 17, 256 x 200 55 / 80 against 66 / 85, 256 x
+// 60 12 / 12 against 28 / 22.
+inline bool tile_rows(const Work& w) { return w.B <= w.N; }
+
 // ------------------------------------------------------------------ launchers
 
 hipError_t launch_prep(hipStream_t s, const Inputs& in, const Work& w) {
@@ -2951,14 +3043,20 @@ hipError_t launch_cn(hipStream_t s, const DevTables& t, const Params& p,
                      const Inputs& in, const Work& w) {
   if (w.N <= kAtm1MaxN) {
     if (w.B == 0) return hipSuccess;
-    const size_t shmem = sizeof(double) * (size_t)(4 + 2 * kCnWaves) * (size_t)w.N;
+    const bool rows = tile_rows(w);
+    const size_t nb = (size_t)(w.N + 7) / 8;
+    const size_t shmem = sizeof(double) * (rows ? 4 * (size_t)w.N + 32 * nb + 128
+                                                : (size_t)(4 + 2 * kCnWaves) * (size_t)w.N);
     // (also the extents, the Z check and, for D4, the element slots)
-    if (p.d4s)
-      hipLaunchKernelGGL(k_cn_sym<false>, dim3((unsigned)w.B), dim3(64 * kCnWaves), shmem, s, t,
-                         p, in, w);
+    const dim3 g((unsigned)(rows ? w.B * (int64_t)nb : w.B)), blk(64 * kCnWaves);
+    if (p.d4s && rows)
+      hipLaunchKernelGGL((k_cn_sym<false, true>), g, blk, shmem, s, t, p, in, w);
+    else if (p.d4s)
+      hipLaunchKernelGGL((k_cn_sym<false, false>), g, blk, shmem, s, t, p, in, w);
+    else if (rows)
+      hipLaunchKernelGGL((k_cn_sym<true, true>), g, blk, shmem, s, t, p, in, w);
     else
-      hipLaunchKernelGGL(k_cn_sym<true>, dim3((unsigned)w.B), dim3(64 * kCnWaves), shmem, s, t,
-                         p, in, w);
+      hipLaunchKernelGGL((k_cn_sym<true, false>), g, blk, shmem, s, t, p, in, w);
     return hipGetLastError();
   }
   D4_LAUNCH_ROWS((k_cn<16>), (k_cn<32>), (k_cn<64>), s, p, w, t, p, in, w);
@@ -3159,9 +3257,16 @@ hipError_t launch_chain(hipStream_t s, const DevTables& t, const Params& p,
     // at most (8 + 3 * 8) * 256 doubles = 64 KiB, the default dynamic LDS limit
     static_assert((kChainAtom + 3 * kChainWaves) * kAtm1MaxN * sizeof(double) <= 65536, "LDS");
     if (w.B == 0) return hipSuccess;
-    const size_t shmem = sizeof(double) * (size_t)(kChainAtom + 3 * kChainWaves) * (size_t)w.N;
-    hipLaunchKernelGGL(k_chain_sym, dim3((unsigned)w.B), dim3(64 * kChainWaves), shmem, s, t, p,
-                       in, w, grad_out);
+    const bool rows = tile_rows(w);
+    const size_t nb = (size_t)(w.N + 7) / 8;
+    const size_t shmem = sizeof(double) * (rows ? kChainAtom * (size_t)w.N + 48 * nb + 192
+                                                : (size_t)(kChainAtom + 3 * kChainWaves) *
+                                                      (size_t)w.N);
+    const dim3 g((unsigned)(rows ? w.B * (int64_t)nb : w.B)), blk(64 * kChainWaves);
+    if (rows)
+      hipLaunchKernelGGL(k_chain_sym<true>, g, blk, shmem, s, t, p, in, w, grad_out);
+    else
+      hipLaunchKernelGGL(k_chain_sym<false>, g, blk, shmem, s, t, p, in, w, grad_out);
     return hipGetLastError();
   }
   D4_LAUNCH_ROWS((k_chain<16>), (k_chain<32>), (k_chain<64>), s, p, w, t, p, in, w, grad_out);
