@@ -11,6 +11,7 @@
 // on its neighbours in the batch), and every output element has exactly one
 // writer, so results are bitwise reproducible and independent of batching.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "d4_device.h"
@@ -1647,9 +1648,15 @@ constexpr double kAtmFar = 1.0e6;  // position of lanes and third atoms without 
 // generator of GF(8): linear over xor like zl << 4 above, and both zl and
 // (zl ^ k) -> zl ^ skew(zl ^ k) are one-to-one, so the eight lanes of a row
 // again read distinct bank groups.
-constexpr int kAtm8RecZ = 16, kAtm8RecRt = 17;
+// Parameter gradients stage a second block of the first layout behind it: (L,
+// A, B, -) of each pair record, L = log t, A and B = d log R0 / d a1 and / d a2.
+// One logarithm and one reciprocal per staged pair in place of a logarithm and
+// two reciprocals per triple: 384 x 6-60 atoms 147 -> 77 us (no spills).
+constexpr int kAtm8RecZ = 16, kAtm8RecZ2 = 17;  // third-atom records (the second: energies)
 template <bool GRAD>
 constexpr int kAtm8Row = GRAD ? 128 : 64;  // doubles per row
+template <bool GRAD, bool PG>
+constexpr int kAtm8Lds = (PG ? 2 : 1) * kAtm8 * kAtm8Row<GRAD>;  // doubles of a chunk
 __device__ __forceinline__ uint32_t atm8_skew(uint32_t zl) {
   return ((zl << 1) & 7u) ^ ((zl >> 2) * 3u);
 }
@@ -1676,11 +1683,10 @@ __device__ __forceinline__ const T* atm8_at(const double* s_zc, uint32_t off) {
 struct Atm8Pair {
   double rx0, rx1, rx2, ry0, ry1, ry2;  // positions
   double a, ia, a2, asq;                // r_xy^2, 1 / r_xy^2, 2 r_xy^2, r_xy^4
-  double txy, pxy, pxy0;                // t_xy, s9 p_xy, p_xy
+  double txy, pxy, pxy0;                // t_xy, s9 p_xy, p_xy (parameter gradients)
   double kxy, kyx;                      // d log sqrt|C6(0)_xy| / d CN_x, / d CN_y
   double gx, gy, gxy;                   // dL/dE of x, y and their sum
   double mxy;                           // 1 if r_xy is within the cutoff
-  double rx4, ry4, Axy, Bxy;            // parameter gradients
 };
 
 template <bool GRAD, bool PG>
@@ -1694,7 +1700,6 @@ __device__ __forceinline__ Atm8Pair atm8_pair(const Params& p, const Inputs& in,
   q.a2 = 2.0;
   q.txy = q.pxy = q.pxy0 = q.kxy = q.kyx = 0.0;
   q.gx = q.gy = q.mxy = 0.0;
-  q.rx4 = q.ry4 = q.Axy = q.Bxy = 0.0;
   if (valid) {
     const double* pt = w.pt + m * N * N;
     const double* pp = w.pp + m * N * N;
@@ -1720,13 +1725,6 @@ __device__ __forceinline__ Atm8Pair atm8_pair(const Params& p, const Inputs& in,
       q.gx = in.gE ? in.gE[m * N + x] : 1.0;
       q.gy = in.gE ? in.gE[m * N + y] : 1.0;
     }
-    if (PG) {
-      q.rx4 = w.rt4[m * N + x];
-      q.ry4 = w.rt4[m * N + y];
-      const double sig = 1.7320508075688772 * q.rx4 * q.ry4;
-      q.Bxy = 1.0 / fma(p.a1, sig, p.a2);
-      q.Axy = sig * q.Bxy;
-    }
   }
   q.gxy = q.gx + q.gy;
   return q;
@@ -1737,13 +1735,39 @@ __device__ __forceinline__ Atm8Pair atm8_pair(const Params& p, const Inputs& in,
 struct Atm8Sums {
   double ex, ey, cx, cy, sca, fx0, fx1, fx2, fy0, fy1, fy2;
   double sal, sw;  // per tile: sums of al (x 1 / r_xy^2 into sca) and of We (x kxy, kyx)
-  double g_s9, g_alp, g_a1, g_a2;
+  double g_s9, g_alp, g_a1, g_a2, sd;  // sd: per tile, the sum of T dL/dT
 };
+
+// log t and the derivatives of log R0 by a1 and a2 of a pair (sx, sy: sqrt of
+// the atoms' r4r2); a pair without atoms (t = 0) has none
+struct Atm8Log {
+  double L, A, B;
+};
+__device__ __forceinline__ Atm8Log atm8_log(const Params& p, double t, double sx, double sy) {
+  if (!(t > 0.0)) return {0.0, 0.0, 0.0};
+  const double sig = 1.7320508075688772 * sx * sy;
+  const double B = rcp_nt(fma(p.a1, sig, p.a2));
+  return {log(t), sig * B, B};
+}
+
+// The pair's own share of the parameter gradients of a tile (x, y: its atoms).
+__device__ __forceinline__ void atm8_fold_pgrad(const Params& p, const Work& w, int64_t m, int x,
+                                                int y, bool valid, const Atm8Pair& q,
+                                                Atm8Sums& u) {
+  if (valid) {
+    const Atm8Log l = atm8_log(p, q.txy, w.rt4[m * w.N + x], w.rt4[m * w.N + y]);
+    u.g_alp = fma(u.sd, l.L, u.g_alp);
+    u.g_a1 = fma(u.sd, l.A, u.g_a1);
+    u.g_a2 = fma(u.sd, l.B, u.g_a2);
+  }
+  u.sd = 0.0;
+}
 
 // Records of one chunk (8 third atoms x 16 columns, two per lane) and the
 // third-atom data (lanes 0..7), held in registers until staged.
 struct Atm8Chunk {
-  double t[2], p[2], kz[2], kc[2], r[5];
+  double t[2], p[2], kz[2], kc[2], r[4];
+  double sz[2], sc[2];  // sqrt(r4r2) of the record's atoms (parameter gradients)
 };
 
 // Load the chunk of third atoms z0 .. z0 + 7 against the x block starting at
@@ -1763,6 +1787,7 @@ __device__ __forceinline__ void atm8_fetch(Atm8Chunk& c, const Inputs& in, const
     const int z = z0 + zl;
     const int col = cl < T8 ? x0 + cl : y0 + cl - T8;
     c.t[r] = c.p[r] = c.kz[r] = c.kc[r] = 0.0;
+    if (PG) c.sz[r] = c.sc[r] = 0.0;
     if (z < n && col < n) {
       const int64_t idx = (int64_t)z * N + col;
       c.t[r] = pt[idx];
@@ -1770,6 +1795,10 @@ __device__ __forceinline__ void atm8_fetch(Atm8Chunk& c, const Inputs& in, const
       if (GRAD) {
         c.kz[r] = pk[idx];
         c.kc[r] = pk[(int64_t)col * N + z];
+      }
+      if (PG) {
+        c.sz[r] = w.rt4[m * N + z];
+        c.sc[r] = w.rt4[m * N + col];
       }
     }
   }
@@ -1781,12 +1810,12 @@ __device__ __forceinline__ void atm8_fetch(Atm8Chunk& c, const Inputs& in, const
     c.r[1] = ok ? R[3 * z + 1] : kAtmFar;
     c.r[2] = ok ? R[3 * z + 2] : kAtmFar;
     c.r[3] = (GRAD && ok) ? (in.gE ? in.gE[m * N + z] : 1.0) : 0.0;
-    c.r[4] = (PG && ok) ? w.rt4[m * N + z] : 0.0;
   }
 }
 
 template <bool GRAD, bool PG>
-__device__ __forceinline__ void atm8_stage(const Atm8Chunk& c, double* s_zc, int lane) {
+__device__ __forceinline__ void atm8_stage(const Params& p, const Atm8Chunk& c, double* s_zc,
+                                           int lane) {
   char* base = reinterpret_cast<char*>(s_zc);
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
@@ -1795,6 +1824,12 @@ __device__ __forceinline__ void atm8_stage(const Atm8Chunk& c, double* s_zc, int
     double2* dst = reinterpret_cast<double2*>(base + atm8_rec<GRAD>(zl, cl));
     dst[0] = make_double2(c.t[r], c.p[r]);
     if (GRAD) dst[1] = make_double2(c.kz[r], c.kc[r]);
+    if (PG) {
+      const Atm8Log l = atm8_log(p, c.t[r], c.sz[r], c.sc[r]);
+      double2* dl = dst + kAtm8 * kAtm8Row<GRAD> / 2;
+      dl[0] = make_double2(l.L, l.A);
+      reinterpret_cast<double*>(dl + 1)[0] = l.B;
+    }
   }
   if (lane < kAtm8) {
     double2* r = reinterpret_cast<double2*>(base + atm8_rec<GRAD>(lane, kAtm8RecZ));
@@ -1802,8 +1837,7 @@ __device__ __forceinline__ void atm8_stage(const Atm8Chunk& c, double* s_zc, int
     if (GRAD)
       r[1] = make_double2(c.r[2], c.r[3]);
     else
-      *reinterpret_cast<double*>(base + atm8_rec<GRAD>(lane, kAtm8RecZ + 1)) = c.r[2];
-    if (PG) *reinterpret_cast<double*>(base + atm8_rec<GRAD>(lane, kAtm8RecRt)) = c.r[4];
+      *reinterpret_cast<double*>(base + atm8_rec<GRAD>(lane, kAtm8RecZ2)) = c.r[2];
   }
 }
 
@@ -1823,23 +1857,18 @@ __device__ __forceinline__ void atm8_chunk(const Params& p, const Atm8Pair& q, A
   const uint32_t ox = lrow ^ atm8_col<GRAD>(cx < 0 ? tx : cx);
   const uint32_t oy = lrow ^ atm8_col<GRAD>(cy < 0 ? T8 + ty : cy);
   const uint32_t oz = lrow ^ atm8_col<GRAD>(kAtm8RecZ);
-  const uint32_t ort = lrow ^ atm8_col<GRAD>(kAtm8RecRt);
-  const double c3sq = p.cut3sq, alp = p.alp, a1p = p.a1, a2p = p.a2, sq3 = 1.7320508075688772;
+  const uint32_t oz2 = lrow ^ atm8_col<GRAD>(kAtm8RecZ2);
+  const double c3sq = p.cut3sq, alp = p.alp;
   // alp T f = alp / 6 (1 - f), f = 1 / (1 + 6 T): H below needs no alp T
   const double alp6 = alp / 6.0, h0 = alp6 - 2.5;
-  // four steps per iteration (two with parameter gradients, whose extra
-  // sums would not fit the registers), so every ring move below is static
-#ifndef D4_ATM8_UNROLL
-#define D4_ATM8_UNROLL 4
-#endif
-  constexpr int kUnroll = PG ? 2 : D4_ATM8_UNROLL;
-  D4_UNROLL(kUnroll)
+  // four steps per iteration, so every ring move below is static
+  D4_UNROLL(4)
   for (int k = 0; k < T8; ++k) {
     const uint32_t ks = atm8_row<GRAD>((uint32_t)k);
     const double2* pz = atm8_at<double2>(s_zc, oz ^ ks);
     const double2 rz01 = pz[0];
     const double2 rz23 =
-        GRAD ? pz[1] : make_double2(*atm8_at<double>(s_zc, ort ^ ks), 0.0);
+        GRAD ? pz[1] : make_double2(*atm8_at<double>(s_zc, oz2 ^ ks), 0.0);
     const double4 rz = make_double4(rz01.x, rz01.y, rz23.x, rz23.y);
     // records of x and y against z = z0 + (tx ^ k)
     const double2* px = atm8_at<double2>(s_zc, ox ^ ks);
@@ -1942,14 +1971,18 @@ __device__ __forceinline__ void atm8_chunk(const Params& p, const Atm8Pair& q, A
       u.cy = fma(We, y23.y, u.cy);
       rr.D = fma(We, x23.x + y23.x, rr.D);
       if (PG) {
-        const double TdT = -6.0 * f * We * T;  // dL6/dT times T
+        // T dL6/dT goes with log T = the sum of the three pairs' L and with
+        // their A and B: the x and y edges of z here, the pair (x, y) by the
+        // tile's sum
+        const double TdT = -6.0 * f * We * T;
         u.g_s9 = fma(W6, P0 * f * g, u.g_s9);
-        u.g_alp = fma(TdT, T > 0.0 ? log(T) / alp : 0.0, u.g_alp);
-        const double rtz = *atm8_at<double>(s_zc, ort ^ ks);
-        const double sxz = sq3 * q.rx4 * rtz, syz = sq3 * q.ry4 * rtz;
-        const double bxz = rcp_nt(fma(a1p, sxz, a2p)), byz = rcp_nt(fma(a1p, syz, a2p));
-        u.g_a1 = fma(TdT * alp / 3.0, q.Axy + sxz * bxz + syz * byz, u.g_a1);
-        u.g_a2 = fma(TdT * alp / 3.0, q.Bxy + bxz + byz, u.g_a2);
+        const double2* lx = px + T8 * kAtm8Row<GRAD> / 2;
+        const double2* ly = py + T8 * kAtm8Row<GRAD> / 2;
+        const double2 lx01 = lx[0], ly01 = ly[0];
+        u.sd += TdT;
+        u.g_alp = fma(TdT, lx01.x + ly01.x, u.g_alp);
+        u.g_a1 = fma(TdT, lx01.y + ly01.y, u.g_a1);
+        u.g_a2 = fma(TdT, lx[1].x + ly[1].x, u.g_a2);
       }
     }
     // hand the sums for z to the lane that takes z at the next step:
@@ -1997,9 +2030,11 @@ __device__ __forceinline__ void atm8_stage_sums(double (*s_red)[64], int lane, d
 
 // Parameter-gradient partials of a wave: s9, alp, a1, a2 (the sums carry a
 // factor 6 from the screening weights).
-__device__ __forceinline__ void atm8_store_pgrad(const Atm8Sums& u, int lane, double* out) {
-  const double sixth = 1.0 / 6.0;
-  const double v4[4] = {u.g_s9 * sixth, u.g_alp * sixth, u.g_a1 * sixth, u.g_a2 * sixth};
+__device__ __forceinline__ void atm8_store_pgrad(const Params& p, const Atm8Sums& u, int lane,
+                                                 double* out) {
+  // T = prod t, t = (R0 / r)^(alp / 3): d log T / d alp = log T / alp
+  const double sixth = 1.0 / 6.0, third = p.alp / 18.0;
+  const double v4[4] = {u.g_s9 * sixth, u.g_alp * sixth / p.alp, u.g_a1 * third, u.g_a2 * third};
   for (int k = 0; k < 4; ++k) {
     const double v = wave_sum(v4[k]);
     if (lane == 0) out[k] = v;
@@ -2011,7 +2046,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     Params p, Inputs in, Work w, int S, int64_t nblocks) {
   constexpr int NA = GRAD ? kAtm1Acc : 1;
   constexpr int T8 = kAtm8;
-  __shared__ __align__(16) double s_zc[T8 * kAtm8Row<GRAD>];
+  __shared__ __align__(16) double s_zc[kAtm8Lds<GRAD, PG>];
   __shared__ double s_red[NA][64];
   double (*s_red2)[64] = reinterpret_cast<double (*)[64]>(s_zc);  // between two tiles
   static_assert(NA * 64 <= T8 * kAtm8Row<GRAD>, "s_red2");
@@ -2118,7 +2153,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     atm8_fetch<GRAD, PG>(ch, in, w, m, n, z1, bx * T8, by * T8, lane);
     for (int z0 = z1; z0 < zend; z0 += T8) {
       __syncthreads();
-      atm8_stage<GRAD, PG>(ch, s_zc, lane);
+      atm8_stage<GRAD, PG>(p, ch, s_zc, lane);
       __syncthreads();
       if (z0 + T8 < zend)  // in flight during this chunk
         atm8_fetch<GRAD, PG>(ch, in, w, m, n, z0 + T8, bx * T8, by * T8, lane);
@@ -2164,6 +2199,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       u.ey = u.ex;
     }
     atm8_fold_sca(q, u);
+    if (PG) atm8_fold_pgrad(p, w, m, x, y, valid, q, u);
     __syncthreads();
     atm8_stage_sums<GRAD>(s_red, lane, u.ex, u.fx0, u.fx1, u.fx2, u.cx, gs);
     atm8_stage_sums<GRAD>(s_red2, lane, u.ey, u.fy0, u.fy1, u.fy2, u.cy, gs);
@@ -2203,7 +2239,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     const int c = e / n, i = e - c * n;
     part[c * N + i] = s_acc[e];
   }
-  if (PG) atm8_store_pgrad(u, lane, w.pg3 + (m * (int64_t)S + s) * 4);
+  if (PG) atm8_store_pgrad(p, u, lane, w.pg3 + (m * (int64_t)S + s) * 4);
 }
 
 // --------------------------------------------------------------------------
@@ -2418,7 +2454,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   constexpr int NA = kAtm1Acc;
   constexpr int T8 = kAtm8;
   constexpr int kWin = NA * T8;  // doubles per slot: [NA][8 atoms]
-  __shared__ __align__(16) double s_zc[T8 * kAtm8Row<GRAD>];
+  __shared__ __align__(16) double s_zc[kAtm8Lds<GRAD, PG>];
   __shared__ double s_red[NA][64];
 
   const int64_t b = blockIdx.x;
@@ -2521,7 +2557,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       if (gz < G) atm8_fetch<GRAD, PG>(ch, in, w, m, n, gz * T8, gx * T8, gy * T8, lane);
       while (gz < G) {
         __syncthreads();
-        atm8_stage<GRAD, PG>(ch, s_zc, lane);
+        atm8_stage<GRAD, PG>(p, ch, s_zc, lane);
         __syncthreads();
         const int gzn = next_z();
         if (gzn < G)  // in flight during this chunk
@@ -2551,6 +2587,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       }
       // the y atoms' tile sums (over the columns)
       atm8_fold_sca(q, u);
+      if (PG) atm8_fold_pgrad(p, w, m, x, y, valid, q, u);
       __syncthreads();
       atm8_stage_sums<GRAD>(s_red, lane, u.ey, u.fy0, u.fy1, u.fy2, u.cy);
       __syncthreads();
@@ -2577,7 +2614,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       slot_of(gx)[lane] += sum;
     }
   }
-  if (PG) atm8_store_pgrad(u, lane, w.pg3 + b * 4);
+  if (PG) atm8_store_pgrad(p, u, lane, w.pg3 + b * 4);
 }
 
 // Atom sums of the screened one-pass kernel: one work-group per 8-atom group
@@ -2958,14 +2995,18 @@ __global__ __launch_bounds__(256) void k_inputs(const int64_t* numbers, int64_t 
 // three-body work-group partials into dL/d(s6, s8, s10, s9, a1, a2, alp).
 // mode: 0 pair-tile kernel (one partial per 16 x 16 pair tile), 1 one-pass
 // kernel (one per split; tile8 picks the 8 x 8 variant), 2 screened one-pass
-// kernel (one per work-group, all written).
+// kernel (one per work-group, all written). Work-group b of the grid sums
+// every gridDim-th round of 256 partials into out[8 b ..]; more than one are
+// added by k_pgrad_last (384 x 6-60 atoms: 42 us in one work-group, 10 in two
+// launches).
 __global__ __launch_bounds__(256) void k_pgrad_reduce(Inputs in, Work w, int mode,
                                                       int tile8, int64_t per_mol, double* out) {
   __shared__ double red[2 * kWaves];
   const int tid = threadIdx.x;
   const int64_t N = w.N;
+  const int64_t first = (int64_t)blockIdx.x * 256 + tid, step = (int64_t)gridDim.x * 256;
   double a[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t row = tid; row < w.B * N; row += 256) {
+  for (int64_t row = first; row < w.B * N; row += step) {
     const double* g = w.pg2 + row * 5;
     a[0] += g[0];
     a[1] += g[1];
@@ -2973,7 +3014,7 @@ __global__ __launch_bounds__(256) void k_pgrad_reduce(Inputs in, Work w, int mod
     a[4] += g[3];
     a[5] += g[4];
   }
-  for (int64_t q = tid; q < w.B * per_mol; q += 256) {
+  for (int64_t q = first; q < w.B * per_mol; q += step) {
     const int64_t m = q / per_mol;
     const int k = (int)(q - m * per_mol);
     const int n = w.natom[m];
@@ -2990,7 +3031,16 @@ __global__ __launch_bounds__(256) void k_pgrad_reduce(Inputs in, Work w, int mod
   }
   for (int k = 0; k < 7; ++k) {
     const double v = block_sum(a[k], red);
-    if (tid == 0) out[k] = v;
+    if (tid == 0) out[8 * blockIdx.x + k] = v;
+  }
+}
+
+// The sums of `parts` (at most 64) work-groups, one per lane.
+__global__ __launch_bounds__(64) void k_pgrad_last(const double* part, int parts, double* out) {
+  const int lane = threadIdx.x;
+  for (int k = 0; k < 7; ++k) {
+    const double v = wave_sum(lane < parts ? part[8 * lane + k] : 0.0);
+    if (lane == 0) out[k] = v;
   }
 }
 
@@ -3289,8 +3339,19 @@ hipError_t launch_pgrad_reduce(hipStream_t s, const Params& p, const Inputs& in,
   const int64_t per_mol = mode == 1   ? one_pass_splits((int)w.N, tile8)
                           : mode == 2 ? atm8s_blocks_per_mol(w.N)
                                       : nb * (nb + 1) / 2;
-  hipLaunchKernelGGL(k_pgrad_reduce, dim3(1), dim3(256), 0, s, in, w, mode, tile8 ? 1 : 0,
-                     per_mol, out);
+  // (the pair-matrix space is free once the three-body rows are summed; it
+  // holds the sums of up to 64 work-groups where there are more partials than
+  // two rounds of one)
+  const int64_t count = std::max(w.B * w.N, w.B * per_mol);
+  const int64_t parts = std::min<int64_t>((count + 511) / 512, 64);
+  if (parts > 1 && w.B * w.N * w.N >= 8 * parts) {
+    hipLaunchKernelGGL(k_pgrad_reduce, dim3((unsigned)parts), dim3(256), 0, s, in, w, mode,
+                       tile8 ? 1 : 0, per_mol, w.pg);
+    hipLaunchKernelGGL(k_pgrad_last, dim3(1), dim3(64), 0, s, w.pg, (int)parts, out);
+  } else {
+    hipLaunchKernelGGL(k_pgrad_reduce, dim3(1), dim3(256), 0, s, in, w, mode, tile8 ? 1 : 0,
+                       per_mol, out);
+  }
   return hipGetLastError();
 }
 

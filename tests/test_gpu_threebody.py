@@ -78,3 +78,21 @@ def test_items_of_the_screened_kernel(n, cutoff):
     assert (ef - efo).abs().max().item() < 1e-13
     assert (gb - gbo).abs().max().item() < 1e-12
     assert ((pb - pbo).abs() <= 1e-10 * pbo.abs()).all()
+
+
+@pytest.mark.parametrize("batch, n", [(1, 9), (1, 130), (3, 24), (40, 64), (700, 12)])
+def test_parameter_gradients(batch, n):
+    """Logarithms per pair and the sums over several work-groups against the
+    16 x 16 kernel's logarithm per triple; sums of all pairs and triples, to
+    1e-10 of their size."""
+    print(f"[case] parameter gradients {batch} x {n}", flush=True)
+    rng = np.random.default_rng(700 + n)
+    mols = [synth.molecule(rng, int(k), synth.MIX_HCNO, 2.8, (0,))
+            for k in rng.integers(max(2, n // 2), n + 1, size=batch)]
+    dev = [t.cuda() for t in synth.pack(mols, pad_to=n)]
+    par = dict(s8=1.2, a1=0.4, a2=5.0, cutoff_disp3=20.0)
+    res = []
+    for kp in (runtime.KernelParams(**par), runtime.KernelParams(**par, atm16=True)):
+        _, ws = runtime.forward(*dev, kp)
+        res.append(runtime.backward(*dev, kp, ws, params=True)[1])
+    assert ((res[0] - res[1]).abs() <= 1e-10 * res[1].abs()).all()
