@@ -134,6 +134,30 @@ __device__ __forceinline__ double sum_lanes8(double v) {
   return v;
 }
 
+// v plus the value 8, 16 and 32 lanes away, in turn: the sum over the eight
+// lanes of a wave with the same lane & 7, without the LDS crossbar (a rotation
+// by 8 in rows of 16 lanes, then the row and half-wave swaps, which return the
+// even and the odd rows' values). The tiled passes are bound by the latency
+// of a tile (lookups, reductions; 36% of the VALU issue): with this and the next
+// tile's constants in flight 256 x 200 atoms take 48 instead of 56 us
+// (coordination numbers) and 70 instead of 81 (chain).
+template <int ROWS16>
+__device__ __forceinline__ double add_swapped(double v) {
+  const int l = __double2loint(v), h = __double2hiint(v);
+  if (ROWS16) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+  const auto lo = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double sum_stride8(double v) {
+  v += dpp_double<0x128>(v);  // row_ror:8
+  return add_swapped<0>(add_swapped<1>(v));
+}
+
 // Coordination numbers of molecules of up to 256 atoms, each unordered pair
 // once: the counting function and the electronegativity factor are
 // symmetric, so both atoms of a pair get the same terms. One work-group of
@@ -282,40 +306,47 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
   const int nb = (n + 7) >> 3;
   const int tiles = ROWS ? (A < nb ? nb : 0) : nb * (nb + 1) / 2;
   double* f = s_f + (size_t)wv * 2 * n;
+  // (the pair constants of the wave's next tile are loaded during this one;
+  // a block row's two or three tiles per wave gain nothing by that)
+  int bx = 0, by = 0;
+  if (!ROWS) {
+    bx = wv;  // tile wv: by (by + 1) / 2 + bx
+    for (; bx > by; ++by) bx -= by + 1;
+  }
+  auto fetch = [&](int tl, PairConst& c) {
+    const int x = 8 * (ROWS ? min(A, tl) : bx) + tx, y = 8 * (ROWS ? max(A, tl) : by) + ty;
+    if (tl >= tiles || x >= y || y >= n) return false;
+    const int zx = (int)s_at[4 * x + 3], zy = (int)s_at[4 * y + 3];
+    if (zx == 0 || zy == 0) return false;
+    c = pair_const(t, zx, zy);
+    return true;
+  };
+  PairConst pc = {0.0, 0.0, 0.0};
+  bool on = !ROWS && fetch(wv, pc);
   for (int tl = wv; tl < tiles; tl += kCnWaves) {
-    int bx, by;
-    if (ROWS) {
-      bx = min(A, tl);
-      by = max(A, tl);
-    } else {
-      by = (int)((sqrt(8.0 * tl + 1.0) - 1.0) * 0.5);
-      while (by * (by + 1) / 2 > tl) --by;
-      while ((by + 1) * (by + 2) / 2 <= tl) ++by;
-      bx = tl - by * (by + 1) / 2;
-    }
-    const int x = 8 * bx + tx, y = 8 * by + ty;
+    const int x = 8 * (ROWS ? min(A, tl) : bx) + tx, y = 8 * (ROWS ? max(A, tl) : by) + ty;
+    if (!ROWS)
+      for (bx += kCnWaves; bx > by; ++by) bx -= by + 1;
+    PairConst pcn = {0.0, 0.0, 0.0};
+    const bool onn = !ROWS && fetch(tl + kCnWaves, pcn);
+    if (ROWS) on = fetch(tl, pc);
     double v[2] = {0.0, 0.0};  // D4 CN term, EEQ CN term
-    if (x < y && y < n) {
+    if (on) {
       const double* ax = s_at + 4 * x;
       const double* ay = s_at + 4 * y;
-      const int zx = (int)ax[3], zy = (int)ay[3];
-      if (zx != 0 && zy != 0) {
-        const double dx = ax[0] - ay[0], dy = ax[1] - ay[1], dz = ax[2] - ay[2];
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double r = r2 * rsqrt_nt(r2);
-        const PairConst pc = pair_const(t, zx, zy);
-        const double c = erf_count(r, pc.irc);
-        if (r <= p.cutcn) v[0] = pc.enf * c;
-        if (r <= p.cuteeq) v[1] = c;
-      }
+      const double dx = ax[0] - ay[0], dy = ax[1] - ay[1], dz = ax[2] - ay[2];
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      const double r = r2 * rsqrt_nt(r2);
+      const double c = erf_count(r, pc.irc);
+      if (r <= p.cutcn) v[0] = pc.enf * c;
+      if (r <= p.cuteeq) v[1] = c;
     }
+    pc = pcn;
+    on = onn;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const double rs = sum_lanes8(v[c]);  // y atom 8 by + ty
-      double cs = v[c];                    // x atom 8 bx + tx
-      cs += __shfl_xor(cs, 8);
-      cs += __shfl_xor(cs, 16);
-      cs += __shfl_xor(cs, 32);
+      const double cs = sum_stride8(v[c]);  // x atom 8 bx + tx
       if (ROWS) {
         double* e = s_f + ((c * nb + tl) * 2) * 8;
         if (tx == 0) e[ty] = rs;
@@ -2826,55 +2857,60 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_chain_sym(DevTables t, Par
   const int nb = (n + 7) >> 3;
   const int tiles = ROWS ? nb : nb * (nb + 1) / 2;
   double* f = s_f + (size_t)wv * 3 * n;
+  // (the pair constants of the wave's next tile are loaded during this one)
+  int bx = 0, by = 0;
+  if (!ROWS) {
+    bx = wv;  // tile wv: by (by + 1) / 2 + bx
+    for (; bx > by; ++by) bx -= by + 1;
+  }
+  auto fetch = [&](int tl, PairConst& c) {
+    const int x = 8 * (ROWS ? min(A, tl) : bx) + tx, y = 8 * (ROWS ? max(A, tl) : by) + ty;
+    if (tl >= tiles || x >= y || y >= n) return false;
+    const int zx = (int)s_at[kChainAtom * x + 7], zy = (int)s_at[kChainAtom * y + 7];
+    if (zx == 0 || zy == 0) return false;
+    c = pair_const(t, zx, zy);
+    return true;
+  };
+  PairConst pc = {0.0, 0.0, 0.0};
+  bool on = fetch(wv, pc);
   for (int tl = wv; tl < tiles; tl += kChainWaves) {
-    int bx, by;
-    if (ROWS) {
-      bx = min(A, tl);
-      by = max(A, tl);
-    } else {
-      by = (int)((sqrt(8.0 * tl + 1.0) - 1.0) * 0.5);
-      while (by * (by + 1) / 2 > tl) --by;
-      while ((by + 1) * (by + 2) / 2 <= tl) ++by;
-      bx = tl - by * (by + 1) / 2;
-    }
-    const int x = 8 * bx + tx, y = 8 * by + ty;
+    const int x = 8 * (ROWS ? min(A, tl) : bx) + tx, y = 8 * (ROWS ? max(A, tl) : by) + ty;
+    if (!ROWS)
+      for (bx += kChainWaves; bx > by; ++by) bx -= by + 1;
+    PairConst pcn = {0.0, 0.0, 0.0};
+    const bool onn = fetch(tl + kChainWaves, pcn);
     double fc[3] = {0.0, 0.0, 0.0};
-    if (x < y && y < n) {
+    if (on) {
       const double* ax = s_at + kChainAtom * x;
       const double* ay = s_at + kChainAtom * y;
-      const int zx = (int)ax[7], zy = (int)ay[7];
-      if (zx != 0 && zy != 0) {
-        const double dx = ax[0] - ay[0], dy = ax[1] - ay[1], dz = ax[2] - ay[2];
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double ir = rsqrt_nt(r2);
-        const double r = r2 * ir;
-        const PairConst pc = pair_const(t, zx, zy);
-        const double dc = erf_count_dr(r, pc.irc);
-        double coef = 0.0;
-        if (r <= p.cutcn) coef += (ax[3] + ay[3]) * pc.enf * dc;
-        if (eeq) {
-          if (r <= p.cuteeq) coef += (ax[4] + ay[4]) * dc;
-          // d/dr erf(gamma r) / r
-          const double gm = pc.gam;
-          const double dA =
-              ir * fma(2.0 * kInvSqrtPi * gm, exp(-gm * gm * r2), -erf(gm * r) * ir);
-          coef -= (ax[5] * ay[6] + ay[5] * ax[6]) * dA;
-        }
-        coef *= ir;
-        fc[0] = coef * dx;
-        fc[1] = coef * dy;
-        fc[2] = coef * dz;
+      const double dx = ax[0] - ay[0], dy = ax[1] - ay[1], dz = ax[2] - ay[2];
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      const double ir = rsqrt_nt(r2);
+      const double r = r2 * ir;
+      const double dc = erf_count_dr(r, pc.irc);
+      double coef = 0.0;
+      if (r <= p.cutcn) coef += (ax[3] + ay[3]) * pc.enf * dc;
+      if (eeq) {
+        if (r <= p.cuteeq) coef += (ax[4] + ay[4]) * dc;
+        // d/dr erf(gamma r) / r
+        const double gm = pc.gam;
+        const double dA =
+            ir * fma(2.0 * kInvSqrtPi * gm, exp(-gm * gm * r2), -erf(gm * r) * ir);
+        coef -= (ax[5] * ay[6] + ay[5] * ax[6]) * dA;
       }
+      coef *= ir;
+      fc[0] = coef * dx;
+      fc[1] = coef * dy;
+      fc[2] = coef * dz;
     }
+    pc = pcn;
+    on = onn;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       // y atom 8 by + ty: minus the sum over its row's eight lanes
       const double rs = sum_lanes8(fc[c]);
       // x atom 8 bx + tx: the sum over the eight rows
-      double cs = fc[c];
-      cs += __shfl_xor(cs, 8);
-      cs += __shfl_xor(cs, 16);
-      cs += __shfl_xor(cs, 32);
+      const double cs = sum_stride8(fc[c]);
       if (ROWS) {
         double* e = s_f + ((c * nb + tl) * 2) * 8;
         if (tx == 0) e[ty] = rs;
