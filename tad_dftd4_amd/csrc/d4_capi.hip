@@ -286,6 +286,26 @@ int run_front(d4_context* ctx, Call& c) {
   return D4_OK;
 }
 
+// True where both halves of an evaluation run on the caller's stream: the fork
+// and the join cost the host and the second queue more than the shorter half of
+// a small evaluation takes. Consecutive calls (calls waited for one by one) on
+// two streams against one, medians over processes in us: energy of 24 atoms
+// 131 / 88 (148 / 132), of 64 132 / 108 (145 / 151), of 100 125 / 141; energy and
+// forces through autograd of 64 atoms 374 / 256 (390 / 320), of 150, backward
+// alone on one, 369 / 342 (396 / 395); 96 x 10-80 given charges 443 / 323 (459 /
+// 392); fused 32 x 8-41 133 / 100 (141 / 153), 128 x 8-60 120 / 145; 384 x 6-60 and
+// 768 x 6-100 fits even. A captured graph pays no host cost and keeps two.
+// `solve`: the charges are solved for (a long half of its own).
+bool single_stream(const Call& c, bool solve, bool grad) {
+  const int64_t N = c.w.N, pairs = c.w.B * N * N;
+  const bool small = !solve    ? N <= 160 && pairs <= (1 << 20)
+                     : N <= 48 ? pairs <= (1 << 19)
+                               : !grad && N <= 64 && pairs <= (1 << 17);
+  if (!small) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(c.s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // The two halves of an evaluation after the coordination numbers:
 //   companion: weights at q = 0 -> three-body pair factors -> three-body term
 //   call's:    EEQ charges -> weights at q -> two-body term
@@ -324,7 +344,8 @@ int run_split(d4_context* ctx, Call& c, bool eeq, bool energy, bool grad, double
     D4_RUN(D4_SLOT_ATM, d4::launch_atm(c.s, c.p, c.in, c.w, energy, grad), "three-body term");
     return D4_OK;
   }
-  if (c.p.one_stream)
+  const bool one = c.p.one_stream || single_stream(c, eeq && c.in.q_in == nullptr, grad);
+  if (one)
     c.aux.s = c.s;  // the three-body side in order on the caller's stream
   else
     D4_TRY(fork_aux(ctx, c), "fork companion stream");
@@ -344,7 +365,7 @@ int run_split(d4_context* ctx, Call& c, bool eeq, bool energy, bool grad, double
   if (eeq) {
     // energies alone: the charge chain (EEQ, weights, two-body) is the shorter
     // one, so the solve may leave half the CUs to the three-body kernel
-    D4_RUN(D4_SLOT_EEQ, d4::launch_eeq(c.s, ctx->t, c.p, c.in, c.w, !grad && !c.p.one_stream),
+    D4_RUN(D4_SLOT_EEQ, d4::launch_eeq(c.s, ctx->t, c.p, c.in, c.w, !grad && !one),
            "EEQ charges");
     D4_RUN(D4_SLOT_WEIGHTS, d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsTwoBody),
            "reference weights");
@@ -353,7 +374,7 @@ int run_split(d4_context* ctx, Call& c, bool eeq, bool energy, bool grad, double
          "two-body term");
   if (grad)
     D4_RUN(D4_SLOT_ADJOINT, d4::launch_adjoint(c.s, ctx->t, c.p, c.in, c.w), "EEQ adjoint");
-  if (!c.p.one_stream) D4_TRY(join_aux(c), "join companion stream");
+  if (!one) D4_TRY(join_aux(c), "join companion stream");
   return D4_OK;
 }
 
