@@ -269,7 +269,7 @@ int run_cn(d4_context* ctx, Call& c) {
   D4_RUN(D4_SLOT_PREP, enter_sorted(c, false), "spatial order");
   if (c.w.N > d4::kAtm1MaxN) {  // (smaller batches: one launch does all three)
     D4_RUN(D4_SLOT_PREP, d4::launch_prep(c.s, c.in, c.w), "prep");
-    if (!c.p.d4s) D4_RUN(D4_SLOT_PREP, d4::launch_zslots(c.s, c.in, c.w), "element slots");
+    D4_RUN(D4_SLOT_PREP, d4::launch_zslots(c.s, c.in, c.w), "element slots");
   }
   D4_RUN(D4_SLOT_CN, d4::launch_cn(c.s, ctx->t, c.p, c.in, c.w), "coordination numbers");
   return D4_OK;
@@ -281,7 +281,7 @@ int run_front(d4_context* ctx, Call& c) {
   int rc = run_cn(ctx, c);
   if (rc != D4_OK) return rc;
   D4_RUN(D4_SLOT_EEQ, d4::launch_eeq(c.s, ctx->t, c.p, c.in, c.w, false), "EEQ charges");
-  D4_RUN(D4_SLOT_WEIGHTS, d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsBoth),
+  D4_RUN(D4_SLOT_WEIGHTS, d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsBoth, false),
          "reference weights");
   return D4_OK;
 }
@@ -314,43 +314,24 @@ bool single_stream(const Call& c, bool solve, bool grad) {
 // EEQ adjoint (which needs only dL/dq of the two-body term) also runs before
 // the join.
 int run_split(d4_context* ctx, Call& c, bool eeq, bool energy, bool grad, double* g_out) {
-  // D4S forms the pair weights inside the pair pass. Up to 160 atoms one fused
-  // pass on the call's stream, which forms them once, is faster (1024 x 20-120
-  // atoms: 1.45 against 1.64 ms with gradients); for longer molecules the
-  // three-body term dominates and the split below, which forms the q = 0 and
-  // the q weights in separate passes but runs the three-body side beside the
-  // charges, wins (256 x 8-200 atoms: 1.18 against 1.34 ms). Both give the
-  // same bits.
-  constexpr int64_t kD4sFusedMaxN = 160;
-  if (c.p.d4s && c.w.N <= kD4sFusedMaxN) {
+  if (c.p.one_stream || single_stream(c, eeq && c.in.q_in == nullptr, grad)) {
+    // in order: one launch forms the weights, one the pairs of both halves
     if (eeq) {
       D4_RUN(D4_SLOT_EEQ, d4::launch_eeq(c.s, ctx->t, c.p, c.in, c.w, false), "EEQ charges");
-      D4_RUN(D4_SLOT_WEIGHTS, d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsBoth),
+      D4_RUN(D4_SLOT_WEIGHTS,
+             d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsBoth, true),
              "reference weights");
     }
-    D4_RUN(D4_SLOT_PAIRS, d4::launch_pairs(c.s, ctx->t, c.p, c.in, c.w, grad, g_out, d4::kPairsBoth),
-           "pair pass");
-    // the three-body term and the EEQ adjoint both need only the pair pass
-    if (grad && !c.p.one_stream) {
-      D4_TRY(fork_aux(ctx, c), "fork companion stream");
-      D4_RUN_AUX(D4_SLOT_ATM, d4::launch_atm(c.aux.s, c.p, c.in, c.w, energy, grad),
-                 "three-body term");
-      D4_RUN(D4_SLOT_ADJOINT, d4::launch_adjoint(c.s, ctx->t, c.p, c.in, c.w), "EEQ adjoint");
-      D4_TRY(join_aux(c), "join companion stream");
-      return D4_OK;
-    }
+    D4_RUN(D4_SLOT_PAIRS,
+           d4::launch_pairs(c.s, ctx->t, c.p, c.in, c.w, grad, g_out, d4::kPairsBoth), "pair pass");
+    D4_RUN(D4_SLOT_ATM, d4::launch_atm(c.s, c.p, c.in, c.w, energy, grad), "three-body term");
     if (grad)
       D4_RUN(D4_SLOT_ADJOINT, d4::launch_adjoint(c.s, ctx->t, c.p, c.in, c.w), "EEQ adjoint");
-    D4_RUN(D4_SLOT_ATM, d4::launch_atm(c.s, c.p, c.in, c.w, energy, grad), "three-body term");
     return D4_OK;
   }
-  const bool one = c.p.one_stream || single_stream(c, eeq && c.in.q_in == nullptr, grad);
-  if (one)
-    c.aux.s = c.s;  // the three-body side in order on the caller's stream
-  else
-    D4_TRY(fork_aux(ctx, c), "fork companion stream");
+  D4_TRY(fork_aux(ctx, c), "fork companion stream");
   if (eeq) {
-    D4_RUN_AUX(D4_SLOT_WEIGHTS, d4::launch_weights(c.aux.s, ctx->t, c.p, c.w, c.in, d4::kPairsAtm),
+    D4_RUN_AUX(D4_SLOT_WEIGHTS, d4::launch_weights(c.aux.s, ctx->t, c.p, c.w, c.in, d4::kPairsAtm, true),
                "reference weights (q = 0)");
   }
   D4_RUN_AUX(D4_SLOT_PAIRS,
@@ -365,16 +346,15 @@ int run_split(d4_context* ctx, Call& c, bool eeq, bool energy, bool grad, double
   if (eeq) {
     // energies alone: the charge chain (EEQ, weights, two-body) is the shorter
     // one, so the solve may leave half the CUs to the three-body kernel
-    D4_RUN(D4_SLOT_EEQ, d4::launch_eeq(c.s, ctx->t, c.p, c.in, c.w, !grad && !one),
-           "EEQ charges");
-    D4_RUN(D4_SLOT_WEIGHTS, d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsTwoBody),
+    D4_RUN(D4_SLOT_EEQ, d4::launch_eeq(c.s, ctx->t, c.p, c.in, c.w, !grad), "EEQ charges");
+    D4_RUN(D4_SLOT_WEIGHTS, d4::launch_weights(c.s, ctx->t, c.p, c.w, c.in, d4::kPairsTwoBody, true),
            "reference weights");
   }
   D4_RUN(D4_SLOT_PAIRS, d4::launch_pairs(c.s, ctx->t, c.p, c.in, c.w, grad, g_out, d4::kPairsTwoBody),
          "two-body term");
   if (grad)
     D4_RUN(D4_SLOT_ADJOINT, d4::launch_adjoint(c.s, ctx->t, c.p, c.in, c.w), "EEQ adjoint");
-  if (!one) D4_TRY(join_aux(c), "join companion stream");
+  D4_TRY(join_aux(c), "join companion stream");
   return D4_OK;
 }
 

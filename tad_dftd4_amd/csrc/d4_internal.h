@@ -352,8 +352,9 @@ hipError_t launch_eeq(hipStream_t s, const DevTables& t, const Params& p,
 constexpr int kPairsBoth = 0;
 constexpr int kPairsAtm = 1;
 constexpr int kPairsTwoBody = 2;
+// `cv`: with the contraction vectors of the part (what the pair passes read)
 hipError_t launch_weights(hipStream_t s, const DevTables& t, const Params& p,
-                          const Work& w, const Inputs& in, int part);
+                          const Work& w, const Inputs& in, int part, bool cv);
 // Element slots of every molecule (after launch_prep), and the C6 contraction
 // vectors of one part (after its weights; D4 model only).
 hipError_t launch_zslots(hipStream_t s, const Inputs& in, const Work& w);

@@ -191,7 +191,7 @@ __device__ __forceinline__ double tile_row_sum(const double* sums, int nb, int A
 // molecule; it takes the tiles of block row A (each pair twice over the
 // molecule) and forms the same sums in the same order, so the results are the
 // same bits.
-template <bool ZS, bool ROWS>
+template <bool ROWS>
 __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p, Inputs in,
                                                             Work w) {
   extern __shared__ double s_dyn[];  // [n][4] x, y, z, Z; [kCnWaves][2][n] sums
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
       if (zi != 0) last = (int)i;
       if (zi < 0 || zi >= kMaxZ) bad = 1;
     }
-    if (ZS && lead)
+    if (lead)
       for (int e = tid; e < kMaxZ; e += NT) s_present[e] = 0;
     last = wave_max(last);
     bad = wave_or(bad);
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
       w.natom[m] = n;
       w.status[m] = bad ? kStatusBadZ : 0;
     }
-    if (ZS && lead) {
+    if (lead) {
       // element slots: the molecule's distinct elements in increasing Z
       for (int i = tid; i < n; i += NT) {
         const int64_t zi = z[i];
@@ -394,12 +394,12 @@ __global__ __launch_bounds__(64 * kCnWaves) void k_cn_sym(DevTables t, Params p,
 
 // part kPairsAtm writes the q = 0 weights (gw0, dgw0), kPairsTwoBody those at
 // the EEQ charges (gw, dgw, dgwq), kPairsBoth all of them.
-// CV (D4, part q = 0 or part q alone): also the atom's C6 contraction
-// vectors, for each element slot e of its molecule v[a] = sum_b
-// RC6[Z_e][Z_j][a][b] gw_j[b] (a < 7; entry 7 is zero) from the weights just
-// formed (lane a walks the slots), which the pair pass reads in place of the
-// per-pair 7 x 7 reference blocks.
-template <bool CV>
+// CV: also the atom's C6 contraction vectors of the part, for each element slot
+// e of its molecule v[a] = sum_b RC6[Z_e][Z_j][a][b] gw_j[b] (a < 7; entry 7 is
+// zero) from the weights just formed (lane a walks the slots), which the pair
+// pass reads in place of the per-pair 7 x 7 reference blocks. D4S weights depend on the partner through its element alone
+// (model/d4s.py:196), so slot e takes those for a partner of element Z_e.
+template <bool CV, bool S>
 __global__ __launch_bounds__(256) void k_weights(DevTables t, Params p, Work w,
                                                  Inputs in, int part) {
   const bool atm = part != kPairsTwoBody, two = part != kPairsAtm;
@@ -422,10 +422,9 @@ __global__ __launch_bounds__(256) void k_weights(DevTables t, Params p, Work w,
   if (used && two) zeta_dzeta(p.ga, gam, qref, q + zeff, zq, dzq);
   if (used && atm) z0 = zeta_fn(p.ga, gam, qref, zeff);
   const int64_t o = row * kRefStride + a;
-  if (p.d4s) {
-    // D4S: the Gaussian part depends on the partner atom and is formed in
-    // the pair pass; keep the charge scaling zeta(q), zeta(0), dzeta/dq of
-    // every reference (model/d4s.py:240-263)
+  if (S) {
+    // D4S: the Gaussian part depends on the partner's element; keep the charge
+    // scaling zeta(q), zeta(0), dzeta/dq of every reference (model/d4s.py:240-263)
     if (two) {
       w.gw[o] = zq;
       w.dgw[o] = 0.0;
@@ -434,6 +433,38 @@ __global__ __launch_bounds__(256) void k_weights(DevTables t, Params p, Work w,
     if (atm) {
       w.gw0[o] = z0;
       w.dgw0[o] = 0.0;
+    }
+    const int nz = w.nzs[m];
+    if (!CV || z == 0 || nz <= 0) return;
+    const double refcn = used ? t.refcn[z * kMaxRef + a] : 0.0;
+    const double d2 = (cn - refcn) * (cn - refcn);
+    const bool three = used && t.ngw[z * kMaxRef + a] == 3;
+    const bool top = used && refcn == t.maxcn[z];
+    const int base = (threadIdx.x & 63) & ~7;
+    const int64_t out = row * kZSlots * 8 + a;
+    for (int e = 0; e < nz; ++e) {
+      const int ze = w.zlist[m * kZSlots + e];
+      double ga = 0.0;  // as in pair_gauss
+      if (used) {
+        const double tmp = exp(-d2 * t.wfpair[z * kMaxZ + ze]);
+        ga = three ? tmp + tmp * tmp + tmp * tmp * tmp : tmp;
+      }
+      const double norm = sum_lanes8(ga);
+      ga = norm > 0.0 ? ga / norm : (top ? 1.0 : 0.0);
+      double rc[kMaxRef];
+#pragma unroll
+      for (int b = 0; b < kMaxRef; ++b)
+        rc[b] = a < kMaxRef ? t.rc6[((size_t)ze * kMaxZ + z) * kRc6Block + a * kMaxRef + b] : 0.0;
+      auto contract = [&](double gsel) {
+        double gg[kMaxRef], v = 0.0;
+#pragma unroll
+        for (int b = 0; b < kMaxRef; ++b) gg[b] = __shfl(gsel, base + b, 64);
+#pragma unroll
+        for (int b = 0; b < kMaxRef; ++b) v += rc[b] * gg[b];
+        return v;
+      };
+      if (atm) w.cv0[out + e * 8] = contract(z0 * ga);
+      if (two) w.cv[out + e * 8] = contract(zq * ga);
     }
     return;
   }
@@ -477,25 +508,28 @@ __global__ __launch_bounds__(256) void k_weights(DevTables t, Params p, Work w,
     w.dgw0[o] = z0 * dg;
   }
   if (CV) {
-    // every lane of the atom's 8-lane group gathers the atom's weights of
-    // the part (uniform per group: the group's lanes are all active here)
-    const double gsel = atm ? z0 * g : zq * g;
+    // every lane of the atom's 8-lane group gathers the atom's weights
+    // (uniform per group: the group's lanes are all active here)
     const int base = (threadIdx.x & 63) & ~7;
-    double gg[kMaxRef];
-#pragma unroll
-    for (int b = 0; b < kMaxRef; ++b) gg[b] = __shfl(gsel, base + b, 64);
     const int nz = w.nzs[m];
-    if (z == 0 || nz <= 0) return;
-    double* out = (atm ? w.cv0 : w.cv) + row * kZSlots * 8 + a;
-    for (int e = 0; e < nz; ++e) {
-      double v = 0.0;
-      if (a < kMaxRef) {
-        const double* blk =
-            t.rc6 + ((size_t)w.zlist[m * kZSlots + e] * kMaxZ + z) * kRc6Block + a * kMaxRef;
+    for (int half = 0; half < 2; ++half) {
+      if (!(half == 0 ? atm : two)) continue;
+      const double gsel = half == 0 ? z0 * g : zq * g;
+      double gg[kMaxRef];
 #pragma unroll
-        for (int b = 0; b < kMaxRef; ++b) v += blk[b] * gg[b];
+      for (int b = 0; b < kMaxRef; ++b) gg[b] = __shfl(gsel, base + b, 64);
+      if (z == 0 || nz <= 0) continue;
+      double* out = (half == 0 ? w.cv0 : w.cv) + row * kZSlots * 8 + a;
+      for (int e = 0; e < nz; ++e) {
+        double v = 0.0;
+        if (a < kMaxRef) {
+          const double* blk =
+              t.rc6 + ((size_t)w.zlist[m * kZSlots + e] * kMaxZ + z) * kRc6Block + a * kMaxRef;
+#pragma unroll
+          for (int b = 0; b < kMaxRef; ++b) v += blk[b] * gg[b];
+        }
+        out[e * 8] = v;
       }
-      out[e * 8] = v;
     }
   }
 }
@@ -560,11 +594,14 @@ __device__ __forceinline__ void pair_gauss(const DevTables& t, int z, int nr, do
 // --------------------------------------------------------------------------
 // pair pass: C6(q) and C6(0) contraction with the reference-C6 table, the
 // rational-damped two-body term, the ATM pair factors; with GRAD also the
-// two-body gradient pieces. With S (D4S model) the weights of both atoms are
-// formed per pair from the charge scaling that k_weights left and the pair's
-// Gaussian weights. PART selects the three-body pair factors (C6 at q = 0:
-// independent of the charges), the two-body term (C6 at the EEQ charges) or
-// both in one pass.
+// two-body gradient pieces. With S (D4S model) the row's Gaussian weights for
+// partners of every element of the molecule are formed once, a lane per
+// element, and kept in LDS (the partner's are in its contraction vectors);
+// molecules of more than kZSlots elements form both per pair. 256 x 20-120 atoms
+// with gradients: 190 us with the weights per pair, 55 + 55 for the two parts.
+// PART selects the three-body pair factors (C6 at q = 0: independent of the
+// charges), the two-body term (C6 at the EEQ charges) or, where both run on one
+// stream anyway, both in one pass.
 // --------------------------------------------------------------------------
 
 constexpr int kPartBoth = 0;
@@ -648,15 +685,16 @@ __device__ __forceinline__ void pair_eval(const DevTables& t, const Params& p, c
                                           int zj, double xj, double yj, double zzj, double r4j,
                                           double cnj, double gj, const double* gwjp,
                                           const double* gw0jp, const double* vj,
-                                          PairSums& acc, double& tf, double& pf, double& pk) {
+                                          const double* v0j, const double* gi, PairSums& acc, double& tf, double& pf, double& pk) {
   constexpr bool ATMF = PART != kPartE2, E2 = PART != kPartAtm;
   const double dx = A.x - xj, dy = A.y - yj, dz = A.zc - zzj;
   const double r2 = dx * dx + dy * dy + dz * dz;
   const double ir = rsqrt_nt(r2);
   const double r = r2 * ir;
-  // D4 split passes of molecules with element slots: the partner's weights
-  // come precontracted with the reference C6 block of this atom's element
-  const bool pv = !S && PART != kPartBoth && vj != nullptr;
+  // molecules with element slots: the partner's weights come precontracted
+  // with the reference C6 block of this atom's element (D4S: and this atom's
+  // Gaussian weights for the partner's element, then their derivatives, in gi)
+  const bool pv = (E2 ? vj : v0j) != nullptr;
   double gwj[kMaxRef], gw0j[kMaxRef];
 #pragma unroll
   for (int b = 0; b < kMaxRef; ++b) {
@@ -667,7 +705,7 @@ __device__ __forceinline__ void pair_eval(const DevTables& t, const Params& p, c
   // partner m use wf(Z_n, Z_m) (model/d4s.py:196). The weights of atom i
   // are zeta_i[a] g[a] (A.gw, A.gw0, A.dgwq hold zeta).
   double g[kMaxRef], dg[kMaxRef];
-  if (S) {
+  if (S && !pv) {
     pair_gauss<GRAD>(t, A.z, A.nr, A.cn, t.wfpair[A.z * kMaxZ + zj], g, dg);
     double gjw[kMaxRef];
     pair_gauss<false>(t, zj, t.nref[zj], cnj, t.wfpair[zj * kMaxZ + A.z], gjw, nullptr);
@@ -682,18 +720,36 @@ __device__ __forceinline__ void pair_eval(const DevTables& t, const Params& p, c
   if (pv) {
     // v[a] = sum_b RC6[Z_i][Z_j][a][b] gw_j[b], summed as below; the weights
     // of reference systems a >= nref are zero, so the sums match bit for bit
-    const double2* v2 = reinterpret_cast<const double2*>(vj);
-    const double2 v01 = v2[0], v23 = v2[1], v45 = v2[2], v67 = v2[3];
-    const double v[kMaxRef] = {v01.x, v01.y, v23.x, v23.y, v45.x, v45.y, v67.x};
+    double v[kMaxRef] = {}, v0[kMaxRef] = {};
+    auto load = [](const double* p8, double* to) {
+      const double2* p2 = reinterpret_cast<const double2*>(p8);
+      const double2 a01 = p2[0], a23 = p2[1], a45 = p2[2], a67 = p2[3];
+      to[0] = a01.x;
+      to[1] = a01.y;
+      to[2] = a23.x;
+      to[3] = a23.y;
+      to[4] = a45.x;
+      to[5] = a45.y;
+      to[6] = a67.x;
+    };
+    if (E2) load(vj, v);
+    if (ATMF) load(v0j, v0);
 #pragma unroll
     for (int a = 0; a < kMaxRef; ++a) {
-      if (E2) c6 += A.gw[a] * v[a];
-      if (ATMF) c60 += A.gw0[a] * v[a];
-      if (GRAD && E2) {
-        dc6cn += A.dgw[a] * v[a];
-        dc6q += A.dgwq[a] * v[a];
+      // D4S: A holds zeta, gi the Gaussian weights and their derivatives
+      const double gs = S ? gi[a] : 1.0, ds = (S && GRAD) ? gi[kMaxRef + a] : 0.0;
+      if (E2) {
+        const double gv = S ? gs * v[a] : v[a];
+        c6 += A.gw[a] * gv;
+        if (GRAD) {
+          dc6cn += S ? A.gw[a] * (ds * v[a]) : A.dgw[a] * v[a];
+          dc6q += A.dgwq[a] * gv;
+        }
       }
-      if (GRAD && ATMF) dc60cn += A.dgw0[a] * v[a];
+      if (ATMF) {
+        c60 += A.gw0[a] * (S ? gs * v0[a] : v0[a]);
+        if (GRAD) dc60cn += S ? A.gw0[a] * (ds * v0[a]) : A.dgw0[a] * v0[a];
+      }
     }
   }
 #pragma unroll
@@ -837,8 +893,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   PairAtom A;
   load_pair_atom<GRAD, S, PART>(t, w, in, row, zi, R, i, A);
   PairSums acc;
-  const int slot = (!S && PART != kPartBoth) ? w.zslot[m * kMaxZ + zi] : -1;
-  const double* cvp = PART == kPartAtm ? w.cv0 : w.cv;
+  const int32_t* zslot = w.zslot + m * kMaxZ;
+  const int slot = zslot[zi];
+  // D4S: the row's Gaussian weights (and derivatives) by the partner's slot; an
+  // odd stride in doubles keeps lanes of different slots on different banks
+  constexpr int GS = GRAD ? 2 * kMaxRef + 1 : kMaxRef;
+  __shared__ double s_g[S ? 64 / RL * kZSlots * GS : 1];
+  double* gis = s_g + threadIdx.x / RL * kZSlots * GS;
+  if (S && slot >= 0) {
+    for (int e = lane; e < w.nzs[m]; e += RL) {
+      double g[kMaxRef], dg[kMaxRef];
+      pair_gauss<GRAD>(t, zi, A.nr, A.cn, t.wfpair[zi * kMaxZ + w.zlist[m * kZSlots + e]], g, dg);
+#pragma unroll
+      for (int a = 0; a < kMaxRef; ++a) {
+        gis[e * GS + a] = g[a];
+        if (GRAD) gis[e * GS + kMaxRef + a] = dg[a];
+      }
+    }
+    // the row's lanes are in one wave, which keeps its LDS accesses in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
   // the partner's Z is loaded one iteration ahead: the table reads of a pair
   // (reference C6 block, r4r2) depend on it
   int znext = lane < n ? (int)Z[lane] : 0;
@@ -858,10 +933,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const double cnj = S ? w.cn[rj] : 0.0;
     const double gj = (GRAD && E2) ? (in.gE ? in.gE[rj] : 1.0) : 0.0;
     double tf, pf, pk;
-    const double* vj = slot >= 0 ? cvp + (rj * kZSlots + slot) * 8 : nullptr;
+    const int64_t at = (rj * kZSlots + slot) * 8;
+    const double* vj = slot >= 0 ? w.cv + at : nullptr;
+    const double* v0j = slot >= 0 ? w.cv0 + at : nullptr;
+    const double* gi = S && slot >= 0 ? gis + zslot[zj] * GS : nullptr;
     pair_eval<GRAD, PG, S, PART>(t, p, A, zj, R[3 * j], R[3 * j + 1], R[3 * j + 2], r4j, cnj,
-                                 gj, gw + rj * kRefStride, gw0 + rj * kRefStride, vj, acc, tf,
-                                 pf, pk);
+                                 gj, gw + rj * kRefStride, gw0 + rj * kRefStride, vj, v0j, gi, acc,
+                                 tf, pf, pk);
     if (ATMF) {
       ptr[j] = tf;
       ppr[j] = pf;
@@ -3133,16 +3211,12 @@ hipError_t launch_cn(hipStream_t s, const DevTables& t, const Params& p,
     const size_t nb = (size_t)(w.N + 7) / 8;
     const size_t shmem = sizeof(double) * (rows ? 4 * (size_t)w.N + 32 * nb + 128
                                                 : (size_t)(4 + 2 * kCnWaves) * (size_t)w.N);
-    // (also the extents, the Z check and, for D4, the element slots)
+    // (also the extents, the Z check and the element slots)
     const dim3 g((unsigned)(rows ? w.B * (int64_t)nb : w.B)), blk(64 * kCnWaves);
-    if (p.d4s && rows)
-      hipLaunchKernelGGL((k_cn_sym<false, true>), g, blk, shmem, s, t, p, in, w);
-    else if (p.d4s)
-      hipLaunchKernelGGL((k_cn_sym<false, false>), g, blk, shmem, s, t, p, in, w);
-    else if (rows)
-      hipLaunchKernelGGL((k_cn_sym<true, true>), g, blk, shmem, s, t, p, in, w);
+    if (rows)
+      hipLaunchKernelGGL(k_cn_sym<true>, g, blk, shmem, s, t, p, in, w);
     else
-      hipLaunchKernelGGL((k_cn_sym<true, false>), g, blk, shmem, s, t, p, in, w);
+      hipLaunchKernelGGL(k_cn_sym<false>, g, blk, shmem, s, t, p, in, w);
     return hipGetLastError();
   }
   D4_LAUNCH_ROWS((k_cn<16>), (k_cn<32>), (k_cn<64>), s, p, w, t, p, in, w);
@@ -3155,12 +3229,14 @@ hipError_t launch_zslots(hipStream_t s, const Inputs& in, const Work& w) {
 }
 
 hipError_t launch_weights(hipStream_t s, const DevTables& t, const Params& p,
-                          const Work& w, const Inputs& in, int part) {
+                          const Work& w, const Inputs& in, int part, bool cv) {
   const unsigned grid = (unsigned)((w.B * w.N * 8 + 255) / 256);
-  if (part != kPairsBoth && !p.d4s)  // with the contraction vectors of the part
-    hipLaunchKernelGGL(k_weights<true>, dim3(grid), dim3(256), 0, s, t, p, w, in, part);
+  if (p.d4s)
+    hipLaunchKernelGGL((k_weights<true, true>), dim3(grid), dim3(256), 0, s, t, p, w, in, part);
+  else if (cv)
+    hipLaunchKernelGGL((k_weights<true, false>), dim3(grid), dim3(256), 0, s, t, p, w, in, part);
   else
-    hipLaunchKernelGGL(k_weights<false>, dim3(grid), dim3(256), 0, s, t, p, w, in, part);
+    hipLaunchKernelGGL((k_weights<false, false>), dim3(grid), dim3(256), 0, s, t, p, w, in, part);
   return hipGetLastError();
 }
 
@@ -3170,7 +3246,8 @@ void launch_pairs_model(hipStream_t s, const DevTables& t, const Params& p, cons
   // the two-body pass runs beside the three-body kernel: one-wave
   // work-groups take a SIMD as soon as one of its three-body waves ends
   // (a four-wave group needs four such SIMDs of one CU at once)
-  constexpr int blk = PART == kPartE2 ? 64 : 256;
+  // (D4S: also one wave, for the row weights in LDS)
+  constexpr int blk = PART == kPartE2 || S ? 64 : 256;
   if (grad && p.pgrad)
     D4_LAUNCH_ROWS_B(blk, (k_pairs<true, true, S, 16, PART>), (k_pairs<true, true, S, 32, PART>),
                      (k_pairs<true, true, S, 64, PART>), s, p, w, t, p, in, w, grad_out);
