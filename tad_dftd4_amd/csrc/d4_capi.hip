@@ -669,7 +669,7 @@ int d4_properties(d4_context* ctx, void* stream, int64_t nbatch, int64_t natoms,
     // C6 is staged in the (unused here) three-body gradient pair array
     if (c6_out || alpha_out)
       D4_TRY(d4::launch_properties(c.s, ctx->t, c.in, c.w, c6_out ? c.w.pg : nullptr,
-                                   alpha_out ? c.w.sE : nullptr),
+                                   alpha_out ? c.w.sE : nullptr, nullptr, nullptr),
              "properties");
     if (c6_out) D4_TRY(d4::launch_scatter_pairs(c.s, c.w, c.w.pg, c6_out), "scatter C6");
     D4_TRY(scatter_atoms(c, c.w.sE, alpha_out, 1), "scatter polarisabilities");
@@ -677,9 +677,11 @@ int d4_properties(d4_context* ctx, void* stream, int64_t nbatch, int64_t natoms,
     D4_TRY(scatter_atoms(c, c.w.cn, cn_out, 1), "scatter coordination numbers");
     return D4_OK;
   }
-  if (c6_out || alpha_out)
-    D4_TRY(d4::launch_properties(c.s, ctx->t, c.in, c.w, c6_out, alpha_out),
+  if (c6_out || alpha_out) {
+    D4_TRY(d4::launch_properties(c.s, ctx->t, c.in, c.w, c6_out, alpha_out, q_out, cn_out),
            "properties");
+    return D4_OK;
+  }
   if (q_out) D4_TRY(d4::launch_copy(c.s, c.w.q, q_out, nbatch * natoms), "copy charges");
   if (cn_out)
     D4_TRY(d4::launch_copy(c.s, c.w.cn, cn_out, nbatch * natoms), "copy coordination numbers");

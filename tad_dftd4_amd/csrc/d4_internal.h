@@ -370,9 +370,10 @@ hipError_t launch_adjoint(hipStream_t s, const DevTables& t, const Params& p,
                           const Inputs& in, const Work& w);
 hipError_t launch_chain(hipStream_t s, const DevTables& t, const Params& p,
                         const Inputs& in, const Work& w, double* grad_out);
-hipError_t launch_properties(hipStream_t s, const DevTables& t,
-                             const Inputs& in, const Work& w, double* c6_out,
-                             double* alpha_out);
+// (q_out, cn_out: optional copies of the charges and coordination numbers)
+hipError_t launch_properties(hipStream_t s, const DevTables& t, const Inputs& in,
+                             const Work& w, double* c6_out, double* alpha_out, double* q_out,
+                             double* cn_out);
 hipError_t launch_copy(hipStream_t s, const double* src, double* dst, int64_t count);
 // Read-back of inputs into pinned host memory: bad = 1 if an atomic number lies
 // outside 0..kMaxZ - 1, values[k] = scalar k (kind 0: double, 1: float).

@@ -3028,8 +3028,8 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_chain_sym(DevTables t, Par
 // --------------------------------------------------------------------------
 
 __global__ __launch_bounds__(256) void k_properties(DevTables t, Inputs in, Work w,
-                                                    double* c6_out,
-                                                    double* alpha_out) {
+                                                    double* c6_out, double* alpha_out,
+                                                    double* q_out, double* cn_out) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
   if (row >= w.B * w.N) return;
@@ -3060,6 +3060,8 @@ __global__ __launch_bounds__(256) void k_properties(DevTables t, Inputs in, Work
       c6_out[row * N + j] = c6;
     }
   }
+  if (q_out && lane == 0) q_out[row] = w.q[row];
+  if (cn_out && lane == 0) cn_out[row] = w.cn[row];
   if (alpha_out && lane == 0) {
     double al = 0.0;
     if (zi != 0) {
@@ -3437,9 +3439,10 @@ hipError_t launch_chain(hipStream_t s, const DevTables& t, const Params& p,
 }
 
 hipError_t launch_properties(hipStream_t s, const DevTables& t, const Inputs& in,
-                             const Work& w, double* c6_out, double* alpha_out) {
+                             const Work& w, double* c6_out, double* alpha_out, double* q_out,
+                             double* cn_out) {
   hipLaunchKernelGGL(k_properties, dim3(rows_grid(w)), dim3(256), 0, s, t, in, w,
-                     c6_out, alpha_out);
+                     c6_out, alpha_out, q_out, cn_out);
   return hipGetLastError();
 }
 
