@@ -2161,9 +2161,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   static_assert(NA * 64 <= T8 * kAtm8Row<GRAD>, "s_red2");
   extern __shared__ double s_acc[];             // [NA][N] atom sums of this split
 
+  // block b runs on XCD b mod 8: the splits of a molecule go round, and so does
+  // the XCD of its first one (with S a multiple of 8 the molecules of few
+  // splits would all run on the first XCDs: 500 x 30-60 atoms padded to 126
+  // with one of 126 365 us, so 240)
   const int64_t b = blockIdx.x, m = b / S;
   if (m >= nblocks) return;  // nblocks: the number of molecules
-  const int s = (int)(b - m * S);
+  const int64_t turn = b - m * S - m % S;
+  const int s = (int)(turn < 0 ? turn + S : turn);
   const int64_t N = w.N;
   const int n = w.natom[m];
   const int Sm = atm8_splits(n);  // this molecule's split count (S is the batch maximum)
