@@ -303,7 +303,11 @@ bool single_stream(const Call& c, bool solve, bool grad) {
                                : !grad && N <= 64 && pairs <= (1 << 17);
   if (!small) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(c.s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c.s, &st) != hipSuccess) {
+    (void)hipGetLastError();  // the launches after this report their own errors
+    return false;
+  }
+  return st == hipStreamCaptureStatusNone;
 }
 
 // The two halves of an evaluation after the coordination numbers:

@@ -222,10 +222,6 @@ __host__ __device__ inline int atm1_splits(int n) {
   const int s = (int)((work + 262143) / 262144);  // about one 64-atom molecule each
   return tiles < 1 ? 1 : (s < 1 ? 1 : (s > tiles ? tiles : s));
 }
-__host__ __device__ inline int one_pass_split_max(int n) {
-  const int a = atm1_splits(n), b = atm8_splits(n);
-  return a > b ? a : b;
-}
 
 // Small molecules take the one-pass three-body kernel.
 inline bool one_pass(const Params& p, const Work& w) {
@@ -305,8 +301,8 @@ inline size_t layout(int64_t B, int64_t N, char* base, Work* w) {
   v.gsph8 = (double*)take(32 * size_t(B) * size_t(n_groups8(N)));
   v.wix = (int64_t*)take(8 * size_t(B) * size_t(atm8s_table_len(N)));
   // (the pair tiles and the screened kernel, which use pg, ph and pe, do not
-  // run with the one-pass kernels; one_pass_split_max(N) * kAtm1Acc * N <=
-  // 3 N^2 or 48 doubles, at most the stride of pg)
+  // run with the one-pass kernels, whose splits times kAtm1Acc * N are at
+  // most 3 N^2 or 48 doubles, the stride of pg)
   v.apart = v.pg;
   v.rt4 = (double*)take(8 * bn);
   v.zslot = (int32_t*)take(4 * size_t(B) * kMaxZ);
