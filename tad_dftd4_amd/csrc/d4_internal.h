@@ -158,9 +158,29 @@ __host__ __device__ inline int atm8_chunks(int nb) {
   return nw * (nb + kAtm8TileCost) + (M > 1 ? (M - 1) * M * (M + 1) / 6 : 0) +
          pairs * kAtm8TileCost;
 }
-__host__ __device__ inline int atm8_splits(int n) {
+__host__ __device__ inline int atm8_splits(int n) {  // (a molecule without atoms: none)
+  if (n < 1) return 0;
   const int s = (n * n + 249) / 250, cap = 3 * n / 5;
   return cap < 1 ? 1 : (s > cap ? cap : s);
+}
+// Where place `pos` of the chunk list lies: place `off` of tile t, a pair tile
+// (bx, by) from t = ceil(nb / 2) on. pos < atm8_chunks(nb), so nb > 0.
+struct Atm8Start {
+  int t, bx, by, off;
+};
+__host__ __device__ inline Atm8Start atm8_seek(int nb, int pos) {
+  const int nw = (nb + 1) / 2, wlen = nb + kAtm8TileCost;
+  if (pos < nw * wlen) return {pos / wlen, 0, 1, pos % wlen};
+  int t = nw, by = 1, off = pos - nw * wlen;
+  int len = nb - 2 + kAtm8TileCost;  // of the tiles (., by), by <= nb - 2
+  while (off >= by * len) {
+    off -= by * len;
+    t += by;
+    ++by;
+    --len;
+  }
+  const int bx = off / len;
+  return {t + bx, bx, by, off - bx * len};
 }
 
 // Screened one-pass three-body kernel (large systems, atoms in spatial

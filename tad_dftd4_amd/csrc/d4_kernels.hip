@@ -2172,7 +2172,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const int64_t N = w.N;
   const int n = w.natom[m];
   const int Sm = atm8_splits(n);  // this molecule's split count (S is the batch maximum)
-  if (s >= Sm) return;
+  if (s >= Sm) return;  // (every split of a molecule without atoms)
   const int nb = (n + T8 - 1) / T8;
   const int nw = (nb + 1) / 2;  // W-tiles, then the pair tiles bx < by <= nb - 2
   const int lane = threadIdx.x, tx = lane & (T8 - 1), ty = lane >> 3;
@@ -2201,27 +2201,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   const int V = atm8_chunks(nb);
   int pos = (int)((int64_t)V * s / Sm);
   const int end = (int)((int64_t)V * (s + 1) / Sm);
-  int t, pbx = 0, pby = 1, off;  // next tile, its blocks if a pair tile, chunks to skip
-  {
-    const int wlen = nb + kAtm8TileCost;
-    if (pos < nw * wlen) {
-      t = pos / wlen;
-      off = pos - t * wlen;
-    } else {
-      off = pos - nw * wlen;
-      int len = nb - 2 + kAtm8TileCost;  // of the tiles (., by)
-      t = nw;
-      while (off >= pby * len) {
-        off -= pby * len;
-        t += pby;
-        ++pby;
-        --len;
-      }
-      pbx = off / len;
-      off -= pbx * len;
-      t += pbx;
-    }
-  }
+  // next tile, its blocks if a pair tile, chunks to skip
+  const Atm8Start from = atm8_seek(nb, pos);
+  int t = from.t, pbx = from.bx, pby = from.by, off = from.off;
   while (pos < end) {
     const bool wt = t < nw;
     int bx, by, x, y, cx, cy, z1;  // staged blocks, pair, its record columns, first chunk
