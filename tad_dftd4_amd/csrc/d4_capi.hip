@@ -1,6 +1,7 @@
 // C ABI of the D4 kernels (include/d4amd.h). Validates arguments, owns the
 // per-device table allocation and sequences the kernels on the caller's
-// stream. No host synchronisation except in d4_molecule_status.
+// stream. No host synchronisation except in d4_inputs_wait (for the read-back
+// alone), d4_molecule_status and d4_profile_read.
 
 #include <string.h>
 
@@ -78,6 +79,23 @@ int hip_error(hipError_t e, const char* where) {
   g_error = std::string(where) + ": " + hipGetErrorString(e);
   return D4_ERR_DEVICE;
 }
+
+// Makes `device` the current one while it lives (an event belongs to the device
+// it is created on, the null stream is the current device's).
+struct OnDevice {
+  int prev = -1;
+  hipError_t error;
+  explicit OnDevice(int device) {
+    error = hipGetDevice(&prev);
+    if (error == hipSuccess && prev != device)
+      error = hipSetDevice(device);
+    else
+      prev = -1;
+  }
+  ~OnDevice() {
+    if (prev >= 0) (void)hipSetDevice(prev);
+  }
+};
 
 #define D4_TRY(expr, where)                      \
   do {                                           \
@@ -826,6 +844,8 @@ int d4_inputs_begin(d4_context* ctx, void* stream, int64_t count, const int64_t*
     sc.kind[k] = kinds[k];
   }
   hipStream_t s = (hipStream_t)stream;
+  const OnDevice on(ctx->device);
+  D4_TRY(on.error, "hipSetDevice");
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   D4_TRY(hipStreamIsCapturing(s, &cap), "hipStreamIsCapturing");
   if (cap != hipStreamCaptureStatusNone)
