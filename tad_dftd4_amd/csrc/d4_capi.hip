@@ -54,6 +54,7 @@ struct d4_context {
   std::unordered_map<hipStream_t, d4_aux> aux;
   std::mutex ticket_mu;
   std::vector<d4_ticket*> tickets;  // idle ones
+  std::vector<d4_ticket*> lost;     // not known to have ended: kept until the context goes
   // diagnostics: per-kernel event timing
   unsigned profile = 0;  // bit k: bracket launches of slot k with events
   std::vector<d4_event_pair> pending;
@@ -75,7 +76,10 @@ int set_error(int code, const std::string& msg) {
   return code;
 }
 
+// (the runtime's own record of the error is cleared with it, so that a later
+// launch does not report it again)
 int hip_error(hipError_t e, const char* where) {
+  (void)hipGetLastError();
   g_error = std::string(where) + ": " + hipGetErrorString(e);
   return D4_ERR_DEVICE;
 }
@@ -533,6 +537,7 @@ int d4_context_destroy(d4_context* ctx) {
     (void)hipEventDestroy(kv.second.join);
     (void)hipStreamDestroy(kv.second.s);
   }
+  ctx->tickets.insert(ctx->tickets.end(), ctx->lost.begin(), ctx->lost.end());
   for (d4_ticket* t : ctx->tickets) {
     (void)hipEventDestroy(t->done);
     (void)hipHostFree(t->values);
@@ -824,6 +829,17 @@ int d4_model_pols_backward(d4_context* ctx, void* stream, int64_t nbatch, int64_
   return D4_OK;
 }
 
+namespace {
+
+// A read-back that ended (`idle`) gives its buffer and event to the next one;
+// the memory of one that may still be written is not used again.
+void end_ticket(d4_context* ctx, d4_ticket* t, bool idle) {
+  std::lock_guard<std::mutex> lock(ctx->ticket_mu);
+  (idle ? ctx->tickets : ctx->lost).push_back(t);
+}
+
+}  // namespace
+
 int d4_inputs_begin(d4_context* ctx, void* stream, int64_t count, const int64_t* numbers,
                     int nscalars, const void* const* scalars, const int32_t* kinds,
                     void** ticket) {
@@ -873,10 +889,13 @@ int d4_inputs_begin(d4_context* ctx, void* stream, int64_t count, const int64_t*
   t->count = nscalars;
   *t->bad() = 0;
   hipError_t e = d4::launch_inputs(s, numbers, count, sc, t->values, t->bad());
-  if (e == hipSuccess) e = hipEventRecord(t->done, s);
   if (e != hipSuccess) {
-    std::lock_guard<std::mutex> lock(ctx->ticket_mu);
-    ctx->tickets.push_back(t);
+    end_ticket(ctx, t, true);
+    return hip_error(e, "input read-back");
+  }
+  e = hipEventRecord(t->done, s);
+  if (e != hipSuccess) {  // the kernel is under way
+    end_ticket(ctx, t, hipStreamSynchronize(s) == hipSuccess);
     return hip_error(e, "input read-back");
   }
   *ticket = t;
@@ -890,10 +909,7 @@ int d4_inputs_wait(d4_context* ctx, void* ticket, double* values, int32_t* bad) 
   const hipError_t e = hipEventSynchronize(t->done);
   for (int k = 0; k < t->count && values != nullptr; ++k) values[k] = t->values[k];
   if (bad != nullptr) *bad = *t->bad();
-  {
-    std::lock_guard<std::mutex> lock(ctx->ticket_mu);
-    ctx->tickets.push_back(t);
-  }
+  end_ticket(ctx, t, e == hipSuccess);
   if (e != hipSuccess) return hip_error(e, "input read-back");
   return D4_OK;
 }

@@ -138,3 +138,54 @@ for device, stream in ((1, DEV1), (1, None), (0, DEV0), (0, None)):
             assert wait(ctx, t) == 0
     lib.d4_context_destroy(ctx)
 """)
+
+
+def test_failed_query_leaves_no_error(runtime_so):
+    """A capture query that fails is reported by its own call; the next call's
+    launches do not find its error."""
+    _run(runtime_so, r"""
+ctx = context(0)
+var("fail_query").value = 906
+rc, t = begin(ctx, DEV0)
+assert rc == L.D4_ERR_DEVICE and not t.value
+assert var("fake_last").value == 0
+rc, t = begin(ctx, DEV0)
+assert rc == 0 and wait(ctx, t) == 0
+""")
+
+
+@pytest.mark.parametrize("sync", [0, 700])
+def test_failed_record(runtime_so, sync):
+    """An event that cannot be recorded behind the launched read: its host memory
+    is used again only after the stream was waited for."""
+    _run(runtime_so, r"""
+ctx = context(0)
+var("fail_record").value = 400
+var("fail_sync").value = %d
+syncs, pinned, launches = (var(k).value for k in ("fake_syncs", "fake_pinned", "fake_launches"))
+rc, t = begin(ctx, DEV0)
+assert rc == L.D4_ERR_DEVICE and not t.value and var("fake_last").value == 0
+assert var("fake_launches").value == launches + 1 and var("fake_syncs").value == syncs + 1
+rc, t = begin(ctx, DEV0)
+assert rc == 0 and wait(ctx, t) == 0
+# a stream that could not be waited for may still write: new memory then
+assert var("fake_pinned").value == pinned + (2 if %d else 1)
+lib.d4_context_destroy(ctx)
+assert var("fake_freed").value == var("fake_pinned").value
+""" % (sync, sync))
+
+
+def test_failed_wait(runtime_so):
+    """A wait that fails is reported, and the host memory that the read may
+    still write is not given to the next call."""
+    _run(runtime_so, r"""
+ctx = context(0)
+rc, t = begin(ctx, DEV0)
+pinned = var("fake_pinned").value
+var("fail_wait").value = 900
+assert wait(ctx, t) == L.D4_ERR_DEVICE and var("fake_last").value == 0
+rc, t = begin(ctx, DEV0)
+assert rc == 0 and var("fake_pinned").value == pinned + 1 and wait(ctx, t) == 0
+lib.d4_context_destroy(ctx)
+assert var("fake_freed").value == var("fake_pinned").value
+""")
