@@ -908,10 +908,13 @@ __device__ __forceinline__ double* tf_matrix(const Work& w, int64_t m) {
 // Row r of an inclusive lower packed index: tri(r) <= e < tri(r + 1).
 __device__ __forceinline__ int incl_row(int e) { return strict_row(e) - 1; }
 
-// Molecule m still factorising at block kb (charges not given, no failure).
-__device__ __forceinline__ bool tf_active(const Inputs& in, const Work& w, int64_t m,
-                                          int kb) {
-  return in.q_in == nullptr && kb < w.natom[m] && !(w.status[m] & kStatusLU);
+// States of the factorisation of molecule m, non-zero where it goes to the
+// pivoted LU: word 0 is written by the assembly, word b + 1 by work-group 0 of
+// block b's launch, which reads word b. A launch so reads nothing that it
+// writes: all waves of its work-groups leave together or stay together. (The
+// words lie in the pivot rows, which the LU kernel fills later.)
+__device__ __forceinline__ int32_t* tf_state(const Work& w, int64_t m) {
+  return w.piv + m * (w.N + 1);
 }
 
 // Assemble the lower triangle of C and the border rows b, e; one wave per row.
@@ -925,10 +928,9 @@ __global__ __launch_bounds__(256) void k_tf_assemble(DevTables t, Params p, Inpu
   const int i = (int)(g - m * rows);
   const int n = w.natom[m];
   if (in.q_in != nullptr || i >= n + 2) return;
-  if (p.force_lu) {  // testing: every system goes to the pivoted-LU kernel
-    if (i == 0 && lane == 0) w.status[m] |= kStatusLU;
-    return;
-  }
+  // (testing: every system goes to the pivoted-LU kernel)
+  if (i == 0 && lane == 0) tf_state(w, m)[0] = p.force_lu;
+  if (p.force_lu) return;
   const int64_t* Z = in.numbers + m * N;
   const double* R = in.positions + m * N * 3;
   double* Ai = tf_matrix(w, m) + (size_t)i * (size_t)N;
@@ -1077,7 +1079,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
   double* W = piv + kTB;          // [3][16] reciprocal pivots
   int* flag = reinterpret_cast<int*>(W + 3 * kNB);
   const int64_t m = blockIdx.x;
-  if (!tf_active(in, w, m, kb)) return;
+  if (in.q_in != nullptr || kb >= w.natom[m]) return;
+  int32_t* state = tf_state(w, m) + kb / kTB;
+  if (state[0]) {
+    if (blockIdx.y == 0 && threadIdx.x == 0) state[1] = 1;
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t N = w.N;
@@ -1220,7 +1227,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
       tl_panels<false>(D, T, own, dmax, c0, nbs, W, flag, wave);
     __syncthreads();
     if (*flag) {  // uniform
-      if (y == 0 && tid == 0) w.status[m] |= kStatusLU;
+      if (y == 0 && tid == 0) state[1] = 1;
       return;
     }
   }
@@ -1236,6 +1243,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     const int c = e >> 6, r = e & (kTB - 1);
     if (c < r && r < nb) A[(size_t)(kb + c) * N + kb + r] = D[r * kTS + c];
   }
+  if (tid == 0) state[1] = 0;
   if (tid < nb) dpiv[kb + tid] = D[tid * (kTS + 1)];
   for (int r = nb; r < dmax; ++r)  // border rows in the diagonal tile
     if (tid < nb) A[(size_t)(kb + r) * N + kb + tid] = D[r * kTS + tid];
@@ -1259,7 +1267,11 @@ __global__ __launch_bounds__(256) void k_tf_reduce(Inputs in, Work w) {
     return;
   }
   for (int i = n + tid; i < N; i += 256) q[i] = 0.0;
-  if (n == 0 || (w.status[m] & kStatusLU)) return;
+  if (n == 0) return;
+  if (tf_state(w, m)[(n - 1) / kTB + 1]) {
+    if (tid == 0) w.status[m] |= kStatusLU;
+    return;
+  }
   // the border rows hold D^-1 L^-1 b and D^-1 L^-1 e
   const double* A = tf_matrix(w, m);
   const double* zb = A + (size_t)n * N;
