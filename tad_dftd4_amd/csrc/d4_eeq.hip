@@ -995,7 +995,10 @@ __device__ __forceinline__ void tl_product(const double* P, int r0, const double
 }
 
 // Rows r0 .. r0 + 63 (below `rows`, else zero), columns c0 .. c0 + 63 (below
-// `cols`, else zero) of A into a tile, eight loads in flight per thread.
+// `cols`, else zero) of A into a tile, eight loads in flight per thread. LOWER:
+// a diagonal tile, whose upper triangle (which work-group 0 of the launch
+// replaces) is neither read nor used.
+template <bool LOWER = false>
 __device__ __forceinline__ void tl_load(const double* A, int64_t N, int r0, int rows, int c0,
                                         int cols, double* T) {
   const int c = threadIdx.x & (kTB - 1), rr = threadIdx.x >> 6;
@@ -1004,7 +1007,10 @@ __device__ __forceinline__ void tl_load(const double* A, int64_t N, int r0, int 
   for (int h = 0; h < 2; ++h) {
     double v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[min(rr + 32 * h + 4 * u, rows - 1) * (int)N];
+    for (int u = 0; u < 8; ++u) {
+      const int r = min(rr + 32 * h + 4 * u, rows - 1);
+      v[u] = p[r * (int)N - (LOWER ? max(0, min(c, cols - 1) - r) : 0)];
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int r = rr + 32 * h + 4 * u;
@@ -1132,13 +1138,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
 
   // a panel row tile: D the diagonal tile (its rows past nb: border rows), T
   // the work-group's own rows
-  const int r0 = kb + y * kTB, rows = last - r0, drows = last - kb;
+  const int r0 = kb + y * kTB, rows = last - r0;
   if (rows <= 0) return;
   const bool own = y > 0;
+  // (border rows in the diagonal tile are work-group 0's alone: it stores them
+  // in place during this launch)
+  const int drows = own ? nb : last - kb;
   double* D = Y;
   double* T = X;
   if (kb == 0) {
-    tl_load(A, N, 0, drows, 0, nb, D);
+    tl_load<true>(A, N, 0, drows, 0, nb, D);
     if (own) tl_load(A, N, r0, rows, 0, nb, T);
     __syncthreads();
   } else {
