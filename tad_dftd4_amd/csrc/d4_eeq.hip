@@ -76,16 +76,6 @@ __device__ __forceinline__ double row_bcast(double v) {
   return r;
 }
 
-// d += u t with u of lane C of each 16-lane row. (A DPP operand may not be
-// written by the two instructions before: here t depends on u through the
-// pivot chain, so u is always older than that.)
-template <int C>
-__device__ __forceinline__ void fmac_bcast(double& d, double u, double t) {
-  asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-      : "+v"(d)
-      : "v"(u), "v"(t), "n"(C));
-}
-
 // A panel: D holds row (lane & 15) of the block itself, d the lane's row below
 // it, w the reciprocal pivots. Entries right of a row's diagonal in D are junk.
 struct Panel {
@@ -93,16 +83,82 @@ struct Panel {
   unsigned long long good;  // non-zero lanes: every pivot so far is positive
 };
 
-// Column J of the elimination for columns C .. C1 - 1 of the block's rows and,
-// with ROWS, of the rows below.
+// Column J of the elimination, u = D[J], for other columns C: D[C] += u t and, with
+// ROWS, d[C] += u t2, with u of lane C of each 16-lane row. A DPP operand may not
+// be written by the two instructions before, and the compiler, which does not look
+// into the assembly, could place a copy of u just there: each statement fills the
+// two slots itself (energies of one 200-atom molecule 159 -> 161 us; without the
+// products in panel_next, a wait in each of more statements, 161-162).
+#define D4_FMAC(acc, u, t, c) \
+  "v_fmac_f64_dpp " acc ", " u ", " t " row_newbcast:" c " row_mask:0xf bank_mask:0xf\n\t"
+
+// The next column, with the products t = -u w and t2 = -d[J] w in the two slots.
+template <bool ROWS, int J>
+__device__ __forceinline__ void panel_next(Panel& P, double& t, double& t2) {
+  if constexpr (ROWS)
+    asm("v_mul_f64 %2, -%4, %6\n\t"
+        "v_mul_f64 %3, -%5, %6\n\t"
+        D4_FMAC("%0", "%4", "%2", "%7")
+        D4_FMAC("%1", "%4", "%3", "%7")
+        : "+&v"(P.D[J + 1]), "+&v"(P.d[J + 1]), "=&v"(t), "=&v"(t2)
+        : "v"(P.D[J]), "v"(P.d[J]), "v"(P.w[J]), "n"(J + 1));
+  else
+    asm("v_mul_f64 %1, -%2, %3\n\t"
+        "s_nop 0\n\t"
+        D4_FMAC("%0", "%2", "%1", "%4")
+        : "+&v"(P.D[J + 1]), "=&v"(t)
+        : "v"(P.D[J]), "v"(P.w[J]), "n"(J + 1));
+}
+
+// Columns C .. C1 - 1, up to four to a statement.
 template <bool ROWS, int J, int C, int C1>
 __device__ __forceinline__ void panel_columns(Panel& P, double t, double t2) {
-  if constexpr (C < C1 && C < kNB) {
-    fmac_bcast<C>(P.D[C], P.D[J], t);
-    if (ROWS) fmac_bcast<C>(P.d[C], P.D[J], t2);
-    panel_columns<ROWS, J, C + 1, C1>(P, t, t2);
-  }
+  constexpr int left = (C1 < kNB ? C1 : kNB) - C, K = left < 4 ? left : 4;
+  if constexpr (K == 1 && ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%2", "%3", "%5") D4_FMAC("%1", "%2", "%4", "%5")
+        : "+&v"(P.D[C]), "+&v"(P.d[C])
+        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C));
+  if constexpr (K == 1 && !ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%1", "%2", "%3")
+        : "+&v"(P.D[C])
+        : "v"(P.D[J]), "v"(t), "n"(C));
+  if constexpr (K == 2 && ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%4", "%5", "%7") D4_FMAC("%2", "%4", "%6", "%7")
+        D4_FMAC("%1", "%4", "%5", "%8") D4_FMAC("%3", "%4", "%6", "%8")
+        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.d[C]), "+&v"(P.d[C + 1])
+        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C), "n"(C + 1));
+  if constexpr (K == 2 && !ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%2", "%3", "%4") D4_FMAC("%1", "%2", "%3", "%5")
+        : "+&v"(P.D[C]), "+&v"(P.D[C + 1])
+        : "v"(P.D[J]), "v"(t), "n"(C), "n"(C + 1));
+  if constexpr (K == 3 && ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%6", "%7", "%9") D4_FMAC("%3", "%6", "%8", "%9")
+        D4_FMAC("%1", "%6", "%7", "%10") D4_FMAC("%4", "%6", "%8", "%10")
+        D4_FMAC("%2", "%6", "%7", "%11") D4_FMAC("%5", "%6", "%8", "%11")
+        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2]), "+&v"(P.d[C]),
+          "+&v"(P.d[C + 1]), "+&v"(P.d[C + 2])
+        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C), "n"(C + 1), "n"(C + 2));
+  if constexpr (K == 3 && !ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%3", "%4", "%5") D4_FMAC("%1", "%3", "%4", "%6")
+        D4_FMAC("%2", "%3", "%4", "%7")
+        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2])
+        : "v"(P.D[J]), "v"(t), "n"(C), "n"(C + 1), "n"(C + 2));
+  if constexpr (K == 4 && ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%8", "%9", "%11") D4_FMAC("%4", "%8", "%10", "%11")
+        D4_FMAC("%1", "%8", "%9", "%12") D4_FMAC("%5", "%8", "%10", "%12")
+        D4_FMAC("%2", "%8", "%9", "%13") D4_FMAC("%6", "%8", "%10", "%13")
+        D4_FMAC("%3", "%8", "%9", "%14") D4_FMAC("%7", "%8", "%10", "%14")
+        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2]), "+&v"(P.D[C + 3]),
+          "+&v"(P.d[C]), "+&v"(P.d[C + 1]), "+&v"(P.d[C + 2]), "+&v"(P.d[C + 3])
+        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C), "n"(C + 1), "n"(C + 2), "n"(C + 3));
+  if constexpr (K == 4 && !ROWS)
+    asm("s_nop 1\n\t" D4_FMAC("%0", "%4", "%5", "%6") D4_FMAC("%1", "%4", "%5", "%7")
+        D4_FMAC("%2", "%4", "%5", "%8") D4_FMAC("%3", "%4", "%5", "%9")
+        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2]), "+&v"(P.D[C + 3])
+        : "v"(P.D[J]), "v"(t), "n"(C), "n"(C + 1), "n"(C + 2), "n"(C + 3));
+  if constexpr (K > 0) panel_columns<ROWS, J, C + K, C1>(P, t, t2);
 }
+#undef D4_FMAC
 
 // Eliminate column J and go on with J + 1, whose pivot chain is spread between
 // the updates of column J. The columns keep their values before the division
@@ -114,8 +170,8 @@ __device__ __forceinline__ void panel_step(Panel& P, int nb, double* W) {
   if constexpr (J + 1 < kNB) {
     P.w[J + 1] = 0.0;
     if (FULL || J + 1 < nb) {  // uniform (columns past nb are padding)
-      const double t = -P.D[J] * P.w[J], t2 = ROWS ? -P.d[J] * P.w[J] : 0.0;
-      panel_columns<ROWS, J, J + 1, J + 2>(P, t, t2);
+      double t, t2 = 0.0;
+      panel_next<ROWS, J>(P, t, t2);
       const double pv = row_bcast<J + 1>(P.D[J + 1]);
       const double r = __builtin_amdgcn_rcp(pv);  // relative error below 2^-23
       panel_columns<ROWS, J, J + 2, J + 5>(P, t, t2);
