@@ -87,78 +87,112 @@ struct Panel {
 // ROWS, d[C] += u t2, with u of lane C of each 16-lane row. A DPP operand may not
 // be written by the two instructions before, and the compiler, which does not look
 // into the assembly, could place a copy of u just there: each statement fills the
-// two slots itself (energies of one 200-atom molecule 159 -> 161 us; without the
-// products in panel_next, a wait in each of more statements, 161-162).
-#define D4_FMAC(acc, u, t, c) \
-  "v_fmac_f64_dpp " acc ", " u ", " t " row_newbcast:" c " row_mask:0xf bank_mask:0xf\n\t"
+// two slots itself, with a link of the pivot chain and a wait. (Captured step of
+// one 150-atom molecule: 151.8 us with the slots left open, 153.5 with two waits
+// in each statement, 152.8 so.)
+#define D4_FMAC(acc, t, c) \
+  "v_fmac_f64_dpp %[" acc "], %[u], %[" t "] row_newbcast:%[" c "] row_mask:0xf bank_mask:0xf\n\t"
+#define D4_COL(k) D4_FMAC("D" k, "t", "c" k)
+#define D4_COL2(k) D4_FMAC("D" k, "t", "c" k) D4_FMAC("d" k, "t2", "c" k)
 
-// The next column, with the products t = -u w and t2 = -d[J] w in the two slots.
+// The next column, with the products t = -u w and t2 = -d[J] w in the two slots,
+// and its pivot for all lanes of a row.
 template <bool ROWS, int J>
-__device__ __forceinline__ void panel_next(Panel& P, double& t, double& t2) {
+__device__ __forceinline__ double panel_next(Panel& P, double& t, double& t2) {
+  double pv;
   if constexpr (ROWS)
-    asm("v_mul_f64 %2, -%4, %6\n\t"
-        "v_mul_f64 %3, -%5, %6\n\t"
-        D4_FMAC("%0", "%4", "%2", "%7")
-        D4_FMAC("%1", "%4", "%3", "%7")
-        : "+&v"(P.D[J + 1]), "+&v"(P.d[J + 1]), "=&v"(t), "=&v"(t2)
-        : "v"(P.D[J]), "v"(P.d[J]), "v"(P.w[J]), "n"(J + 1));
-  else
-    asm("v_mul_f64 %1, -%2, %3\n\t"
+    asm("v_mul_f64 %[t], -%[u], %[w]\n\t"
+        "v_mul_f64 %[t2], -%[v], %[w]\n\t"
+        D4_COL2("0")
         "s_nop 0\n\t"
-        D4_FMAC("%0", "%2", "%1", "%4")
-        : "+&v"(P.D[J + 1]), "=&v"(t)
-        : "v"(P.D[J]), "v"(P.w[J]), "n"(J + 1));
+        "v_mov_b64_dpp %[pv], %[D0] row_newbcast:%[c0] row_mask:0xf bank_mask:0xf"
+        : [D0] "+&v"(P.D[J + 1]), [d0] "+&v"(P.d[J + 1]), [t] "=&v"(t), [t2] "=&v"(t2),
+          [pv] "=&v"(pv)
+        : [u] "v"(P.D[J]), [v] "v"(P.d[J]), [w] "v"(P.w[J]), [c0] "n"(J + 1));
+  else
+    asm("v_mul_f64 %[t], -%[u], %[w]\n\t"
+        "s_nop 0\n\t"
+        D4_COL("0")
+        "s_nop 1\n\t"
+        "v_mov_b64_dpp %[pv], %[D0] row_newbcast:%[c0] row_mask:0xf bank_mask:0xf"
+        : [D0] "+&v"(P.D[J + 1]), [t] "=&v"(t), [pv] "=&v"(pv)
+        : [u] "v"(P.D[J]), [w] "v"(P.w[J]), [c0] "n"(J + 1));
+  return pv;
 }
 
-// Columns C .. C1 - 1, up to four to a statement.
-template <bool ROWS, int J, int C, int C1>
-__device__ __forceinline__ void panel_columns(Panel& P, double t, double t2) {
-  constexpr int left = (C1 < kNB ? C1 : kNB) - C, K = left < 4 ? left : 4;
-  if constexpr (K == 1 && ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%2", "%3", "%5") D4_FMAC("%1", "%2", "%4", "%5")
-        : "+&v"(P.D[C]), "+&v"(P.d[C])
-        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C));
-  if constexpr (K == 1 && !ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%1", "%2", "%3")
-        : "+&v"(P.D[C])
-        : "v"(P.D[J]), "v"(t), "n"(C));
-  if constexpr (K == 2 && ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%4", "%5", "%7") D4_FMAC("%2", "%4", "%6", "%7")
-        D4_FMAC("%1", "%4", "%5", "%8") D4_FMAC("%3", "%4", "%6", "%8")
-        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.d[C]), "+&v"(P.d[C + 1])
-        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C), "n"(C + 1));
-  if constexpr (K == 2 && !ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%2", "%3", "%4") D4_FMAC("%1", "%2", "%3", "%5")
-        : "+&v"(P.D[C]), "+&v"(P.D[C + 1])
-        : "v"(P.D[J]), "v"(t), "n"(C), "n"(C + 1));
-  if constexpr (K == 3 && ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%6", "%7", "%9") D4_FMAC("%3", "%6", "%8", "%9")
-        D4_FMAC("%1", "%6", "%7", "%10") D4_FMAC("%4", "%6", "%8", "%10")
-        D4_FMAC("%2", "%6", "%7", "%11") D4_FMAC("%5", "%6", "%8", "%11")
-        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2]), "+&v"(P.d[C]),
-          "+&v"(P.d[C + 1]), "+&v"(P.d[C + 2])
-        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C), "n"(C + 1), "n"(C + 2));
-  if constexpr (K == 3 && !ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%3", "%4", "%5") D4_FMAC("%1", "%3", "%4", "%6")
-        D4_FMAC("%2", "%3", "%4", "%7")
-        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2])
-        : "v"(P.D[J]), "v"(t), "n"(C), "n"(C + 1), "n"(C + 2));
-  if constexpr (K == 4 && ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%8", "%9", "%11") D4_FMAC("%4", "%8", "%10", "%11")
-        D4_FMAC("%1", "%8", "%9", "%12") D4_FMAC("%5", "%8", "%10", "%12")
-        D4_FMAC("%2", "%8", "%9", "%13") D4_FMAC("%6", "%8", "%10", "%13")
-        D4_FMAC("%3", "%8", "%9", "%14") D4_FMAC("%7", "%8", "%10", "%14")
-        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2]), "+&v"(P.D[C + 3]),
-          "+&v"(P.d[C]), "+&v"(P.d[C + 1]), "+&v"(P.d[C + 2]), "+&v"(P.d[C + 3])
-        : "v"(P.D[J]), "v"(t), "v"(t2), "n"(C), "n"(C + 1), "n"(C + 2), "n"(C + 3));
-  if constexpr (K == 4 && !ROWS)
-    asm("s_nop 1\n\t" D4_FMAC("%0", "%4", "%5", "%6") D4_FMAC("%1", "%4", "%5", "%7")
-        D4_FMAC("%2", "%4", "%5", "%8") D4_FMAC("%3", "%4", "%5", "%9")
-        : "+&v"(P.D[C]), "+&v"(P.D[C + 1]), "+&v"(P.D[C + 2]), "+&v"(P.D[C + 3])
-        : "v"(P.D[J]), "v"(t), "n"(C), "n"(C + 1), "n"(C + 2), "n"(C + 3));
-  if constexpr (K > 0) panel_columns<ROWS, J, C + K, C1>(P, t, t2);
+// Columns C .. C + K - 1 (K <= 4) behind x = the link of the chain that LEAD names.
+enum { kLeadRcp, kLeadError, kLeadSquare, kLeadStep };
+#define D4_COLUMNS(LEAD, ...)                                                              \
+  if constexpr (K == 1 && ROWS)                                                            \
+    asm(LEAD D4_COL2("0")                                                                  \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [d0] "+&v"(P.d[C])                             \
+        : [u] "v"(P.D[J]), [t] "v"(t), [t2] "v"(t2), [c0] "n"(C), __VA_ARGS__);            \
+  if constexpr (K == 1 && !ROWS)                                                           \
+    asm(LEAD D4_COL("0")                                                                   \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C])                                                 \
+        : [u] "v"(P.D[J]), [t] "v"(t), [c0] "n"(C), __VA_ARGS__);                          \
+  if constexpr (K == 2 && ROWS)                                                            \
+    asm(LEAD D4_COL2("0") D4_COL2("1")                                                     \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [d0] "+&v"(P.d[C]), [D1] "+&v"(P.D[C + 1]),    \
+          [d1] "+&v"(P.d[C + 1])                                                           \
+        : [u] "v"(P.D[J]), [t] "v"(t), [t2] "v"(t2), [c0] "n"(C), [c1] "n"(C + 1),         \
+          __VA_ARGS__);                                                                    \
+  if constexpr (K == 2 && !ROWS)                                                           \
+    asm(LEAD D4_COL("0") D4_COL("1")                                                       \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [D1] "+&v"(P.D[C + 1])                         \
+        : [u] "v"(P.D[J]), [t] "v"(t), [c0] "n"(C), [c1] "n"(C + 1), __VA_ARGS__);         \
+  if constexpr (K == 3 && ROWS)                                                            \
+    asm(LEAD D4_COL2("0") D4_COL2("1") D4_COL2("2")                                        \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [d0] "+&v"(P.d[C]), [D1] "+&v"(P.D[C + 1]),    \
+          [d1] "+&v"(P.d[C + 1]), [D2] "+&v"(P.D[C + 2]), [d2] "+&v"(P.d[C + 2])           \
+        : [u] "v"(P.D[J]), [t] "v"(t), [t2] "v"(t2), [c0] "n"(C), [c1] "n"(C + 1),         \
+          [c2] "n"(C + 2), __VA_ARGS__);                                                   \
+  if constexpr (K == 3 && !ROWS)                                                           \
+    asm(LEAD D4_COL("0") D4_COL("1") D4_COL("2")                                           \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [D1] "+&v"(P.D[C + 1]), [D2] "+&v"(P.D[C + 2]) \
+        : [u] "v"(P.D[J]), [t] "v"(t), [c0] "n"(C), [c1] "n"(C + 1), [c2] "n"(C + 2),      \
+          __VA_ARGS__);                                                                    \
+  if constexpr (K == 4 && ROWS)                                                            \
+    asm(LEAD D4_COL2("0") D4_COL2("1") D4_COL2("2") D4_COL2("3")                           \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [d0] "+&v"(P.d[C]), [D1] "+&v"(P.D[C + 1]),    \
+          [d1] "+&v"(P.d[C + 1]), [D2] "+&v"(P.D[C + 2]), [d2] "+&v"(P.d[C + 2]),          \
+          [D3] "+&v"(P.D[C + 3]), [d3] "+&v"(P.d[C + 3])                                   \
+        : [u] "v"(P.D[J]), [t] "v"(t), [t2] "v"(t2), [c0] "n"(C), [c1] "n"(C + 1),         \
+          [c2] "n"(C + 2), [c3] "n"(C + 3), __VA_ARGS__);                                  \
+  if constexpr (K == 4 && !ROWS)                                                           \
+    asm(LEAD D4_COL("0") D4_COL("1") D4_COL("2") D4_COL("3")                               \
+        : [x] "=&v"(x), [D0] "+&v"(P.D[C]), [D1] "+&v"(P.D[C + 1]), [D2] "+&v"(P.D[C + 2]), \
+          [D3] "+&v"(P.D[C + 3])                                                           \
+        : [u] "v"(P.D[J]), [t] "v"(t), [c0] "n"(C), [c1] "n"(C + 1), [c2] "n"(C + 2),      \
+          [c3] "n"(C + 3), __VA_ARGS__);
+
+template <int LEAD, bool ROWS, int J, int C, int K>
+__device__ __forceinline__ double panel_columns(Panel& P, double t, double t2, double a, double b) {
+  double x;
+  if constexpr (K == 0 && LEAD == kLeadRcp) x = __builtin_amdgcn_rcp(a);
+  if constexpr (K == 0 && LEAD == kLeadError) x = fma(-a, b, 1.0);
+  if constexpr (K == 0 && LEAD == kLeadSquare) x = fma(a, a, a);
+  if constexpr (K == 0 && LEAD == kLeadStep) x = fma(b, a, b);
+  if constexpr (LEAD == kLeadRcp) {
+    D4_COLUMNS("v_rcp_f64 %[x], %[a]\n\ts_nop 0\n\t", [a] "v"(a))
+  } else if constexpr (LEAD == kLeadError) {
+    D4_COLUMNS("v_fma_f64 %[x], -%[a], %[b], 1.0\n\ts_nop 0\n\t", [a] "v"(a), [b] "v"(b))
+  } else if constexpr (LEAD == kLeadSquare) {
+    D4_COLUMNS("v_fma_f64 %[x], %[a], %[a], %[a]\n\ts_nop 0\n\t", [a] "v"(a))
+  } else {
+    D4_COLUMNS("v_fma_f64 %[x], %[b], %[a], %[b]\n\ts_nop 0\n\t", [a] "v"(a), [b] "v"(b))
+  }
+  return x;
 }
+#undef D4_COLUMNS
+#undef D4_COL2
+#undef D4_COL
 #undef D4_FMAC
+
+// Columns left of at most `most` from column C on.
+constexpr int panel_part(int c, int most) {
+  return kNB - c < 0 ? 0 : kNB - c < most ? kNB - c : most;
+}
 
 // Eliminate column J and go on with J + 1, whose pivot chain is spread between
 // the updates of column J. The columns keep their values before the division
@@ -171,18 +205,18 @@ __device__ __forceinline__ void panel_step(Panel& P, int nb, double* W) {
     P.w[J + 1] = 0.0;
     if (FULL || J + 1 < nb) {  // uniform (columns past nb are padding)
       double t, t2 = 0.0;
-      panel_next<ROWS, J>(P, t, t2);
-      const double pv = row_bcast<J + 1>(P.D[J + 1]);
-      const double r = __builtin_amdgcn_rcp(pv);  // relative error below 2^-23
-      panel_columns<ROWS, J, J + 2, J + 5>(P, t, t2);
-      const double e = fma(-pv, r, 1.0);
-      panel_columns<ROWS, J, J + 5, J + 7>(P, t, t2);
-      const double e2 = fma(e, e, e);
-      panel_columns<ROWS, J, J + 7, J + 9>(P, t, t2);
-      P.w[J + 1] = fma(r, e2, r);  // third-order step: 1 / pv
+      const double pv = panel_next<ROWS, J>(P, t, t2);
+      // 1 / pv from the hardware estimate (relative error below 2^-23) by a
+      // third-order step, its links between the other columns
+      constexpr int C0 = J + 2, K0 = panel_part(C0, 4), C1 = C0 + K0, K1 = panel_part(C1, 3),
+                    C2 = C1 + K1, K2 = panel_part(C2, 3), C3 = C2 + K2, K3 = panel_part(C3, 4);
+      static_assert(C3 + K3 >= kNB, "all columns");
+      const double r = panel_columns<kLeadRcp, ROWS, J, C0, K0>(P, t, t2, pv, pv);
+      const double e = panel_columns<kLeadError, ROWS, J, C1, K1>(P, t, t2, pv, r);
+      const double e2 = panel_columns<kLeadSquare, ROWS, J, C2, K2>(P, t, t2, e, e);
+      P.w[J + 1] = panel_columns<kLeadStep, ROWS, J, C3, K3>(P, t, t2, e2, r);
       if (WLDS) W[J + 1] = P.w[J + 1];  // (every lane the same value)
       P.good &= __builtin_amdgcn_fcmp(pv, 0.0, kFcmpOgt);
-      panel_columns<ROWS, J, J + 9, kNB>(P, t, t2);
       __builtin_amdgcn_sched_barrier(0);  // (hoisting across columns only costs registers)
     }
     panel_step<ROWS, FULL, WLDS, J + 1>(P, nb, W);
