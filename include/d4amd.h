@@ -4,9 +4,10 @@
  * Plain pointers and sizes only. Every device pointer argument is memory
  * that the caller owns (allocated by the caller, e.g. by PyTorch); the
  * library owns only its per-device context (the element tables resident in
- * HBM). Streams are passed as `void*` holding a `hipStream_t`; every entry
- * point only enqueues work on that stream (no host synchronisation), so a
- * caller may capture the calls in a HIP graph.
+ * HBM) and the pinned buffers of its input read-backs. Streams are passed as
+ * `void*` holding a `hipStream_t`; every compute entry point only enqueues work
+ * on that stream (no host synchronisation), so a caller may capture the calls
+ * in a HIP graph. d4_inputs_wait, d4_molecule_status and d4_profile_read wait.
  *
  * Batch convention (as in the reference): `numbers` is (nbatch, natoms)
  * int64 with Z = 0 marking padding atoms, `positions` is (nbatch, natoms, 3)
@@ -59,8 +60,9 @@ extern "C" {
 #define D4_FLAG_ROWS_32 512
 #define D4_FLAG_ROWS_64 768
 #define D4_FLAG_ROWS_MASK 768
-#define D4_FLAG_ATM8 1024  /* one-pass three-body kernel with 8 x 8 pair tiles (the
-                              default) */
+#define D4_FLAG_ATM8 1024  /* accepted, without effect: 8 x 8 pair tiles are what the
+                              one-pass three-body kernel takes without
+                              D4_FLAG_ATM16 */
 #define D4_FLAG_ONE_STREAM 2048 /* testing/profiling: run the three-body side on the
                                    caller's stream too (no companion stream), so a
                                    kernel trace shows each kernel's own time */

@@ -1,7 +1,8 @@
 // HIP kernels (gfx950) for the EEQ charges and their adjoint.
 //
 // Molecules whose packed Coulomb factor fits in LDS are solved by one
-// work-group each (L D L^T by whole waves, FP64 matrix instructions); larger molecules use the tiled multi-work-group path.
+// work-group each (L D L^T by whole waves, FP64 matrix instructions); larger
+// molecules use the tiled multi-work-group path.
 // Every output element has one writer and every reduction a fixed order.
 
 #include <map>
@@ -1050,9 +1051,11 @@ __global__ __launch_bounds__(256) void k_tf_assemble(DevTables t, Params p, Inpu
 }
 
 // The tiled kernels take their LDS as dynamic shared memory and at most 80
-// VGPRs: a work-group then fits beside the three-body kernel's waves (two per
-// SIMD with 216 VGPRs, 86 KB of LDS per CU) on any CU instead of waiting until
-// one is nearly empty.
+// VGPRs (k_tl_step spills 31 of them, k_tl_solve 20): a work-group then fits
+// beside the three-body kernel's waves with gradients (two per SIMD with 192
+// VGPRs, 86 KB of LDS per CU) on any CU instead of waiting until one is nearly
+// empty. Beside the energy kernel (108 VGPRs, four waves per SIMD) it waits for
+// the first ones to end.
 constexpr int kTS = kTB + 1;  // row stride of a tile in LDS
 constexpr size_t kTlLds = sizeof(double) * (2 * kTB * kTS + kTB + 3 * kNB + 2);
 
@@ -1706,10 +1709,10 @@ __global__ __launch_bounds__(256) void k_adjoint(DevTables t, Params p, Inputs i
 // share the first bin), so that the longest solves start first and the short
 // ones fill in behind them (the adjoint of the 1024 x 20-120 batch alone 67 ->
 // 48 us). Which work-group solves which molecule does not change any result;
-// the order within a bin is arbitrary. (The charge kernel keeps the batch
-// order: taking the largest first there made it faster alone, 217 -> 153 us,
-// but the two-stream step slower, 1.10 -> 1.13 ms, as it then crowds the
-// three-body pair pass that runs beside it.)
+// the order within a bin is arbitrary. (The charge kernel reads the order from
+// its end, smallest first: with the largest first it is faster alone, but the
+// two-stream step slower, 0.892 -> 0.921 ms, as it then crowds the three-body
+// pair pass beside it; smallest first 0.890 -> 0.884 ms.)
 constexpr int kOrdMax = 256;
 
 __global__ __launch_bounds__(1024) void k_eeq_order(Work w) {

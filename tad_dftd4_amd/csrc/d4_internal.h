@@ -145,9 +145,9 @@ __host__ __device__ inline int atm1_splits(int n);
 // of chunks (tile, 8 third atoms), each tile preceded by kAtm8TileCost places
 // for its own loads and sums; the atm8_splits(n) waves of a molecule, also a
 // function of n alone, take equal parts of that list. n^2 / 250 parts keep the
-// partial sums (5 n doubles each) a fixed small share of the n^3 / 6 triples:
-// 12 to 16 chunks per part up to 160 atoms, more above, where 3 n / 5 parts is
-// what the buffer holds. Steps in us with n^2 / 160, / 250, / 400: 256 x 8-200
+// partial sums (5 n doubles each) a small share of the n^3 / 6 triples: a part
+// holds 2 places at 16 atoms, 8 at 64, 18 at 160, 42 at 256 (from 151 on 3 n / 5
+// parts, what the buffer holds). Steps in us with n^2 / 160, / 250, / 400: 256 x 8-200
 // energies 466 / 458 / 467, 1024 x 20-120 forces 931 / 886 / 897, 256 x 20-120
 // D4S 480 / 471 / 485; whole tiles dealt to at most 64 parts: 589 / 894 / 509.
 constexpr int kAtm8 = 8;
@@ -254,7 +254,7 @@ __host__ __device__ inline int one_pass_splits(int n, bool tile8) {
 }
 
 // The one-pass kernel is the 8 x 8 one unless the caller asks for 16 x 16
-// (energy steps, us, 16 x 16 against 8 x 8: one 64-atom molecule 104 / 62, 384
+// (D4_FLAG_ATM8 only says so; energy steps, us, 16 x 16 against 8 x 8: one 64-atom molecule 104 / 62, 384
 // x 6-60 atoms 160 / 102, 1024 x 20-120 693 / 586, 256 x 8-160 372 / 345, 256 x
 // 8-200 531 / 527).
 inline bool one_pass_tile8(const Params& p) { return !p.atm16; }

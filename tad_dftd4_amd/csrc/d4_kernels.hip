@@ -2467,7 +2467,8 @@ __global__ __launch_bounds__(64) void k_atm8s_count(Params p, Inputs in, Work w)
 }
 
 // Work items of every molecule: x-group g with w_g places gets 1 + w_g G / (u
-// (G - g)) items (of at least eight places), u the smallest size for which the
+// (G - g)) items, at most 1 + w_g / 8 (four places and more to an item where
+// there are two or more of them), u the smallest size for which the
 // windows (an item of g has one per group from g on) and the grid suffice.
 // Later groups, whose items need fewer windows and run last, are split finer:
 // the kernel ends evenly.

@@ -1,7 +1,8 @@
 """
 Device runtime: per-device contexts (element tables resident in HBM),
 workspace sizing, and thin wrappers that call the C ABI on torch tensors
-with torch's current HIP stream. No host synchronisation happens here.
+with torch's current HIP stream. The compute calls do not synchronise the
+host; ``InputCheck.wait``, ``molecule_status`` and ``profile_read`` wait.
 """
 
 from __future__ import annotations

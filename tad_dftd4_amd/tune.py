@@ -4,9 +4,9 @@ Launch-shape tuner.
 Two launch shapes of the batched path change speed but not results (beyond
 rounding): the lanes per atom row of the CN, pair and chain passes (16, 32
 or 64: a quarter, half or full wave walks one atom's partners) and the pair
-tile of the one-pass three-body kernel (8 x 8 or 16 x 16 pairs per
-work-group, used up to 256 atoms). Built in, both follow fixed rules of the
-padded length and the mode. ``tune`` times every candidate on the device for
+tile of the one-pass three-body kernel (8 x 8 or 16 x 16 pairs, used up to
+256 atoms). Built in, the lanes follow a fixed rule of the padded length and
+the tile is 8 x 8. ``tune`` times every candidate on the device for
 a list of padded-length buckets and both modes (atom energies; energies and
 gradient), on synthetic molecules of the batch workloads' kind (jittered
 2.8 bohr grid, Z <= 54 mix, charges -1/0/+1), with HIP events on the calling
@@ -107,7 +107,9 @@ def active() -> ShapeTable | None:
 
 def candidates(n_max: int) -> list[tuple[int, int]]:
     """(row_lanes, atm_tile) pairs worth timing for a bucket; (0, 0) is the
-    built-in rule. Past the one-pass limit the tile has no effect."""
+    built-in rule (up to 256 atoms the same launches as the rule's lanes with 8:
+    the two times show a run's noise). Past the one-pass limit the tile has no
+    effect."""
     tiles = TILES if n_max <= ONE_PASS_MAX else (0,)
     return [(0, 0)] + [(r, t) for r in ROWS for t in tiles]
 
