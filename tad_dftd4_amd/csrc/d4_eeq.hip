@@ -59,11 +59,11 @@ __device__ __forceinline__ double lane_bcast(double v, int src) {
 // next steps in flight.
 // What bounds it: instruction issue (one wave issues an FP64 instruction every
 // 6 cycles) in the panels' few waves and in the assembly, then the chains.
-// One 150-atom molecule takes 64 us (assembly 14, panels 17, updates 18,
+// One 150-atom molecule takes 63 us (assembly 14, panels 17, updates 18,
 // substitution 8, the rest loads and barriers); the blocked Cholesky with
 // inverse diagonal blocks and 4 x 4 register tiles that was here before, by
 // four waves with barriers in the substitutions, took 147 us. 1024 molecules
-// of 20-120 atoms: 108 instead of 177 us.
+// of 20-120 atoms alone: 86 instead of 177 us.
 
 typedef double d4_acc __attribute__((ext_vector_type(4)));
 
